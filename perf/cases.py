@@ -252,11 +252,11 @@ class _Memory:
                                          "version": 3, "strides": None}
 
 
-def _tree(bvh):
-    """The Woop rows and triangle ids of a BVH, in leaf order, as tensors over its own buffers."""
+def _woop(bvh):
+    """The Woop rows of a BVH, in leaf order, as a tensor over its own buffer
+    (which every rebuild of the same scene writes again)."""
     w = bvh.view()
-    parts = {"woop": (w.woop, (w.n_references, 12), "<f4"), "ids": (w.tri_indices, (w.n_references,), "<i4")}
-    return {k: torch.as_tensor(_Memory(bvh, *p), device=DEV) for k, p in parts.items()}
+    return torch.as_tensor(_Memory(bvh, w.woop, (w.n_references, 12), "<f4"), device=DEV)
 
 
 BUILDERS = {"lbvh": hx.LBVHBuilder, "ploc": hx.PLOCBuilder, "atr": hx.ATRBuilder, "insertion": hx.InsertionBuilder}
@@ -275,9 +275,10 @@ def prepare(case, seed):
         builder = BUILDERS[case["method"]](ctx, **params)
         scene = hx.Scene(v, t)
         bvh = builder.build(scene)
-        # The presplitter's reference count is the scene's own, so those trees
-        # are seen through the hits alone, as the nodes of every tree are.
-        return dict(case=case, builder=builder, bvh=bvh, tree={} if case["presplit"] else _tree(bvh),
+        # Leaf order shows in the Woop rows and in the ids of the hits, nodes in
+        # the hits.  A presplit scene's reference count is its own, so those
+        # trees are seen through the hits alone.
+        return dict(case=case, builder=builder, bvh=bvh, tree={} if case["presplit"] else {"woop": _woop(bvh)},
                     tracer=hx.HipTracer(ctx, bvh), rays=hx.RayBuffer(_primary(case["geometry"], case["rays"], g)))
     if kind == "trace":
         v, t = _geometry(case["geometry"], case["n"], g)
@@ -501,7 +502,7 @@ def exact(case, seed):
         g = _gen(seed)
         v, t = _geometry(case["geometry"], case["n"], g)
         _, h, p, q = _brute(_primary(case["geometry"], case["rays"], g), v, t)
-        tree = {} if case["presplit"] else {"woop": None, "ids": None}
+        tree = {} if case["presplit"] else {"woop": None}
         return {**tree, "hits": {"id": None, "t": h, "u": p, "v": q}}
     if kind == "trace":
         if case["any_hit"] or case["rays"] == "diffuse" or case["n"] * case["count"] > MOST_PAIRS:
