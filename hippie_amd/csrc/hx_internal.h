@@ -69,8 +69,8 @@ struct Tuning {
     int trace_lds_stack = 16;    // traversal-stack entries kept in LDS: 0, 16, 24, 32, 64
     int trace_fetch = 40;        // refill a wave when fewer lanes than this are still busy
     int trace_blocks_per_cu = 0; // persistent trace workgroups per CU (0 = occupancy limit)
-    int trace_postpone = 3;      // leaves a lane holds back while its wave traverses (1 to 4)
-    int trace_woop_ahead = 1;    // Woop rows of the next triangle read during a test (1 or 2)
+    int trace_postpone = 2;      // leaves a lane holds back while its wave traverses (1 to 4)
+    int trace_woop_ahead = 2;    // Woop rows of the next triangle read during a test (1 or 2)
     int sort_digit_bits = 8;     // radix digit width: 8 or 10
     int sort_items = 16;         // keys per thread in a sort pass: 8, 16 or 32
     int sort_lookback = 4;       // predecessor tiles read per look-back round trip: 4, 8 or 16
@@ -557,6 +557,8 @@ struct TraceArgs {
     const int32_t* order;   // optional: ray slot -> ray index (sorted trace)
     int32_t* control;       // [0] ray counter, [1] overflow counter
     int fetch_threshold;    // dynamic fetch: busy lanes below which a wave refills
+    int lanes;              // rays per wave, and the run length's divisor (set by the launch)
+    int run_shift;
     // Batched trace (else NULL): each ray traverses its own mesh's BVH.
     const int32_t* ray_mesh;
     const int4* mesh_tab;   // per mesh {node base, ...}

@@ -5,10 +5,10 @@
 // :572-842 (traceSort), rt/tracer/HipTracerKernels.h:29-199,
 // rt/ray/RayBufferKernels.cu:12-56,492-614.
 //
-// Wave64 design: each wave fetches rays for its terminated lanes with one
-// atomicAdd (64-bit ballot + mbcnt), traverses with the Aila-Laine
-// while-while loop, postpones one leaf per lane, and refills when fewer than
-// kDynamicFetch of its 64 lanes are still busy.
+// Wave64 design: each wave takes runs of rays for its terminated lanes (64-bit
+// ballot + mbcnt) from a pool of its own (RayPool), traverses with the
+// Aila-Laine while-while loop, postpones leaves, and refills when fewer than
+// fetch_threshold of its lanes are still busy.
 #include "hx_device.h"
 #include "hx_internal.h"
 
@@ -34,17 +34,66 @@ HX_DEV float span_end(float a0, float a1, float b0, float b1, float c0, float c1
     return __int_as_float(min(min(__float_as_int(fmax_s(a0, a1)), __float_as_int(fmax_s(b0, b1))), c));
 }
 
-// Bin node reads (k_trace).  A vector load of a node costs the CU's texture
-// address and data units four 16-byte-per-lane instructions however many lanes
-// share the node, and on coherent (sorted primary) rays those units, not the
-// ALUs, set the pace.  When every active lane of the wave visits the same node
-// -- the common case near the root for coherent rays -- the node is read with
-// scalar loads instead (constant address space: the trace never writes the
-// nodes), so no vector-memory instruction is issued for it.
-HX_DEV int64_t first_lane_i64(int64_t v) {
-    return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
-                     (uint32_t)__builtin_amdgcn_readfirstlane((int)v));
-}
+// The rays of one wave.  Every wave starts on its own run of rays and, when it
+// is used up, takes the next run with one atomicAdd on the launch's counter.
+// One atomic on one address per refill is what held traces back before: device
+// atomics on an address shared by the eight XCDs serialise at the memory side
+// (~10 ns each), and 1,048,576 rays half of which miss at the root take one per
+// ~24 rays.  With runs of up to kRunMax rays those rays went from 516 to 419 us
+// and 1,000,000 diffuse rays from 900 to 704 us.  Runs shrink with the rays left
+// (1 / (4 x waves) of them, at least one ray per lane) so that the last waves
+// finish together: a fixed run of 1/2 of a wave's share cost 15 % on 16.7M
+// diffuse rays, runs of 1024 rays cost 10 % on sorted primaries (3.51 against
+// 3.19 ms) since the waves of a CU then work far apart.
+constexpr int kRunMax = 256;
+struct RayPool {
+    int next, end;   // this wave's rays
+    int base;        // first ray of the latest run: the rays left start about here
+    int dyn0;        // first ray that is handed out by the counter
+    int n, lanes, shift;
+
+    HX_DEV int run() const { return max(lanes, min((n - base) >> shift, kRunMax)); }
+    HX_DEV void start(const TraceArgs& a) {
+        n = (int)a.n_rays;
+        lanes = a.lanes;
+        shift = a.run_shift;
+        base = 0;
+        const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kTraceBlock / kWave) + threadIdx.x / kWave);
+        const int r = run();
+        next = wave * r;
+        end = min(next + r, n);
+        dyn0 = base = (int)gridDim.x * (kTraceBlock / kWave) * r;
+    }
+    // A ray slot for each lane with `want` (>= n: none left); called by the
+    // whole wave.  mask, count: the lanes that want one.
+    HX_DEV int take(bool want, uint64_t mask, int count, int32_t* counter) {
+        const int below = count_below(mask);
+        const int avail = max(end - next, 0);
+        int mine = next + below;
+        if (count > avail) {
+            int first = n;
+            const int r = run();
+            if (base < n) {
+                if (want && below == 0) first = atomicAdd(counter, r);
+                first = dyn0 + __builtin_amdgcn_readlane(first, __ffsll((unsigned long long)mask) - 1);
+            }
+            if (below >= avail) mine = first + (below - avail);
+            base = first;
+            next = first + (count - avail);
+            end = min(first + r, n);
+        } else {
+            next += count;
+        }
+        return mine;
+    }
+};
+
+// SGPR budget of the trace kernels.  Above 80 scalar registers (96 with the
+// 16 the trap handler keeps) a SIMD holds 7 waves instead of 8 although the
+// occupancy query still says 8: 16.7M diffuse rays took 7.25 ms with 82 to 94
+// registers and 6.27 ms with 76 to 80.  The Bin kernel is held to the 64 vector
+// registers of 8 waves too (it needs 64 or 65).
+#define HX_TRACE_KERNEL __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_num_sgpr(80)))
 
 // Traversal stack: entries [0, LDS_DEPTH) in LDS, one column per lane (entry e
 // of lane t at e * kTraceBlock + t, so a wave's accesses hit distinct banks);
@@ -73,9 +122,19 @@ struct TraversalStack {
 // HipTracerBinKernels.cu:169-177; 2 is the reference's commented variant,
 // :171-173, 255; up to 4 here).  Held leaves wait in leafAddr (newest) ..
 // leafAddr4; a lane whose slots are full stops until its wave has a leaf in
-// every lane.  The closest hit does not depend on the order leaves are tested.
+// every lane, or until at most half of the wave's live lanes still look for one
+// (the lanes that wait cost more than the leaf phases saved: 16.7M diffuse rays
+// 6.62 -> 6.26 ms, 2M any-hit rays 1.79 -> 1.52 ms).  The closest hit does not
+// depend on the order leaves are tested; any-hit rays test theirs oldest first,
+// which is traversal order, so that the hit they report is the same however
+// many are held.
+//
+// Nodes are always read by vector loads.  Scalar loads when a whole wave visits
+// one node paid for themselves only while the ray counter set the pace; with
+// RayPool they cost 1,048,576 primaries 3 % and 16,384 rays 10 % (the check and
+// the scalar cache's latency) and gave sorted primaries nothing.
 template <bool STATS, bool ORDERED, int LDS_DEPTH, int POSTPONE, int AHEAD>
-__global__ __launch_bounds__(kTraceBlock) void k_trace(TraceArgs a) {
+HX_TRACE_KERNEL __attribute__((amdgpu_waves_per_eu(8))) void k_trace(TraceArgs a) {
     __shared__ int32_t s_stack[LDS_DEPTH > 0 ? LDS_DEPTH * kTraceBlock : 1];
     TraversalStack<LDS_DEPTH> stack;
     stack.col = (lds_i32*)(s_stack + threadIdx.x);
@@ -89,20 +148,17 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace(TraceArgs a) {
     int32_t nNodes = 0, nTris = 0;
     // Batched trace: this lane's mesh (node base, first triangle position).
     int64_t nodeBase = 0, triBase = 0;
-    int32_t* rayCounter = a.control;
+    if (lane_id() >= a.lanes) return;
+    RayPool pool;
+    pool.start(a);
 
     while (true) {
         // Fetch new rays for the terminated lanes of this wave.
         const bool terminated = nodeAddr == kSentinel;
         const uint64_t tmask = ballot64(terminated);
-        const int ntm = __popcll(tmask);
-        const int below = count_below(tmask);
-        const int leader = __ffsll((unsigned long long)tmask) - 1;
-        int base = 0;
-        if (terminated && below == 0) base = atomicAdd(rayCounter, ntm);
-        base = __shfl(base, leader, kWave);
+        const int slot = pool.take(terminated, tmask, __popcll(tmask), a.control);
         if (terminated) {
-            rayidx = (int64_t)base + below;
+            rayidx = slot;
             if (rayidx >= a.n_rays) break;
             if (ORDERED) rayidx = a.order[rayidx];
             if (a.ray_mesh) {
@@ -140,12 +196,22 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace(TraceArgs a) {
         }
 
         while (nodeAddr != kSentinel) {
+            const int half = __popcll(ballot64(true)) >> 1;
             while ((uint32_t)nodeAddr < (uint32_t)kSentinel) {
                 if (STATS) ++nNodes;
-                // The box test is written out in both branches so that, for a
-                // whole-wave node, it reads the scalar registers directly.
-                auto box_test = [&](float4 n0xy, float4 n1xy, float4 nz, float& c0min, float& c0max, float& c1min,
-                                    float& c1max) {
+                float c0min, c0max, c1min, c1max;
+                int2 cn;
+                {
+                    const int64_t na = nodeBase + nodeAddr;
+                    const float4* np = reinterpret_cast<const float4*>(a.nodes + 4 * na);
+                    const float4 n0xy = np[0];
+                    const float4 n1xy = np[1];
+                    const float4 nz = np[2];
+                    const int4 links = a.nodes[4 * na + 3];
+                    // The child links share the node's cache line: keep their
+                    // load with the box loads instead of after the box test.
+                    asm volatile("" ::"v"(links.x), "v"(links.y));
+                    cn = make_int2(links.x, links.y);
                     const float c0lox = fmaf(n0xy.x, idx, -oodx);
                     const float c0hix = fmaf(n0xy.y, idx, -oodx);
                     const float c0loy = fmaf(n0xy.z, idy, -oody);
@@ -162,32 +228,6 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace(TraceArgs a) {
                     const float c1hiy = fmaf(n1xy.w, idy, -oody);
                     c1min = span_begin(c1lox, c1hix, c1loy, c1hiy, c1loz, c1hiz, tmin);
                     c1max = span_end(c1lox, c1hix, c1loy, c1hiy, c1loz, c1hiz, hitT);
-                };
-                float c0min, c0max, c1min, c1max;
-                int2 cn;
-                {
-                    const int64_t na = nodeBase + nodeAddr;
-                    const int64_t n0 = first_lane_i64(na);
-                    if (__all(na == n0)) {
-                        typedef const __attribute__((address_space(4))) float const_f32;
-                        typedef const __attribute__((address_space(4))) int32_t const_i32;
-                        const_f32* f = (const_f32*)(a.nodes + 4 * n0);
-                        const_i32* w = (const_i32*)(a.nodes + 4 * n0);
-                        box_test(make_float4(f[0], f[1], f[2], f[3]), make_float4(f[4], f[5], f[6], f[7]),
-                                 make_float4(f[8], f[9], f[10], f[11]), c0min, c0max, c1min, c1max);
-                        cn = make_int2(w[12], w[13]);
-                    } else {
-                        const float4* np = reinterpret_cast<const float4*>(a.nodes + 4 * na);
-                        const float4 n0xy = np[0];
-                        const float4 n1xy = np[1];
-                        const float4 nz = np[2];
-                        const int4 links = a.nodes[4 * na + 3];
-                        // The child links share the node's cache line: keep their
-                        // load with the box loads instead of after the box test.
-                        asm volatile("" ::"v"(links.x), "v"(links.y));
-                        cn = make_int2(links.x, links.y);
-                        box_test(n0xy, n1xy, nz, c0min, c0max, c1min, c1max);
-                    }
                 }
                 const bool swp = c1min < c0min;
                 const bool t0 = c0max >= c0min;
@@ -215,13 +255,21 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace(TraceArgs a) {
                 const int32_t lastSlot = POSTPONE == 1 ? leafAddr : POSTPONE == 2 ? leafAddr2
                                          : POSTPONE == 3 ? leafAddr3 : leafAddr4;
                 if (nodeAddr < 0 && lastSlot >= 0) {
-                    if (POSTPONE >= 4) leafAddr4 = leafAddr3;
-                    if (POSTPONE >= 3) leafAddr3 = leafAddr2;
-                    if (POSTPONE >= 2) leafAddr2 = leafAddr;
-                    leafAddr = nodeAddr;
+                    if (a.any_hit) {
+                        const bool h1 = leafAddr < 0, h2 = leafAddr2 < 0, h3 = leafAddr3 < 0;
+                        if (POSTPONE >= 4) leafAddr4 = h3 ? nodeAddr : 0;
+                        if (POSTPONE >= 3) leafAddr3 = h2 && !h3 ? nodeAddr : leafAddr3;
+                        if (POSTPONE >= 2) leafAddr2 = h1 && !h2 ? nodeAddr : leafAddr2;
+                        leafAddr = h1 ? leafAddr : nodeAddr;
+                    } else {
+                        if (POSTPONE >= 4) leafAddr4 = leafAddr3;
+                        if (POSTPONE >= 3) leafAddr3 = leafAddr2;
+                        if (POSTPONE >= 2) leafAddr2 = leafAddr;
+                        leafAddr = nodeAddr;
+                    }
                     nodeAddr = stack.get(sp--);
                 }
-                if (!__any(leafAddr >= 0)) break;
+                if (!__any(leafAddr >= 0) || __popcll(ballot64(true)) <= half) break;
             }
 
             while (leafAddr < 0) {
@@ -339,7 +387,7 @@ struct WideStackSize {
 };
 
 template <int N, bool STATS, bool ORDERED, int LDS_DEPTH>
-__global__ __launch_bounds__(kTraceBlock) void k_trace_wide(TraceArgs a) {
+HX_TRACE_KERNEL void k_trace_wide(TraceArgs a) {
     constexpr int kSize = WideStackSize<N>::kSize;
     __shared__ int32_t s_stack[LDS_DEPTH > 0 ? LDS_DEPTH * kTraceBlock : 1];
     TraversalStack<LDS_DEPTH, kSize> stack;
@@ -351,20 +399,17 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_wide(TraceArgs a) {
     int32_t nodeAddr = kSentinel, leafAddr = 0, hitIndex = -1, hitId = -1;
     int64_t rayidx = 0;
     int32_t nNodes = 0, nTris = 0;
-    int32_t* rayCounter = a.control;
     const float4* nodes4 = reinterpret_cast<const float4*>(a.nodes);
+    if (lane_id() >= a.lanes) return;
+    RayPool pool;
+    pool.start(a);
 
     while (true) {
         const bool terminated = nodeAddr == kSentinel;
         const uint64_t tmask = ballot64(terminated);
-        const int ntm = __popcll(tmask);
-        const int below = count_below(tmask);
-        const int leader = __ffsll((unsigned long long)tmask) - 1;
-        int base = 0;
-        if (terminated && below == 0) base = atomicAdd(rayCounter, ntm);
-        base = __shfl(base, leader, kWave);
+        const int slot = pool.take(terminated, tmask, __popcll(tmask), a.control);
         if (terminated) {
-            rayidx = (int64_t)base + below;
+            rayidx = slot;
             if (rayidx >= a.n_rays) break;
             if (ORDERED) rayidx = a.order[rayidx];
             const float4 o = a.rays[2 * rayidx + 0];
@@ -387,12 +432,11 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_wide(TraceArgs a) {
             if (STATS) { nNodes = 0; nTris = 0; }
         }
         while (nodeAddr != kSentinel) {
+            const int half = __popcll(ballot64(true)) >> 1;
             while ((uint32_t)nodeAddr < (uint32_t)kSentinel) {
                 if (STATS) ++nNodes;
                 float dist[N];
                 int32_t link[N];
-                // Child c's test; written out in both node-read branches so that
-                // a whole-wave node is tested straight from scalar registers.
                 auto child_test = [&](int c, float4 xy, float4 zl) {
                     const float lox = fmaf(xy.x, idx, -oodx);
                     const float hix = fmaf(xy.y, idx, -oodx);
@@ -406,26 +450,15 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_wide(TraceArgs a) {
                     dist[c] = hit ? cmin : __int_as_float(0x7f800000);
                     link[c] = hit ? __float_as_int(zl.z) : kSentinel;
                 };
-                const int32_t n0 = __builtin_amdgcn_readfirstlane(nodeAddr);
-                if (__all(nodeAddr == n0)) {
-                    typedef const __attribute__((address_space(4))) float const_f32;
-                    const_f32* f = (const_f32*)(nodes4 + (int64_t)n0 * 2 * N);
+                const float4* np = nodes4 + (int64_t)nodeAddr * 2 * N;
+                float4 xys[N], zls[N];
 #pragma unroll
-                    for (int c = 0; c < N; ++c)
-                        child_test(c, make_float4(f[4 * c], f[4 * c + 1], f[4 * c + 2], f[4 * c + 3]),
-                                   make_float4(f[4 * (N + c)], f[4 * (N + c) + 1], f[4 * (N + c) + 2],
-                                               f[4 * (N + c) + 3]));
-                } else {
-                    const float4* np = nodes4 + (int64_t)nodeAddr * 2 * N;
-                    float4 xys[N], zls[N];
-#pragma unroll
-                    for (int c = 0; c < N; ++c) {
-                        xys[c] = np[c];
-                        zls[c] = np[N + c];
-                    }
-#pragma unroll
-                    for (int c = 0; c < N; ++c) child_test(c, xys[c], zls[c]);
+                for (int c = 0; c < N; ++c) {
+                    xys[c] = np[c];
+                    zls[c] = np[N + c];
                 }
+#pragma unroll
+                for (int c = 0; c < N; ++c) child_test(c, xys[c], zls[c]);
 #pragma unroll
                 for (int q = 0; q < WideNet<N>::kPairs; ++q) {
                     const int2 pr = WideNet<N>::pair(q);
@@ -458,7 +491,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_wide(TraceArgs a) {
                     leafAddr = nodeAddr;
                     nodeAddr = stack.get(sp--);
                 }
-                if (!__any(leafAddr >= 0)) break;
+                if (!__any(leafAddr >= 0) || __popcll(ballot64(true)) <= half) break;
             }
 
             while (leafAddr < 0) {
@@ -614,6 +647,26 @@ __global__ void k_zero_control(int32_t* control) {
     if (threadIdx.x < 2) control[threadIdx.x] = 0;
 }
 
+// Rays per wave, workgroups and run lengths of a launch.  A wave costs the same
+// whether 16 or 64 of its lanes carry rays, and lanes that diverge wait for each
+// other, so a launch that cannot fill the chip with full waves spreads its rays
+// over more of them: half as many rays per wave while that still leaves waves
+// idle, down to 16 (65,536 rays over 1M triangles 500 -> 357 us, 16,384 over
+// 64k 187 -> 157 us; 8 or 4 rays per wave were slower, 484 us, since the address
+// units take 4 lanes a cycle and neighbouring rays share nodes).
+unsigned trace_shape(Context* c, int occ, TraceArgs& a) {
+    const int per_cu = c->tune.trace_blocks_per_cu > 0 ? std::min(c->tune.trace_blocks_per_cu, occ) : occ;
+    const int64_t waves = (int64_t)c->cu_count * per_cu * (kTraceBlock / kWave);
+    a.lanes = kWave;
+    while (a.lanes > 16 && a.n_rays <= waves * (a.lanes / 2)) a.lanes /= 2;
+    a.run_shift = 2;
+    while (((int64_t)1 << (a.run_shift - 2)) < waves) ++a.run_shift;
+    a.fetch_threshold = std::max(1, a.fetch_threshold * a.lanes / kWave);
+    const int64_t per_block = (int64_t)a.lanes * (kTraceBlock / kWave);
+    return (unsigned)std::max<int64_t>(1, std::min<int64_t>((int64_t)c->cu_count * per_cu,
+                                                            (a.n_rays + per_block - 1) / per_block));
+}
+
 template <bool STATS, bool ORDERED, int LDS_DEPTH, int POSTPONE, int AHEAD>
 int launch_trace_t(Context* c, const TraceArgs& a) {
     // Occupancy limit of this instantiation, queried once per process.
@@ -624,11 +677,10 @@ int launch_trace_t(Context* c, const TraceArgs& a) {
                                                              kTraceBlock, 0));
         occ = std::max(q, 1);
     }
-    const int per_cu = c->tune.trace_blocks_per_cu > 0 ? std::min(c->tune.trace_blocks_per_cu, occ) : occ;
-    const int64_t want = (a.n_rays + kTraceBlock - 1) / kTraceBlock;
-    const unsigned blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>((int64_t)c->cu_count * per_cu, want));
+    TraceArgs t = a;
+    const unsigned blocks = trace_shape(c, occ, t);
     hipLaunchKernelGGL((k_trace<STATS, ORDERED, LDS_DEPTH, POSTPONE, AHEAD>), dim3(blocks), dim3(kTraceBlock), 0,
-                       c->stream, a);
+                       c->stream, t);
     return check_launch("trace");
 }
 
@@ -651,9 +703,8 @@ int launch_trace_ahead(Context* c, const TraceArgs& a) {
 
 template <bool STATS, bool ORDERED>
 int launch_trace_postpone(Context* c, const TraceArgs& a) {
-    // An any-hit trace reports the first hit in traversal order, which holding
-    // leaves back changes: it keeps the reference's one postponed leaf.
-    if (a.any_hit) return launch_trace_ahead<STATS, ORDERED, 1>(c, a);
+    // Counts of an any-hit trace stay those of the reference's one postponed leaf.
+    if (STATS && a.any_hit) return launch_trace_ahead<STATS, ORDERED, 1>(c, a);
     switch (c->tune.trace_postpone) {
         case 2: return launch_trace_ahead<STATS, ORDERED, 2>(c, a);
         case 3: return launch_trace_ahead<STATS, ORDERED, 3>(c, a);
@@ -671,10 +722,9 @@ int launch_trace_wide_t(Context* c, const TraceArgs& a) {
                                                              0));
         occ = std::max(q, 1);
     }
-    const int per_cu = c->tune.trace_blocks_per_cu > 0 ? std::min(c->tune.trace_blocks_per_cu, occ) : occ;
-    const int64_t want = (a.n_rays + kTraceBlock - 1) / kTraceBlock;
-    const unsigned blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>((int64_t)c->cu_count * per_cu, want));
-    hipLaunchKernelGGL((k_trace_wide<N, STATS, ORDERED, LDS_DEPTH>), dim3(blocks), dim3(kTraceBlock), 0, c->stream, a);
+    TraceArgs t = a;
+    const unsigned blocks = trace_shape(c, occ, t);
+    hipLaunchKernelGGL((k_trace_wide<N, STATS, ORDERED, LDS_DEPTH>), dim3(blocks), dim3(kTraceBlock), 0, c->stream, t);
     return check_launch("trace_wide");
 }
 
