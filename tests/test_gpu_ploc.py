@@ -111,3 +111,12 @@ def test_ploc_rebuild_reuses_handle(oracle, ctx):
     cg = oracle.bin_canonical(bvh.nodes_host(), bvh.n_interior, bvh.n_leaves, bvh.tri_indices_host())
     co = oracle.bin_canonical(ref["nodes"], ref["n_interior"], ref["n_leaves"], ref["tri_idx"])
     assert np.array_equal(cg, co)
+
+
+# Tiles of 1024 clusters, the one-workgroup tail from 2048 down, and the widest
+# window that fits in LDS (r = 1024).
+@pytest.mark.parametrize("n", [2, 3, 1023, 1024, 1025, 2047, 2048, 2049, 3073, 5000])
+@pytest.mark.parametrize("radius", [1, 3, 26, 1024, 1025])
+def test_ploc_tile_and_window_edges(oracle, ctx, n, radius):
+    v, t = scenes.merge(scenes.uniform_soup(n - n // 2, seed=n), scenes.gaussian_mixture_soup(n // 2, seed=radius))
+    _check(oracle, ctx, v, t, radius, max_radius=2048)
