@@ -134,7 +134,7 @@ struct TraversalStack {
 // RayPool they cost 1,048,576 primaries 3 % and 16,384 rays 10 % (the check and
 // the scalar cache's latency) and gave sorted primaries nothing.
 template <bool STATS, bool ORDERED, int LDS_DEPTH, int POSTPONE, int AHEAD>
-HX_TRACE_KERNEL __attribute__((amdgpu_waves_per_eu(8))) void k_trace(TraceArgs a) {
+HX_TRACE_KERNEL __attribute__((amdgpu_waves_per_eu(LDS_DEPTH <= 16 ? 8 : 1))) void k_trace(TraceArgs a) {
     __shared__ int32_t s_stack[LDS_DEPTH > 0 ? LDS_DEPTH * kTraceBlock : 1];
     TraversalStack<LDS_DEPTH> stack;
     stack.col = (lds_i32*)(s_stack + threadIdx.x);
