@@ -187,7 +187,7 @@ struct hx_bvh {
     int wide = 0;
     bool wide_lbvh_root = false;
     int64_t wide_entries = 0;
-    DevBuf wide_cost, wide_cnt, e_b, e_budget, e_leaf, e_parent, e_rank, e_first, e_nchild, wide_scan, wide_partial;
+    DevBuf wide_cost, wide_cnt, e_b, e_budget, e_leaf, e_parent, e_rank, e_first, e_nchild, wide_levels, wide_partial;
     float host_box[6] = {0, 0, 0, 0, 0, 0};
     bool box_known = false;
 };
@@ -434,9 +434,9 @@ int run_presplit(hx_bvh* b) {
     Context* c = &b->ctx->c;
     const int64_t n = b->n_tri;
     const int M = b->batched ? b->n_meshes : 1;
-    const int64_t ntiles = (n + 4095) / 4096;
+    const int64_t ntiles = (n + hx::kPsTile - 1) / hx::kPsTile;
     HX_TRY(b->ps_prio.reserve(4 * (size_t)n));
-    HX_TRY(b->ps_work.reserve(16 * (size_t)M + 4 * (size_t)M + 4 * (size_t)ntiles + 2048));
+    HX_TRY(b->ps_work.reserve((16 + 4 + 8 + 8 + 8) * (size_t)M + 4 * (size_t)ntiles + 4096));
     hx::PsArgs a{};
     a.n = n;
     a.verts = b->verts;
@@ -455,7 +455,10 @@ int run_presplit(hx_bvh* b) {
     };
     a.macc = reinterpret_cast<unsigned long long*>(carve_w(16 * (size_t)M));
     a.Dm = reinterpret_cast<float*>(carve_w(4 * (size_t)M));
-    a.qcount = reinterpret_cast<int32_t*>(carve_w(8));
+    a.smax = reinterpret_cast<int64_t*>(carve_w(8 * (size_t)M));
+    a.sum1 = reinterpret_cast<int64_t*>(carve_w(8 * (size_t)M));
+    a.dlim = reinterpret_cast<float*>(carve_w(8 * (size_t)M));
+    a.qcount = reinterpret_cast<int32_t*>(carve_w(16));
     a.partial = reinterpret_cast<int32_t*>(carve_w(4 * (size_t)ntiles));
     std::vector<int64_t> tri_counts(M), ref_counts(M);
     std::vector<float> D(M);
@@ -922,8 +925,8 @@ hx::WideArgs wide_args(hx_bvh* b, bool lbvh_root) {
     a.e_rank = b->e_rank.as<int32_t>();
     a.e_first = b->e_first.as<int32_t>();
     a.e_nchild = b->e_nchild.as<int32_t>();
-    a.scan = b->wide_scan.as<int2>();
-    a.scan_part = b->wide_scan.as<int2>() + (2 * b->n_refs + 1);
+    a.rec = b->wide_levels.as<int4>();
+    a.partial = reinterpret_cast<int2*>(a.rec + hx::kWideRecords);
     a.nodes = b->nodes.as<int4>();
     return a;
 }
@@ -938,7 +941,7 @@ int run_wide(hx_bvh* b, bool lbvh_root) {
         HX_TRY(d->reserve(4 * (size_t)(2 * n)));
     HX_TRY(b->e_budget.reserve((size_t)(2 * n)));
     HX_TRY(b->e_leaf.reserve((size_t)(2 * n)));
-    HX_TRY(b->wide_scan.reserve(8 * (size_t)(2 * n + 1 + (2 * n) / 2048 + 2)));
+    HX_TRY(b->wide_levels.reserve(sizeof(int4) * hx::kWideRecords + sizeof(int2) * hx::kWidePartials));
     int64_t ni = 0, nl = 0, ne = 0;
     HX_TRY(hx::launch_wide_build(c, wide_args(b, lbvh_root), &ni, &nl, &ne));
     b->wide = N;

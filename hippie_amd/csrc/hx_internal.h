@@ -336,16 +336,20 @@ struct PsArgs {
     float* Dm;                  // per-mesh multiplier (M floats, device)
     float* prio;                // n
     unsigned long long* macc;   // 2 per mesh: priority fixed-point sum, budget sum
-    int32_t* partial;           // one entry per 4096 triangles
+    int64_t* smax;              // per mesh: the reference budget,
+    int64_t* sum1;              //   the priority sum's integer part,
+    float* dlim;                //   and the bisection bounds of D (min, max)
+    int32_t* partial;           // one entry per kPsTile triangles
     float4* ref_min;            // n_refs
     float4* ref_max;
     int32_t* ref_tri;
     int4* task[2];              // (triangle, budget, first slot, 0)
     float4* tmn[2];
     float4* tmx[2];
-    int32_t* qcount;            // 2
+    int32_t* qcount;            // 4: three counts in turn, and the largest one
     int64_t queue_cap;
 };
+constexpr int kPsTile = 1024;
 // Host float -> int with the device convert's saturation (NaN -> 0).
 inline int32_t f2i_host(float x) {
     if (x != x) return 0;
@@ -462,6 +466,7 @@ int launch_sort_pairs(Context* c, void* keys[2], int32_t* vals[2], int64_t n, in
 // hx_wide.hip: Quad / Oct layouts from a built binary tree (internal nodes
 // 0..n-2 with left/right/parent and inclusive leaf ranges first/last, leaves
 // n-1+p, boxes of all 2n-1 nodes) and their traversal.
+constexpr int kWidePartials = 2048, kWideRecords = 16;
 struct WideArgs {
     int64_t n;
     int N;                    // children per node: 4 or 8
@@ -489,8 +494,8 @@ struct WideArgs {
     int32_t* e_rank;
     int32_t* e_first;
     int32_t* e_nchild;
-    int2* scan;               // per-level counts, 2n + 1
-    int2* scan_part;          // their per-block sums, 2n / 2048 + 2
+    int2* partial;            // per-workgroup counts of a level, kWidePartials
+    int4* rec;                // level records, kWideRecords
     int4* nodes;              // out: 2N int4 per node
 };
 int launch_wide_build(Context* c, const WideArgs& a, int64_t* n_interior, int64_t* n_leaves, int64_t* n_entries);

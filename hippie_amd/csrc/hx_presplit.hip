@@ -35,8 +35,8 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
-constexpr int kItems = 16;
-constexpr int kTile = kBlock * kItems;
+constexpr int kItems = kPsTile / kBlock;
+constexpr int kTile = kPsTile;
 
 inline unsigned grid_for(int64_t n, int block = kBlock) { return (unsigned)((n + block - 1) / block); }
 
@@ -138,9 +138,10 @@ HX_DEV const float* frame_box(const PsArgs& a, int m) { return a.mesh_of ? a.mes
 // Per-mesh sums acc[2 * m + k] accumulated by a wave over its iterations:
 // while the wave's live lanes share the mesh of the running sum it grows in
 // registers, and it goes out with one device-scope atomic when the mesh
-// changes or the wave ends (device atomics on one word serialise, so a
-// per-wave atomic over 16M references would take milliseconds).  Waves
-// whose lanes span meshes add per lane.
+// changes (device atomics on one word serialise, so a per-wave atomic over 16M
+// references would take milliseconds).  Waves whose lanes span meshes add per
+// lane.  At the end the waves of the workgroup join their last runs, so a
+// workgroup inside one mesh costs one atomic.
 struct MeshSum {
     unsigned long long* acc;
     int k;
@@ -149,6 +150,23 @@ struct MeshSum {
     HX_DEV void flush() {
         if (m >= 0 && s && lane_id() == 0) atomicAdd(acc + 2 * (int64_t)m + k, s);
         s = 0;
+    }
+    // The last runs of the workgroup's waves; every thread calls it.
+    HX_DEV void finish() {
+        __shared__ unsigned long long sums[kWavesPerBlock];
+        __shared__ int meshes[kWavesPerBlock];
+        if (lane_id() == 0) {
+            sums[threadIdx.x / kWave] = s;
+            meshes[threadIdx.x / kWave] = m;
+        }
+        __syncthreads();
+        if (threadIdx.x != 0) return;
+        for (int w = 0; w < kWavesPerBlock;) {
+            const int mesh = meshes[w];
+            unsigned long long v = 0;
+            for (; w < kWavesPerBlock && meshes[w] == mesh; ++w) v += sums[w];
+            if (mesh >= 0 && v) atomicAdd(acc + 2 * (int64_t)mesh + k, v);
+        }
     }
     HX_DEV void add(bool live, int mesh, unsigned long long v) {
         const uint64_t act = ballot64(live);
@@ -173,8 +191,15 @@ struct MeshSum {
     }
 };
 
-// Each workgroup takes kSumChunk consecutive references.
-constexpr int kSumChunk = 64 * kBlock;
+// Each workgroup of a sum takes `chunk` consecutive triangles, so that about
+// kSumBlocks workgroups cover them: enough to fill the chip, few enough that
+// their atomics on one word stay cheap (16,384 triangles each left 31
+// workgroups for 500,009: 176 us for the priorities and 39 us for a round of
+// the bisection, now 22 and 10 us).
+constexpr int kSumBlocks = 512;
+inline int64_t sum_chunk(int64_t n) {
+    return std::max<int64_t>((n + kSumBlocks - 1) / kSumBlocks + kBlock - 1, kBlock) / kBlock * kBlock;
+}
 
 // computePriorities (:11-71).
 HX_DEV float priority(const float3 v[3], const SceneFrame& S) {
@@ -195,11 +220,10 @@ HX_DEV float priority(const float3 v[3], const SceneFrame& S) {
 }
 
 // Priorities and their exact fixed-point sums per mesh (macc[2m]).
-__global__ __launch_bounds__(kBlock) void k_ps_priority(PsArgs a) {
+__global__ __launch_bounds__(kBlock) void k_ps_priority(PsArgs a, int64_t chunk) {
     MeshSum sum{a.macc, 0};
-    const int64_t end = min((int64_t)(blockIdx.x + 1) * kSumChunk, a.n);
-    for (int64_t t = blockIdx.x * (int64_t)kSumChunk + threadIdx.x; t < (int64_t)(blockIdx.x + 1) * kSumChunk;
-         t += kBlock) {
+    const int64_t end = min((int64_t)(blockIdx.x + 1) * chunk, a.n);
+    for (int64_t t = blockIdx.x * chunk + threadIdx.x; t < (int64_t)(blockIdx.x + 1) * chunk; t += kBlock) {
         const bool live = t < end;
         unsigned long long s = 0;
         int m = 0;
@@ -214,15 +238,14 @@ __global__ __launch_bounds__(kBlock) void k_ps_priority(PsArgs a) {
         }
         sum.add(live, m, s);
     }
-    sum.flush();
+    sum.finish();
 }
 
 // sumPrioritiesRound (:116-148): per-mesh sums of floor(D_m p) (macc[2m+1]).
-__global__ __launch_bounds__(kBlock) void k_ps_round_sum(PsArgs a) {
+__global__ __launch_bounds__(kBlock) void k_ps_round_sum(PsArgs a, int64_t chunk) {
     MeshSum sum{a.macc, 1};
-    const int64_t end = min((int64_t)(blockIdx.x + 1) * kSumChunk, a.n);
-    for (int64_t t = blockIdx.x * (int64_t)kSumChunk + threadIdx.x; t < (int64_t)(blockIdx.x + 1) * kSumChunk;
-         t += kBlock) {
+    const int64_t end = min((int64_t)(blockIdx.x + 1) * chunk, a.n);
+    for (int64_t t = blockIdx.x * chunk + threadIdx.x; t < (int64_t)(blockIdx.x + 1) * chunk; t += kBlock) {
         const bool live = t < end;
         unsigned long long s = 0;
         int m = 0;
@@ -232,7 +255,7 @@ __global__ __launch_bounds__(kBlock) void k_ps_round_sum(PsArgs a) {
         }
         sum.add(live, m, s);
     }
-    sum.flush();
+    sum.finish();
 }
 
 // Per-tile sums of floor(D p) + 1.
@@ -254,14 +277,17 @@ __global__ __launch_bounds__(kBlock) void k_ps_tile_sums(PsArgs a) {
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_ps_scan(int32_t* __restrict__ partial, int count) {
-    __shared__ int wt[kWavesPerBlock];
+constexpr int kScanBlock = 1024;
+__global__ __launch_bounds__(kScanBlock) void k_ps_scan(int32_t* __restrict__ partial, int count,
+                                                        int32_t* __restrict__ qcount) {
+    __shared__ int wt[kScanBlock / kWave];
+    if (threadIdx.x < 4) qcount[threadIdx.x] = 0;
     int carry = 0;
-    for (int base = 0; base < count; base += kBlock) {
+    for (int base = 0; base < count; base += kScanBlock) {
         const int t = base + threadIdx.x;
         const int v = t < count ? partial[t] : 0;
         int tot;
-        const int inc = block_inclusive_scan<kWavesPerBlock>(v, Sum(), wt, tot);
+        const int inc = block_inclusive_scan<kScanBlock / kWave>(v, Sum(), wt, tot);
         if (t < count) partial[t] = carry + inc - v;
         carry += tot;
     }
@@ -273,22 +299,46 @@ HX_DEV void write_ref(const PsArgs& a, int off, int tri, const Box3& b) {
     a.ref_tri[off] = tri;
 }
 
-// Append a task to queue q (wave-aggregated slot reservation; the order of
-// the queue does not matter, every task carries its output slots).
-HX_DEV void push_task(const PsArgs& a, int q, bool live, int tri, int count, int off, const Box3& b) {
-    const uint64_t m = ballot64(live);
-    if (!m) return;
-    const int leader = __builtin_ctzll(m);
-    int base = 0;
-    if (lane_id() == leader) base = atomicAdd(a.qcount + q, __builtin_popcountll(m));
-    base = __shfl(base, leader, kWave);
-    if (live) {
-        const int slot = base + count_below(m);
-        if (slot >= a.queue_cap) return;  // reported by the host from the count
-        a.task[q][slot] = make_int4(tri, count, off, 0);
-        a.tmn[q][slot] = make_float4(b.mn.x, b.mn.y, b.mn.z, 0.0f);
-        a.tmx[q][slot] = make_float4(b.mx.x, b.mx.y, b.mx.z, 0.0f);
+// Append tasks to queue q, counted in qcount[cnt] (the order of the queue does
+// not matter, every task carries its output slots).  The R batches of tasks of a
+// workgroup share one slot reservation: one atomic per wave on the one counter
+// (~10 ns each) was most of the first pass, 63 us for 500,009 triangles, now
+// 16 us.  reserve: first slot of batch r for this thread's lane, every
+// thread of the workgroup calls it.
+template <int R>
+HX_DEV void reserve_slots(const PsArgs& a, int cnt, const bool (&live)[R], int (&slot)[R]) {
+    __shared__ int s_base[R][kWavesPerBlock];
+    const int w = threadIdx.x / kWave;
+    uint64_t m[R];
+    __syncthreads();  // the previous reservation has been read
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        m[r] = ballot64(live[r]);
+        if (lane_id() == 0) s_base[r][w] = __popcll(m[r]);
     }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int tot = 0;
+        for (int r = 0; r < R; ++r)
+            for (int v = 0; v < kWavesPerBlock; ++v) {
+                const int x = s_base[r][v];
+                s_base[r][v] = tot;
+                tot += x;
+            }
+        const int base = tot ? atomicAdd(a.qcount + cnt, tot) : 0;
+        for (int r = 0; r < R; ++r)
+            for (int v = 0; v < kWavesPerBlock; ++v) s_base[r][v] += base;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) slot[r] = s_base[r][w] + count_below(m[r]);
+}
+
+HX_DEV void push_task(const PsArgs& a, int q, int slot, bool live, int tri, int count, int off, const Box3& b) {
+    if (!live || slot >= a.queue_cap) return;  // an overflow is reported by the host from the count
+    a.task[q][slot] = make_int4(tri, count, off, 0);
+    a.tmn[q][slot] = make_float4(b.mn.x, b.mn.y, b.mn.z, 0.0f);
+    a.tmx[q][slot] = make_float4(b.mx.x, b.mx.y, b.mx.z, 0.0f);
 }
 
 // initSplitTasks (:150-187): slot offsets from the tile scan; an unsplit
@@ -297,10 +347,20 @@ __global__ __launch_bounds__(kBlock) void k_ps_init(PsArgs a) {
     __shared__ int wt[kWavesPerBlock];
     const int64_t base = blockIdx.x * (int64_t)kTile;
     int carry = a.partial[blockIdx.x];
+    int budget[kItems], slot[kItems];
+    bool split[kItems];
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) {
+        const int64_t t = base + k * kBlock + threadIdx.x;
+        budget[k] = t < a.n ? f2i_sat(a.Dm[mesh_at(a, (int)t)] * a.prio[t]) : 0;
+        split[k] = budget[k] > 0;
+    }
+    reserve_slots(a, 0, split, slot);
+#pragma unroll
     for (int k = 0; k < kItems; ++k) {
         const int64_t t = base + k * kBlock + threadIdx.x;
         const bool in = t < a.n;
-        const int cnt = in ? f2i_sat(a.Dm[mesh_at(a, (int)t)] * a.prio[t]) : 0;
+        const int cnt = budget[k];
         const int w = in ? cnt + 1 : 0;
         int tot;
         const int inc = block_inclusive_scan<kWavesPerBlock>(w, Sum(), wt, tot);
@@ -313,15 +373,13 @@ __global__ __launch_bounds__(kBlock) void k_ps_init(PsArgs a) {
             b = tri_bounds(v);
             if (cnt == 0) write_ref(a, off, (int)t, b);
         }
-        push_task(a, 0, in && cnt > 0, (int)t, cnt, off, b);
+        push_task(a, 0, slot[k], split[k], (int)t, cnt, off, b);
     }
 }
 
 // split (:189-419) of every queued task into two children; a child with no
 // budget left is written as a reference, the others go to the next queue.
-__global__ __launch_bounds__(kBlock) void k_ps_split(PsArgs a, int q, int count) {
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    const bool live = k < count;
+HX_DEV void split_task(const PsArgs& a, int q, int next, bool live, int k) {
     int tri = 0, lc = 0, rc = 0, loff = 0, roff = 0;
     Box3 lb = box_empty(), rb = box_empty();
     if (live) {
@@ -394,8 +452,28 @@ __global__ __launch_bounds__(kBlock) void k_ps_split(PsArgs a, int q, int count)
         if (lc <= 0) write_ref(a, loff, tri, lb);
         if (rc <= 0) write_ref(a, roff, tri, rb);
     }
-    push_task(a, q ^ 1, live && lc > 0, tri, lc, loff, lb);
-    push_task(a, q ^ 1, live && rc > 0, tri, rc, roff, rb);
+    const bool again[2] = {live && lc > 0, live && rc > 0};
+    int slot[2];
+    reserve_slots(a, next, again, slot);
+    push_task(a, q ^ 1, slot[0], again[0], tri, lc, loff, lb);
+    push_task(a, q ^ 1, slot[1], again[1], tri, rc, roff, rb);
+}
+
+// Split round `round`: the tasks of queue round & 1, counted in qcount[round % 3],
+// into the other queue, counted in the next word; the word after that is cleared
+// for the round to come, and qcount[3] keeps the largest count.  The rounds read
+// their counts on the device, so the host reads one count per batch of rounds
+// instead of one per round; an empty round costs a launch.
+__global__ __launch_bounds__(kBlock) void k_ps_split(PsArgs a, int round) {
+    const int cur = round % 3, next = (round + 1) % 3;
+    const int count = a.qcount[cur];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        a.qcount[(round + 2) % 3] = 0;
+        if (count > a.qcount[3]) a.qcount[3] = count;
+    }
+    const int64_t todo = min((int64_t)count, a.queue_cap);
+    for (int64_t base = blockIdx.x * (int64_t)kBlock; base < todo; base += (int64_t)gridDim.x * kBlock)
+        split_task(a, round & 1, next, base + threadIdx.x < todo, (int)(base + threadIdx.x));
 }
 
 __global__ void k_ps_zero_u64(unsigned long long* p, int64_t n) {
@@ -403,31 +481,42 @@ __global__ void k_ps_zero_u64(unsigned long long* p, int64_t n) {
         p[i] = 0ull;
 }
 
-__global__ void k_ps_zero_q(int32_t* qcount, int q) {
-    if (threadIdx.x == 0) qcount[q] = 0;
-}
+constexpr int kSplitBatch = 4;       // split rounds launched between host reads
+constexpr int kSplitBlocks = 2048;
 
-__global__ void k_ps_zero_both(int32_t* qcount) {
-    if (threadIdx.x < 2) qcount[threadIdx.x] = 0;
-}
-
-// Per-mesh round sums of floor(D_m p) for the multipliers `D` (M entries).
-unsigned sum_blocks(int64_t n) { return (unsigned)std::max<int64_t>(1, (n + kSumChunk - 1) / kSumChunk); }
-
-int round_sums(Context* c, const PsArgs& a, int M, const std::vector<float>& D, std::vector<int64_t>& out) {
-    HX_HIP(hipMemcpyAsync(a.Dm, D.data(), sizeof(float) * (size_t)M, hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(k_ps_zero_u64, dim3(std::min<unsigned>(grid_for(2 * (int64_t)M), 1024u)), dim3(kBlock), 0,
-                       c->stream, a.macc, 2 * (int64_t)M);
-    HX_TRY(check_launch("ps_zero"));
-    hipLaunchKernelGGL(k_ps_round_sum, dim3(sum_blocks(a.n)), dim3(kBlock), 0, c->stream, a);
-    HX_TRY(check_launch("ps_round_sum"));
-    std::vector<unsigned long long> h(2 * (size_t)M);
-    HX_HIP(hipMemcpyAsync(h.data(), a.macc, sizeof(unsigned long long) * h.size(), hipMemcpyDeviceToHost,
-                          c->stream));
-    HX_HIP(hipStreamSynchronize(c->stream));
-    out.resize(M);
-    for (int m = 0; m < M; ++m) out[m] = (int64_t)h[2 * (size_t)m + 1];
-    return HX_OK;
+// computeD (Presplitter.cpp:124-155) for every mesh, Smax = (int)(beta * n_m); a
+// mesh whose priority sum floors to 0 gets D = 0 (no splits).  Step 0 takes the
+// priority sums and sets the first multiplier, step 1 the bounds from its
+// rounded sum, steps 2..7 a bisection each; after step kBisect + 1 Dm is the
+// lower bound.  Clears the sums for the next round.  On the device, the eight
+// rounds run without the host (each was a round trip of 40 to 75 us).
+constexpr int kBisect = 6;
+__global__ __launch_bounds__(kBlock) void k_ps_bisect(PsArgs a, int M, int step) {
+    const int m = blockIdx.x * kBlock + threadIdx.x;
+    if (m >= M) return;
+    const int64_t smax = a.smax[m];
+    float dmin = a.dlim[2 * m], dmax = a.dlim[2 * m + 1];
+    if (step == 0) {
+        const int64_t s1 = (int64_t)(a.macc[2 * (int64_t)m] >> 32);
+        a.sum1[m] = s1;
+        dmin = s1 > 0 ? (float)(smax / s1) : 0.0f;
+        dmax = 0.0f;
+    }
+    const bool live = a.sum1[m] > 0;
+    const int64_t s = (int64_t)a.macc[2 * (int64_t)m + 1];
+    if (step == 1) {
+        dmax = live ? (dmin * (float)smax) / (float)s : 0.0f;
+    } else if (step > 1 && live) {
+        const float cur = 0.5f * (dmin + dmax);
+        if (s > smax) dmax = cur;
+        else dmin = cur;
+    }
+    a.dlim[2 * m] = dmin;
+    a.dlim[2 * m + 1] = dmax;
+    const bool bisecting = step >= 1 && step <= kBisect;
+    a.Dm[m] = bisecting ? (live ? 0.5f * (dmin + dmax) : 0.0f) : dmin;
+    a.macc[2 * (int64_t)m] = 0;
+    a.macc[2 * (int64_t)m + 1] = 0;
 }
 
 __global__ __launch_bounds__(kBlock) void k_refs_to_tris(int32_t* __restrict__ ids, const int32_t* __restrict__ ref_tri,
@@ -446,47 +535,28 @@ int launch_refs_to_tris(Context* c, int32_t* ids, const int32_t* ref_tri, int64_
 int launch_presplit_count(Context* c, const PsArgs& a, float beta, int M, const int64_t* tri_counts,
                           int64_t* ref_counts, float* D_out) {
     LaunchScope ls(c, "presplit_count");
+    const int64_t chunk = sum_chunk(a.n);
+    const dim3 blocks((unsigned)((a.n + chunk - 1) / chunk));
+    std::vector<int64_t> smax(M);
+    for (int m = 0; m < M; ++m) smax[m] = f2i_host(beta * (float)tri_counts[m]);
+    HX_HIP(hipMemcpyAsync(a.smax, smax.data(), sizeof(int64_t) * (size_t)M, hipMemcpyHostToDevice, c->stream));
     hipLaunchKernelGGL(k_ps_zero_u64, dim3(std::min<unsigned>(grid_for(2 * (int64_t)M), 1024u)), dim3(kBlock), 0,
                        c->stream, a.macc, 2 * (int64_t)M);
     HX_TRY(check_launch("ps_zero"));
-    hipLaunchKernelGGL(k_ps_priority, dim3(sum_blocks(a.n)), dim3(kBlock), 0, c->stream, a);
+    hipLaunchKernelGGL(k_ps_priority, blocks, dim3(kBlock), 0, c->stream, a, chunk);
     HX_TRY(check_launch("ps_priority"));
+    for (int step = 0; step <= kBisect + 1; ++step) {
+        hipLaunchKernelGGL(k_ps_bisect, dim3(grid_for(M)), dim3(kBlock), 0, c->stream, a, M, step);
+        HX_TRY(check_launch("ps_bisect"));
+        hipLaunchKernelGGL(k_ps_round_sum, blocks, dim3(kBlock), 0, c->stream, a, chunk);
+        HX_TRY(check_launch("ps_round_sum"));
+    }
     std::vector<unsigned long long> h(2 * (size_t)M);
     HX_HIP(hipMemcpyAsync(h.data(), a.macc, sizeof(unsigned long long) * h.size(), hipMemcpyDeviceToHost,
                           c->stream));
+    HX_HIP(hipMemcpyAsync(D_out, a.Dm, sizeof(float) * (size_t)M, hipMemcpyDeviceToHost, c->stream));
     HX_HIP(hipStreamSynchronize(c->stream));
-    // computeD (Presplitter.cpp:124-155) per mesh, Smax = (int)(beta * n_m);
-    // a mesh whose priority sum floors to 0 gets D = 0 (no splits).
-    std::vector<int64_t> smax(M), s1(M), s;
-    std::vector<float> dmin(M, 0.0f), dmax(M, 0.0f), cur(M, 0.0f);
-    std::vector<char> live(M, 0);
-    bool any = false;
-    for (int m = 0; m < M; ++m) {
-        smax[m] = f2i_host(beta * (float)tri_counts[m]);
-        s1[m] = (int64_t)(h[2 * (size_t)m] >> 32);
-        live[m] = s1[m] > 0;
-        any = any || live[m];
-        if (live[m]) dmin[m] = (float)(smax[m] / s1[m]);
-    }
-    if (any) {
-        HX_TRY(round_sums(c, a, M, dmin, s));
-        for (int m = 0; m < M; ++m)
-            if (live[m]) dmax[m] = (dmin[m] * (float)smax[m]) / (float)s[m];
-        for (int r = 0; r < 6; ++r) {
-            for (int m = 0; m < M; ++m) cur[m] = live[m] ? 0.5f * (dmin[m] + dmax[m]) : 0.0f;
-            HX_TRY(round_sums(c, a, M, cur, s));
-            for (int m = 0; m < M; ++m) {
-                if (!live[m]) continue;
-                if (s[m] > smax[m]) dmax[m] = cur[m];
-                else dmin[m] = cur[m];
-            }
-        }
-    }
-    HX_TRY(round_sums(c, a, M, dmin, s));
-    for (int m = 0; m < M; ++m) {
-        ref_counts[m] = tri_counts[m] + s[m];
-        D_out[m] = dmin[m];
-    }
+    for (int m = 0; m < M; ++m) ref_counts[m] = tri_counts[m] + (int64_t)h[2 * (size_t)m + 1];
     return HX_OK;
 }
 
@@ -494,34 +564,30 @@ int launch_presplit_refs(Context* c, const PsArgs& a, int64_t n_refs) {
     LaunchScope ls(c, "presplit_split");
     const int64_t n = a.n;
     const int ntiles = (int)((n + kTile - 1) / kTile);
-    hipLaunchKernelGGL(k_ps_zero_both, dim3(1), dim3(64), 0, c->stream, a.qcount);
-    HX_TRY(check_launch("ps_zero"));
     hipLaunchKernelGGL(k_ps_tile_sums, dim3(ntiles), dim3(kBlock), 0, c->stream, a);
     HX_TRY(check_launch("ps_tile_sums"));
-    hipLaunchKernelGGL(k_ps_scan, dim3(1), dim3(kBlock), 0, c->stream, a.partial, ntiles);
+    hipLaunchKernelGGL(k_ps_scan, dim3(1), dim3(kScanBlock), 0, c->stream, a.partial, ntiles, a.qcount);
     HX_TRY(check_launch("ps_scan"));
     hipLaunchKernelGGL(k_ps_init, dim3(ntiles), dim3(kBlock), 0, c->stream, a);
     HX_TRY(check_launch("ps_init"));
-    int q = 0;
-    int32_t count = 0;
-    HX_HIP(hipMemcpyAsync(&count, a.qcount + q, sizeof(count), hipMemcpyDeviceToHost, c->stream));
-    HX_HIP(hipStreamSynchronize(c->stream));
     // Every split consumes one unit of budget, so the rounds end; the bound
     // guards against a miscount.
-    for (int64_t round = 0; count > 0; ++round) {
-        if ((int64_t)count > a.queue_cap || round > n_refs) {
-            set_error("presplit: split queue overflow (%d tasks, capacity %lld)", count, (long long)a.queue_cap);
+    const unsigned grid = std::min<unsigned>(grid_for(a.queue_cap), kSplitBlocks);
+    int32_t q[4];
+    for (int round = 0;;) {
+        for (int k = 0; k < kSplitBatch; ++k, ++round) {
+            hipLaunchKernelGGL(k_ps_split, dim3(grid), dim3(kBlock), 0, c->stream, a, round);
+            HX_TRY(check_launch("ps_split"));
+        }
+        HX_HIP(hipMemcpyAsync(q, a.qcount, sizeof(q), hipMemcpyDeviceToHost, c->stream));
+        HX_HIP(hipStreamSynchronize(c->stream));
+        const int32_t most = std::max(q[3], q[round % 3]);
+        if ((int64_t)most > a.queue_cap || round > n_refs + kSplitBatch) {
+            set_error("presplit: split queue overflow (%d tasks, capacity %lld)", most, (long long)a.queue_cap);
             return HX_ERR_HIP;
         }
-        hipLaunchKernelGGL(k_ps_zero_q, dim3(1), dim3(64), 0, c->stream, a.qcount, q ^ 1);
-        HX_TRY(check_launch("ps_zero_q"));
-        hipLaunchKernelGGL(k_ps_split, dim3(grid_for(count)), dim3(kBlock), 0, c->stream, a, q, (int)count);
-        HX_TRY(check_launch("ps_split"));
-        q ^= 1;
-        HX_HIP(hipMemcpyAsync(&count, a.qcount + q, sizeof(count), hipMemcpyDeviceToHost, c->stream));
-        HX_HIP(hipStreamSynchronize(c->stream));
+        if (q[round % 3] == 0) return HX_OK;
     }
-    return HX_OK;
 }
 
 }  // namespace hx

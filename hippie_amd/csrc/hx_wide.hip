@@ -11,7 +11,7 @@
 //  1. k_wide_dp: bottom-up over the binary tree (one thread per leaf, arrival
 //     counters), the DP of the best cost of a subtree with j = 1..N-1 slots and
 //     the split (k, j-k) of those slots between its children (or "leaf").
-//  2. Top-down, one launch pair per wide level: each wide interior expands its
+//  2. Top-down, by wide levels on the device: each wide interior expands its
 //     children (the first child whose best split fits the remaining slots is
 //     replaced by its two children, as collapseWide does), a scan of (children,
 //     interior children) per level numbers the next level breadth-first --
@@ -184,98 +184,30 @@ HX_DEV bool child_is_leaf(const WideArgs& a, int64_t T, int b, int k) {
     return a.cnt[(k - 1) * T + b] == kLeafCnt;
 }
 
-// Per entry of a level: (children, interior children) for the level scan.
-template <int N>
-__global__ __launch_bounds__(kWideBlock) void k_wide_count(WideArgs a, int64_t lo, int64_t hi, int2* __restrict__ out) {
-    const int64_t e = lo + blockIdx.x * (int64_t)kWideBlock + threadIdx.x;
-    if (e >= hi) return;
-    int2 r = make_int2(0, 0);
-    if (!a.e_leaf[e]) {
-        const int64_t T = 2 * a.n - 1;
-        int cb[N], ck[N];
-        const int m = expand<N>(a, T, a.e_b[e], a.e_budget[e], e == 0, cb, ck);
-        int ni = 0;
-        for (int i = 0; i < m; ++i) ni += child_is_leaf<N>(a, T, cb[i], ck[i]) ? 0 : 1;
-        r = make_int2(m, ni);
-    }
-    out[e - lo] = r;
-}
-
-// Exclusive scan of a level's int2 counts in place, total at v[m]: per-block
-// sums (kScanPer items per block), one workgroup scans the sums, then each
-// block scans its items from its offset.
-constexpr int kScanItems = 8;
-constexpr int kScanPer = kWideBlock * kScanItems;
-
 HX_DEV int2 add2(int2 p, int2 q) { return make_int2(p.x + q.x, p.y + q.y); }
 
-__global__ __launch_bounds__(kWideBlock) void k_scan_reduce(const int2* __restrict__ v, int64_t m, int2* __restrict__ part) {
-    __shared__ int2 wt[kWideBlock / kWave];
-    const int64_t base = blockIdx.x * (int64_t)kScanPer;
-    int2 s = make_int2(0, 0);
-#pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-        const int64_t i = base + k * kWideBlock + threadIdx.x;
-        if (i < m) s = add2(s, v[i]);
-    }
-    int2 total;
-    block_inclusive_scan<kWideBlock / kWave>(s, add2, wt, total);
-    if (threadIdx.x == 0) part[blockIdx.x] = total;
-}
-
-__global__ __launch_bounds__(1024) void k_scan_parts(int2* __restrict__ part, int64_t nb) {
-    __shared__ int2 wt[1024 / kWave];
-    __shared__ int2 carry;
-    if (threadIdx.x == 0) carry = make_int2(0, 0);
-    __syncthreads();
-    for (int64_t base = 0; base < nb; base += 1024) {
-        const int64_t i = base + threadIdx.x;
-        const int2 x = i < nb ? part[i] : make_int2(0, 0);
-        int2 total;
-        const int2 inc = block_inclusive_scan<1024 / kWave>(x, add2, wt, total);
-        const int2 c0 = carry;
-        if (i < nb) part[i] = make_int2(c0.x + inc.x - x.x, c0.y + inc.y - x.y);
-        __syncthreads();
-        if (threadIdx.x == 0) carry = add2(c0, total);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) part[nb] = carry;
-}
-
-__global__ __launch_bounds__(kWideBlock) void k_scan_apply(int2* __restrict__ v, int64_t m, const int2* __restrict__ part) {
-    __shared__ int2 wt[kWideBlock / kWave];
-    const int64_t base = blockIdx.x * (int64_t)kScanPer;
-    int2 carry = part[blockIdx.x];
-#pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-        const int64_t i = base + k * kWideBlock + threadIdx.x;
-        const int2 x = i < m ? v[i] : make_int2(0, 0);
-        int2 total;
-        const int2 inc = block_inclusive_scan<kWideBlock / kWave>(x, add2, wt, total);
-        if (i < m) v[i] = make_int2(carry.x + inc.x - x.x, carry.y + inc.y - x.y);
-        carry = add2(carry, total);
-    }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) v[m] = carry;
-}
-
-// Children of the level's interiors written as the next level, breadth-first:
-// an interior child gets interior rank int_base + (interior children before it),
-// a leaf child leaf rank leaf_base + (leaf children before it).
+// (children, interior children) of entry e, and the children themselves.
 template <int N>
-__global__ __launch_bounds__(kWideBlock) void k_wide_scatter(WideArgs a, int64_t lo, int64_t hi, const int2* __restrict__ off,
-                                                             int64_t int_base, int64_t leaf_base) {
-    const int64_t e = lo + blockIdx.x * (int64_t)kWideBlock + threadIdx.x;
-    if (e >= hi || a.e_leaf[e]) return;
-    const int64_t T = 2 * a.n - 1;
-    int cb[N], ck[N];
+HX_DEV int2 expand_entry(const WideArgs& a, int64_t T, int64_t e, int* cb, int* ck) {
+    if (a.e_leaf[e]) return make_int2(0, 0);
     const int m = expand<N>(a, T, a.e_b[e], a.e_budget[e], e == 0, cb, ck);
-    const int2 o = off[e - lo];
-    int64_t slot = hi + o.x;
-    int ir = (int)(int_base + o.y);
-    int lr = (int)(leaf_base + (o.x - o.y));
+    int ni = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+        if (i < m) ni += child_is_leaf<N>(a, T, cb[i], ck[i]) ? 0 : 1;
+    return make_int2(m, ni);
+}
+
+// The m children of interior e as entries slot.., interior ranks from ir, leaf
+// ranks from lr.
+template <int N>
+HX_DEV void place_children(const WideArgs& a, int64_t T, int64_t e, int m, const int* cb, const int* ck, int64_t slot,
+                           int ir, int lr) {
     a.e_first[e] = (int32_t)slot;
     a.e_nchild[e] = m;
-    for (int i = 0; i < m; ++i, ++slot) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        if (i >= m) break;
         const bool leaf = child_is_leaf<N>(a, T, cb[i], ck[i]);
         a.e_b[slot] = cb[i];
         a.e_budget[slot] = (int8_t)ck[i];
@@ -284,12 +216,132 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_scatter(WideArgs a, int64_t
         a.e_rank[slot] = leaf ? lr++ : ir++;
         a.e_first[slot] = -1;
         a.e_nchild[slot] = 0;
+        ++slot;
     }
 }
 
+// Levels run on the device.  A level's record is {first entry, end, interiors so
+// far, leaves so far}; a finished collapse has an empty level, which every later
+// launch passes on.  The host reads one record per batch instead of one count
+// per level: a level was five launches and a host round trip (~60 us for levels
+// of a few entries; 500,009 triangles presplit at 0.3 have 18), it is now two
+// launches, and runs of levels of up to 1024 entries share one workgroup.
+// An interior child gets interior rank int_base + (interior children before it),
+// a leaf child leaf rank leaf_base + (leaf children before it).
+constexpr int kWideMaxBlocks = 2048;   // workgroups of a level; each takes one contiguous chunk
+constexpr int kWideSmall = 1024;
+
+struct WideChunk {
+    int64_t b0, b1;   // this workgroup's entries
+    int blocks;       // workgroups with entries
+};
+HX_DEV WideChunk wide_chunk(int4 r) {
+    const int64_t m = (int64_t)r.y - r.x;
+    const int64_t chunk = ((m + gridDim.x - 1) / gridDim.x + kWideBlock - 1) / kWideBlock * kWideBlock;
+    WideChunk c;
+    c.b0 = r.x + blockIdx.x * chunk;
+    c.b1 = min(c.b0 + chunk, (int64_t)r.y);
+    c.blocks = chunk > 0 ? (int)((m + chunk - 1) / chunk) : 0;
+    return c;
+}
+
+HX_DEV int2 block_sum2(int2 s, int2* ws) {
+    s = make_int2(wave_sum_i32(s.x), wave_sum_i32(s.y));
+    if (lane_id() == 0) ws[threadIdx.x / kWave] = s;
+    __syncthreads();
+    int2 t = ws[0];
+    for (int w = 1; w < kWideBlock / kWave; ++w) t = add2(t, ws[w]);
+    return t;
+}
+
 template <int N>
-__global__ __launch_bounds__(kWideBlock) void k_wide_root(WideArgs a) {
+__global__ __launch_bounds__(kWideBlock) void k_wide_count(WideArgs a, const int4* __restrict__ rec,
+                                                           int2* __restrict__ partial) {
+    __shared__ int2 ws[kWideBlock / kWave];
+    const WideChunk c = wide_chunk(*rec);
+    if (c.b0 >= c.b1) return;
+    int2 s = make_int2(0, 0);
+    int cb[N], ck[N];
+    for (int64_t e = c.b0 + threadIdx.x; e < c.b1; e += kWideBlock)
+        s = add2(s, expand_entry<N>(a, 2 * a.n - 1, e, cb, ck));
+    s = block_sum2(s, ws);
+    if (threadIdx.x == 0) partial[blockIdx.x] = s;
+}
+
+// The next level of the record rec (rec[1] receives its record).  Each
+// workgroup adds up the chunks' counts itself (at most kWideMaxBlocks of them).
+// More entries than the caller reserved end the collapse: *err = their number.
+template <int N>
+__global__ __launch_bounds__(kWideBlock) void k_wide_scatter(WideArgs a, int4* __restrict__ rec,
+                                                             const int2* __restrict__ partial,
+                                                             int32_t* __restrict__ err) {
+    __shared__ int2 ws[2][kWideBlock / kWave];
+    const int4 r = *rec;
+    if (r.y <= r.x) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) rec[1] = r;
+        return;
+    }
+    const WideChunk c = wide_chunk(r);
+    if (c.b0 >= c.b1) return;
+    int2 pre = make_int2(0, 0), all = make_int2(0, 0);
+    for (int t = threadIdx.x; t < c.blocks; t += kWideBlock) {
+        const int2 v = partial[t];
+        all = add2(all, v);
+        if (t < (int)blockIdx.x) pre = add2(pre, v);
+    }
+    all = block_sum2(all, ws[0]);
+    pre = block_sum2(pre, ws[1]);
+    const bool fits = (int64_t)r.y + all.x <= 2 * a.n;
+    if ((int)blockIdx.x == c.blocks - 1 && threadIdx.x == 0) {
+        rec[1] = fits ? make_int4(r.y, r.y + all.x, r.z + all.y, r.w + all.x - all.y) : make_int4(r.y, r.y, r.z, r.w);
+        if (!fits) *err = r.y + all.x;
+    }
+    if (!fits) return;
+    const int64_t T = 2 * a.n - 1;
+    __shared__ int2 wt[kWideBlock / kWave];
+    int cb[N], ck[N];
+    for (int64_t base = c.b0; base < c.b1; base += kWideBlock) {
+        const int64_t e = base + threadIdx.x;
+        const int2 x = e < c.b1 ? expand_entry<N>(a, T, e, cb, ck) : make_int2(0, 0);
+        int2 tot;
+        const int2 inc = block_inclusive_scan<kWideBlock / kWave>(x, add2, wt, tot);
+        const int2 o = make_int2(pre.x + inc.x - x.x, pre.y + inc.y - x.y);
+        if (x.x > 0) place_children<N>(a, T, e, x.x, cb, ck, (int64_t)r.y + o.x, r.z + o.y, r.w + (o.x - o.y));
+        pre = add2(pre, tot);
+    }
+}
+
+// Levels of at most kWideSmall entries, one after the other in one workgroup.
+template <int N>
+__global__ __launch_bounds__(kWideSmall) void k_wide_small(WideArgs a, const int4* __restrict__ in,
+                                                           int4* __restrict__ out, int32_t* __restrict__ err) {
+    __shared__ int2 wt[kWideSmall / kWave];
+    const int64_t T = 2 * a.n - 1;
+    int4 r = *in;
+    while (r.y > r.x && r.y - r.x <= kWideSmall) {
+        const int e = r.x + (int)threadIdx.x;
+        int cb[N], ck[N];
+        const int2 x = e < r.y ? expand_entry<N>(a, T, e, cb, ck) : make_int2(0, 0);
+        int2 tot;
+        const int2 inc = block_inclusive_scan<kWideSmall / kWave>(x, add2, wt, tot);
+        if ((int64_t)r.y + tot.x > 2 * a.n) {
+            if (threadIdx.x == 0) *err = r.y + tot.x;
+            r.x = r.y;
+            break;
+        }
+        const int2 o = make_int2(inc.x - x.x, inc.y - x.y);
+        if (x.x > 0) place_children<N>(a, T, e, x.x, cb, ck, (int64_t)r.y + o.x, r.z + o.y, r.w + (o.x - o.y));
+        r = make_int4(r.y, r.y + tot.x, r.z + tot.y, r.w + tot.x - tot.y);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *out = r;
+}
+
+template <int N>
+__global__ __launch_bounds__(kWideBlock) void k_wide_root(WideArgs a, int4* __restrict__ rec, int32_t* __restrict__ err) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *rec = make_int4(0, 1, 1, 0);
+        *err = 0;
         a.e_b[0] = root_of(a);
         a.e_budget[0] = 1;
         a.e_leaf[0] = 0;
@@ -416,11 +468,13 @@ __global__ __launch_bounds__(256) void k_wide_cost_sum(const double* __restrict_
     if (threadIdx.x == 0) *out = s[0];
 }
 
+constexpr int kWideBatch = 12;  // levels launched between host reads
+static_assert(kWideBatch + 3 <= kWideRecords, "records of a batch");
+
 unsigned grid_of(int64_t n) { return (unsigned)std::max<int64_t>(1, (n + kWideBlock - 1) / kWideBlock); }
 
 template <int N>
 int build_wide_n(Context* c, WideArgs a, int64_t* n_interior, int64_t* n_leaves, int64_t* n_entries) {
-    const int64_t T = 2 * a.n - 1;
     {
         LaunchScope ls(c, "wide_dp");
         if (a.n > 1) {
@@ -431,39 +485,37 @@ int build_wide_n(Context* c, WideArgs a, int64_t* n_interior, int64_t* n_leaves,
         hipLaunchKernelGGL(k_wide_dp<N>, dim3(grid_of(a.n)), dim3(kWideBlock), 0, c->stream, a);
         HX_TRY(check_launch("wide_dp"));
     }
-    (void)T;
     LaunchScope ls(c, "wide_levels");
-    hipLaunchKernelGGL(k_wide_root<N>, dim3(1), dim3(64), 0, c->stream, a);
+    // Records: a batch's start, one per launch, and the error word behind them.
+    int4* rec = a.rec;
+    int32_t* err = &rec[kWideBatch + 2].x;
+    hipLaunchKernelGGL(k_wide_root<N>, dim3(1), dim3(64), 0, c->stream, a, rec, err);
     HX_TRY(check_launch("wide_root"));
-    int64_t lo = 0, hi = 1, int_total = 1, leaf_total = 0;
-    int2 tot;
-    while (hi > lo) {
-        const int64_t m = hi - lo;
-        hipLaunchKernelGGL(k_wide_count<N>, dim3(grid_of(m)), dim3(kWideBlock), 0, c->stream, a, lo, hi, a.scan);
-        HX_TRY(check_launch("wide_count"));
-        const int64_t nb = (m + kScanPer - 1) / kScanPer;
-        hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(kWideBlock), 0, c->stream, a.scan, m, a.scan_part);
-        HX_TRY(check_launch("wide_scan_reduce"));
-        hipLaunchKernelGGL(k_scan_parts, dim3(1), dim3(1024), 0, c->stream, a.scan_part, nb);
-        HX_TRY(check_launch("wide_scan_parts"));
-        hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(kWideBlock), 0, c->stream, a.scan, m, a.scan_part);
-        HX_TRY(check_launch("wide_scan_apply"));
-        HX_HIP(hipMemcpyAsync(&tot, a.scan + m, sizeof(int2), hipMemcpyDeviceToHost, c->stream));
-        HX_HIP(hipStreamSynchronize(c->stream));
-        if (tot.x == 0) break;
-        if (hi + tot.x > 2 * a.n) {
-            set_error("wide collapse: %lld nodes exceed the %lld entries reserved", (long long)(hi + tot.x),
-                      (long long)(2 * a.n));
-            return HX_ERR_HIP;
+    const unsigned grid = std::min<unsigned>(grid_of(a.n), kWideMaxBlocks);
+    int4 last[2];  // the batch's last record and the error word
+    const int4* start = rec;
+    do {
+        hipLaunchKernelGGL(k_wide_small<N>, dim3(1), dim3(kWideSmall), 0, c->stream, a, start, rec, err);
+        HX_TRY(check_launch("wide_small"));
+        for (int k = 0; k < kWideBatch; ++k) {
+            hipLaunchKernelGGL(k_wide_count<N>, dim3(grid), dim3(kWideBlock), 0, c->stream, a, rec + k, a.partial);
+            HX_TRY(check_launch("wide_count"));
+            hipLaunchKernelGGL(k_wide_scatter<N>, dim3(grid), dim3(kWideBlock), 0, c->stream, a, rec + k, a.partial,
+                               err);
+            HX_TRY(check_launch("wide_scatter"));
         }
-        hipLaunchKernelGGL(k_wide_scatter<N>, dim3(grid_of(m)), dim3(kWideBlock), 0, c->stream, a, lo, hi, a.scan,
-                           int_total, leaf_total);
-        HX_TRY(check_launch("wide_scatter"));
-        int_total += tot.y;
-        leaf_total += tot.x - tot.y;
-        lo = hi;
-        hi += tot.x;
+        hipLaunchKernelGGL(k_wide_small<N>, dim3(1), dim3(kWideSmall), 0, c->stream, a, rec + kWideBatch,
+                           rec + kWideBatch + 1, err);
+        HX_TRY(check_launch("wide_small"));
+        HX_HIP(hipMemcpyAsync(last, rec + kWideBatch + 1, sizeof(last), hipMemcpyDeviceToHost, c->stream));
+        HX_HIP(hipStreamSynchronize(c->stream));
+        start = rec + kWideBatch + 1;
+    } while (last[0].y > last[0].x);
+    if (last[1].x) {
+        set_error("wide collapse: %lld nodes exceed the %lld entries reserved", (long long)last[1].x, (long long)(2 * a.n));
+        return HX_ERR_HIP;
     }
+    const int64_t hi = last[0].y, int_total = last[0].z, leaf_total = last[0].w;
     *n_interior = int_total;
     *n_leaves = leaf_total;
     *n_entries = hi;

@@ -112,3 +112,16 @@ def test_presplit_rejects_negative_beta_and_batches(ctx):
     v, t = _scene(n_soup=1000, seed=86)
     with pytest.raises(Exception):
         hx.LBVHBuilder(ctx, presplitting=1, presplitter_beta=-0.5).build(hx.Scene(v, t))
+
+
+# Workgroups of the sums take at least 256 triangles each and tiles hold 1024:
+# sizes at those edges, and slivers whose splits run for several rounds.
+@pytest.mark.parametrize("n", [1, 2, 255, 257, 1023, 1025, 131073])
+@pytest.mark.parametrize("beta", [0.3, 4.0])
+def test_presplit_sum_and_tile_edges(oracle, ctx, n, beta):
+    v, t = scenes.sliver_soup(n, np.random.default_rng(n))
+    bvh = hx.LBVHBuilder(ctx, morton_bits=60, presplitting=1, presplitter_beta=beta).build(hx.Scene(v, t))
+    ref = oracle.presplit(v, t, beta=beta)
+    assert bvh.info("references") == len(ref["tri"])
+    tri = np.bincount(bvh.tri_indices_host(), minlength=n)
+    assert np.array_equal(tri, np.bincount(ref["tri"], minlength=n))

@@ -131,3 +131,20 @@ def test_wide_refit_and_rebuild(oracle, ctx, layout):
     assert np.array_equal(got[:, :2], brute[:, :2])
     assert np.array_equal(wb.woop_host().view(np.uint32),
                           oracle.woopify(v2, t, wb.tri_indices_host()).view(np.uint32))
+
+
+# Level kernels: one workgroup up to 1024 entries a level, chunks of 256 above,
+# batches of 12 levels per host read (a chain of nested slabs makes a deep tree).
+@pytest.mark.parametrize("layout", ["quad", "oct"])
+@pytest.mark.parametrize("n", [1, 2, 5, 1024, 4097, 40000])
+def test_wide_levels_match_bin_hits(ctx, layout, n):
+    v, t = scenes.uniform_soup(n, seed=n + 3)
+    scale = np.exp2(-np.repeat(np.arange(n) % 60, 3) / 3.0).astype(np.float32)[:, None]
+    v = (v * scale).astype(np.float32)
+    rays = scenes.random_rays(4000, seed=9)
+    res = []
+    for lay in ("bin", layout):
+        bvh = hx.LBVHBuilder(ctx, morton_bits=60, layout=lay).build(hx.Scene(v, t))
+        assert bvh.n_nodes <= 2 * n + 1
+        res.append(hx.HipTracer(ctx, bvh).trace(hx.RayBuffer(rays)).cpu().numpy())
+    assert np.array_equal(*res)
