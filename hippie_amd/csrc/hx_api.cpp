@@ -710,7 +710,8 @@ int run_insertion(hx_bvh* b) {
     a.best_left = reinterpret_cast<int32_t*>(carve(4 * N));
     a.best_right = reinterpret_cast<int32_t*>(carve(4 * N));
     a.best_parent = reinterpret_cast<int32_t*>(carve(4 * N));
-    a.acc = reinterpret_cast<unsigned long long*>(carve(32));
+    a.acc = reinterpret_cast<unsigned long long*>(carve(8 * hx::kInsAcc));
+    a.ctrl = reinterpret_cast<hx::InsCtrl*>(carve(sizeof(hx::InsCtrl)));
     a.refs = reinterpret_cast<int32_t*>(carve(4 * (size_t)n));
     a.height = reinterpret_cast<int32_t*>(carve(4 * (size_t)n));
     a.rec = reinterpret_cast<int4*>(carve(64 * N));

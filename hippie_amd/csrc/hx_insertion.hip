@@ -56,6 +56,28 @@ HX_DEV Box3 box_union(const Box3& a, const Box3& b) {
     return r;
 }
 
+// Where no box is inverted (no triangle has three NaNs on an axis: the sticky
+// `odd` flag of InsCtrl says so, and k_ins_pack looks) the union is six hardware
+// min/max instead of 24 selects (48 instructions); it can differ from the
+// selects only in the sign of a zero, which no area comparison sees.
+HX_DEV float vmin(float a, float b) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+HX_DEV float vmax(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+HX_DEV Box3 walk_union(const Box3& a, const Box3& b, bool odd) {
+    if (odd) return box_union(a, b);
+    Box3 r;
+    r.mn = make_float3(vmin(a.mn.x, b.mn.x), vmin(a.mn.y, b.mn.y), vmin(a.mn.z, b.mn.z));
+    r.mx = make_float3(vmax(a.mx.x, b.mx.x), vmax(a.mx.y, b.mx.y), vmax(a.mx.z, b.mx.z));
+    return r;
+}
+
 HX_DEV float area_of(const Box3& b) { return box_area(b.mn, b.mx); }
 
 HX_DEV int sibling_of(const InsArgs& a, int v, int p) { return a.left[p] == v ? a.right[p] : a.left[p]; }
@@ -68,13 +90,24 @@ HX_DEV int sibling_of(const InsArgs& a, int v, int p) { return a.left[p] == v ? 
 //       1 if the node is its parent's left child (the root: -1, 0)    [3] unused
 // With the sibling in the node's own record a step up the tree reads the
 // line it already holds instead of the parent's.  Written before every find
-// from the arrays the other kernels update.
+// from the arrays the other kernels update.  The pass also keeps the tree if the
+// last step left it the best so far, and clears the locks and climb counters.
 __global__ __launch_bounds__(kBlock) void k_ins_pack(InsArgs a) {
+    const InsCtrl* ct = a.ctrl;
+    if (ct->done) return;
     const int N = (int)(2 * a.n - 1);
     const int nl = (int)a.n - 1;
     const int v = blockIdx.x * kBlock + threadIdx.x;
     if (v >= N) return;
+    if (ct->best_is_current) {
+        a.best_left[v] = a.left[v];
+        a.best_right[v] = a.right[v];
+        a.best_parent[v] = a.parent[v];
+    }
+    a.locks[v] = 0ull;
+    if (v < nl) a.counters[v] = 0;
     const float4 mn = a.nmin[v], mx = a.nmax[v];
+    if (!(mn.x <= mx.x && mn.y <= mx.y && mn.z <= mx.z)) a.ctrl->odd = 1;
     const int l = v < nl ? a.left[v] : -1, r = v < nl ? a.right[v] : -1;
     const int p = a.parent[v];
     int sib = -1, is_left = 0;
@@ -94,7 +127,7 @@ struct WalkNode {
     int parent, left;
 };
 
-HX_DEV WalkNode walk_node(const InsArgs& a, int v) {
+HX_DEV WalkNode walk_node(const InsArgs& a, int v) {  // rows 0 and 1
     const float4* rec = reinterpret_cast<const float4*>(a.rec) + 4 * (int64_t)v;
     const float4 r0 = rec[0], r1 = rec[1];
     WalkNode w;
@@ -110,6 +143,19 @@ HX_DEV int2 walk_side(const InsArgs& a, int v) {
     return *reinterpret_cast<const int2*>(reinterpret_cast<const int32_t*>(a.rec + 4 * (int64_t)v + 2) + 2);
 }
 
+// The node this thread works on in the current step (in = mod k + rem), or -1:
+// past the step's nodes, the root, or the loop has ended.
+struct StepNodes {
+    int in;
+};
+HX_DEV StepNodes step_nodes(const InsArgs& a) {
+    const InsCtrl* ct = a.ctrl;
+    const int mod = ct->mod, rem = ct->steps % mod;
+    const int N = (int)(2 * a.n - 1);
+    const int64_t in = (int64_t)mod * (blockIdx.x * (int64_t)kBlock + threadIdx.x) + rem;
+    return StepNodes{ct->done || in <= 0 || in >= N ? -1 : (int)in};
+}
+
 // findBestNode (InsertionBuilderKernels.cu:11-185).  The walk visits the
 // sibling's subtree (the sibling itself is the current position and is not a
 // candidate), then climbs: at each ancestor it visits the other child's
@@ -117,74 +163,74 @@ HX_DEV int2 walk_side(const InsArgs& a, int v) {
 // is a candidate).  Going down, `red` gains each visited node's growth; a
 // subtree is skipped when even a perfect merge cannot beat the best so far.
 // The walk is bounded by 4N + 64 visits (a consistent tree needs fewer than
-// 2N + depth); a thread that runs out reports no move.
-__global__ __launch_bounds__(kBlock) void k_ins_find(InsArgs a, int mod, int rem, int count) {
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= count) return;
+// 2N + 2 depth); a thread that runs out reports no move.
+// One record is read per visit, whatever the lane's state: some lane of a wave
+// is at an ancestor at almost every visit, so reading the ancestor within the
+// visit cost the whole wave a second memory round trip: 2,000,000 triangles
+// 86.7 -> 81.2 ms, 150,000 clustered ones 8.4 -> 8.0 ms (100,003 uniform ones,
+// whose walks are short, 4.3 -> 4.4 ms).
+__global__ __launch_bounds__(kBlock) void k_ins_find(InsArgs a) {
+    const StepNodes st = step_nodes(a);
+    if (st.in < 0) return;
     const int N = (int)(2 * a.n - 1);
-    const int in = mod * k + rem;
-    if (in <= 0 || in >= N) return;
+    const int in = st.in;
+    const bool odd = a.ctrl->odd != 0;
     const int nl = (int)a.n - 1;
     const WalkNode inNode = walk_node(a, in);
+    const int sib = walk_side(a, in).x;
     const int p = inNode.parent;
     const Box3 inBox = inNode.box;
     const float pArea = area_of(walk_node(a, p).box);
     const float bound = pArea - area_of(inBox);
     Box3 highest = box_empty();
-    const int sib = walk_side(a, in).x;
     int out = sib, highestIdx = p;
-    bool down = true;
+    // kDown: a node of the subtree being searched; kUp: back at it with its
+    // subtree done; kTop: an ancestor of in, its other child's subtree done.
+    enum { kDown, kUp, kTop };
+    int state = kDown;
     int best = -1;
     float bestRed = 0.0f, red = 0.0f;
     const int64_t limit = 4 * (int64_t)N + 64;
     int64_t it = 0;
     for (; it < limit; ++it) {
-        WalkNode on = walk_node(a, out);
-        Box3 outBox = on.box;
-        Box3 merged = box_union(inBox, outBox);
-        if (down) {
-            if (out != sib) {
-                const float direct = pArea - area_of(merged);
-                if (bestRed < direct + red) {
-                    bestRed = direct + red;
-                    best = out;
-                }
-            }
-            red += area_of(outBox) - area_of(merged);
-            if (out >= nl || red + bound <= bestRed) down = false;
+        const WalkNode on = walk_node(a, out);
+        int2 side = make_int2(-1, 0);
+        if (state != kDown) side = walk_side(a, out);
+        const Box3 merged = walk_union(inBox, state == kTop ? highest : on.box, odd);
+        const float outArea = area_of(on.box), mergedArea = area_of(merged);
+        const float direct = pArea - mergedArea;
+        const bool candidate = state == kDown ? out != sib : state == kTop && out != p && out != 0;
+        if (candidate && bestRed < direct + red) {
+            bestRed = direct + red;
+            best = out;
+        }
+        if (state == kDown) {
+            red += outArea - mergedArea;
+            if (out >= nl || red + bound <= bestRed) state = kUp;
             else out = on.left;
-        } else {
-            int op = on.parent;
-            red -= area_of(outBox) - area_of(merged);
-            if (op == highestIdx) {
-                box_grow(highest, outBox.mn);
-                box_grow(highest, outBox.mx);
-                out = op;
-                const WalkNode up = walk_node(a, out);
-                if (out != p && out != 0) {
-                    merged = box_union(inBox, highest);
-                    const float direct = pArea - area_of(merged);
-                    if (bestRed < direct + red) {
-                        bestRed = direct + red;
-                        best = out;
-                    }
-                    outBox = up.box;
-                    red += area_of(outBox) - area_of(highest);
-                }
-                op = up.parent;
-                if (op < 0) break;
-                highestIdx = op;
-                down = true;
-                out = walk_side(a, out).x;  // out's parent is highestIdx
-            } else {
-                const int2 side = walk_side(a, out);  // out's parent is op
-                if (side.y) {
-                    down = true;
-                    out = side.x;
+        } else if (state == kUp) {
+            red -= outArea - mergedArea;
+            if (on.parent == highestIdx) {
+                if (odd) {
+                    box_grow(highest, on.box.mn);
+                    box_grow(highest, on.box.mx);
                 } else {
-                    out = op;
+                    highest = walk_union(highest, on.box, false);
                 }
+                out = on.parent;
+                state = kTop;
+            } else if (side.y) {
+                state = kDown;
+                out = side.x;
+            } else {
+                out = on.parent;
             }
+        } else {
+            if (candidate) red += outArea - area_of(highest);
+            if (on.parent < 0) break;
+            highestIdx = on.parent;
+            state = kDown;
+            out = side.x;
         }
     }
     if (it >= limit) best = -1;
@@ -223,12 +269,9 @@ HX_DEV unsigned long long lock_key(const InsArgs& a, int in) {
     return ((unsigned long long)__float_as_uint(a.red[in]) << 32) | (unsigned long long)(unsigned)in;
 }
 
-__global__ __launch_bounds__(kBlock) void k_ins_lock(InsArgs a, int mod, int rem, int count) {
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= count) return;
-    const int N = (int)(2 * a.n - 1);
-    const int in = mod * k + rem;
-    if (in <= 0 || in >= N) return;
+__global__ __launch_bounds__(kBlock) void k_ins_lock(InsArgs a) {
+    const int in = step_nodes(a).in;
+    if (in < 0) return;
     const int out = a.out[in];
     if (out < 0) return;
     const unsigned long long key = lock_key(a, in);
@@ -237,39 +280,44 @@ __global__ __launch_bounds__(kBlock) void k_ins_lock(InsArgs a, int mod, int rem
     for (int j = 0; j < m; ++j) atomicMax(a.locks + set[j], key);
 }
 
-// Wave-aggregated add of a per-lane count to a 64-bit counter.
-HX_DEV void count_add(unsigned long long* ctr, bool flag) {
-    const uint64_t m = ballot64(flag);
-    if (m && lane_id() == __builtin_ctzll(m)) atomicAdd(ctr, (unsigned long long)__builtin_popcountll(m));
+// checkLocks (:273-358).
+__global__ __launch_bounds__(kBlock) void k_ins_check(InsArgs a) {
+    const int in = step_nodes(a).in;
+    if (in < 0) return;
+    const int out = a.out[in];
+    if (out < 0) return;
+    const unsigned long long key = lock_key(a, in);
+    int set[8];
+    const int m = lock_set(a, in, out, set);
+    bool ok = true;
+    for (int j = 0; j < m; ++j) ok = ok && a.locks[set[j]] == key;
+    if (!ok) a.out[in] = -1;
 }
 
-// checkLocks (:273-358): acc[1] counts the moves found.
-__global__ __launch_bounds__(kBlock) void k_ins_check(InsArgs a, int mod, int rem, int count) {
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    const int N = (int)(2 * a.n - 1);
-    const int in = mod * k + rem;
-    const bool live = k < count && in > 0 && in < N;
-    const int out = live ? a.out[in] : -1;
-    if (out >= 0) {
-        const unsigned long long key = lock_key(a, in);
-        int set[8];
-        const int m = lock_set(a, in, out, set);
-        bool ok = true;
-        for (int j = 0; j < m; ++j) ok = ok && a.locks[set[j]] == key;
-        if (!ok) a.out[in] = -1;
+// Sum over the workgroup, to thread 0; every thread calls it.
+HX_DEV unsigned long long block_sum64(unsigned long long s) {
+    __shared__ unsigned long long ws[kBlock / kWave];
+#pragma unroll
+    for (int m = 1; m < kWave; m <<= 1) {
+        const uint32_t lo = __shfl_xor((uint32_t)s, m, kWave);
+        const uint32_t hi = __shfl_xor((uint32_t)(s >> 32), m, kWave);
+        s += ((unsigned long long)hi << 32) | lo;
     }
-    count_add(a.acc + 1, out >= 0);
+    if (lane_id() == 0) ws[threadIdx.x / kWave] = s;
+    __syncthreads();
+    s = 0;
+    for (int w = 0; w < kBlock / kWave; ++w) s += ws[w];
+    return s;
 }
 
 // reinsert (:361-455): unlink in's parent (under the root, the sibling's
 // slot is reused and its children move up to the root), then make it the
-// parent of out and in.  acc[2] counts the moves applied.
-__global__ __launch_bounds__(kBlock) void k_ins_reinsert(InsArgs a, int mod, int rem, int count) {
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    const int N = (int)(2 * a.n - 1);
-    const int in = mod * k + rem;
-    const bool live = k < count && in > 0 && in < N;
-    const int out = live ? a.out[in] : -1;
+// parent of out and in.  The moves applied are counted per workgroup in one of
+// kInsAcc - 1 words (one device atomic per wave on one word, ~10 ns each, was
+// most of the check and reinsert passes at 100,003 triangles: 22 and 18 us).
+__global__ __launch_bounds__(kBlock) void k_ins_reinsert(InsArgs a) {
+    const int in = step_nodes(a).in;
+    const int out = in >= 0 ? a.out[in] : -1;
     if (out >= 0) {
         int p = a.parent[in];
         const int sib = sibling_of(a, in, p);
@@ -307,7 +355,8 @@ __global__ __launch_bounds__(kBlock) void k_ins_reinsert(InsArgs a, int mod, int
             a.right[0] = p;
         }
     }
-    count_add(a.acc + 2, out >= 0);
+    const unsigned long long moved = block_sum64(out >= 0 ? 1ull : 0ull);
+    if (threadIdx.x == 0 && moved) atomicAdd(a.acc + 1 + blockIdx.x % (kInsAcc - 1), moved);
 }
 
 HX_DEV float4 ld_agent4(const float4* p) {
@@ -335,7 +384,7 @@ template <bool SIZES>
 __global__ __launch_bounds__(kBlock) void k_ins_refit(InsArgs a) {
     const int j = blockIdx.x * kBlock + threadIdx.x;
     const int nl = (int)a.n - 1;
-    if (j > nl) return;
+    if (j > nl || (!SIZES && a.ctrl->done)) return;
     int node = a.parent[nl + j];
     for (int guard = 0; node >= 0 && guard <= nl; ++guard) {
         if (__hip_atomic_fetch_add(&a.counters[node], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) break;
@@ -371,7 +420,10 @@ HX_DEV unsigned long long fixed_term(float t) {
     return (unsigned long long)((double)t * 4294967296.0);
 }
 
+// One atomic per workgroup (256 of them: 41 us -> 8 us a step at 100,003
+// triangles against one per wave of 1024 workgroups).
 __global__ __launch_bounds__(kBlock) void k_ins_cost(InsArgs a) {
+    if (a.ctrl->done) return;
     const int64_t N = 2 * a.n - 1;
     const int nl = (int)a.n - 1;
     const float scene = area_of(node_box(a, 0));
@@ -380,103 +432,97 @@ __global__ __launch_bounds__(kBlock) void k_ins_cost(InsArgs a) {
         const float P = area_of(node_box(a, (int)v)) / scene;
         s += fixed_term((v >= nl ? a.ci : a.ct) * P);
     }
-#pragma unroll
-    for (int m = 1; m < kWave; m <<= 1) {
-        const uint32_t lo = __shfl_xor((uint32_t)s, m, kWave);
-        const uint32_t hi = __shfl_xor((uint32_t)(s >> 32), m, kWave);
-        s += ((unsigned long long)hi << 32) | lo;
+    s = block_sum64(s);
+    if (threadIdx.x == 0 && s) atomicAdd(a.acc, s);
+}
+
+// The loop's bookkeeping after a step, on the device so that the host reads it
+// once per batch of steps (a step's host round trip was ~70 us).
+__global__ void k_ins_step(InsArgs a, int start_mod) {
+    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    InsCtrl& ct = *a.ctrl;
+    if (start_mod > 0) {  // before the first step
+        ct.best = ct.prev = 3.402823466e+38;
+        ct.total = 0;
+        ct.steps = ct.done = ct.odd = 0;
+        ct.mod = start_mod;
+        ct.best_is_current = 1;
+        for (int k = 0; k < kInsAcc; ++k) a.acc[k] = 0ull;
+        return;
     }
-    if (lane_id() == 0 && s) atomicAdd(a.acc, s);
+    if (ct.done) return;
+    const double cost = (double)a.acc[0] * (1.0 / 4294967296.0);
+    long long moved = 0;
+    for (int k = 1; k < kInsAcc; ++k) moved += (long long)a.acc[k];
+    for (int k = 0; k < kInsAcc; ++k) a.acc[k] = 0ull;
+    ct.total += moved;
+    ct.best_is_current = ct.best > cost ? 1 : 0;
+    if (ct.best_is_current) ct.best = cost;
+    ++ct.steps;
+    const bool stalled = fabs(ct.prev - cost) <= 0.01;
+    ct.prev = cost;
+    if (((stalled || moved == 0) && ct.mod == 1) || ct.steps >= kInsMaxSteps) ct.done = 1;
+    else if (stalled) ct.mod = max(1, ct.mod - 1);
 }
 
-__global__ void k_ins_zero(unsigned long long* p, int count) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) p[i] = 0ull;
+// The best tree back into place unless the last step left it there.
+__global__ __launch_bounds__(kBlock) void k_ins_restore(InsArgs a) {
+    if (a.ctrl->best_is_current) return;
+    const int v = blockIdx.x * kBlock + threadIdx.x;
+    if (v >= (int)(2 * a.n - 1)) return;
+    a.left[v] = a.best_left[v];
+    a.right[v] = a.best_right[v];
+    a.parent[v] = a.best_parent[v];
 }
 
-__global__ __launch_bounds__(kBlock) void k_ins_copy3(const int32_t* __restrict__ a, const int32_t* __restrict__ b,
-                                                     const int32_t* __restrict__ c, int32_t* __restrict__ da,
-                                                     int32_t* __restrict__ db, int32_t* __restrict__ dc, int count) {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < count) {
-        da[i] = a[i];
-        db[i] = b[i];
-        dc[i] = c[i];
-    }
-}
-
-int copy_tree(Context* c, const int32_t* l, const int32_t* r, const int32_t* p, int32_t* dl, int32_t* dr,
-              int32_t* dp, int count) {
-    hipLaunchKernelGGL(k_ins_copy3, dim3(grid_for(count)), dim3(kBlock), 0, c->stream, l, r, p, dl, dr, dp, count);
-    return check_launch("ins_copy");
-}
+constexpr int kInsBatch = 4;  // steps launched between host reads
 
 }  // namespace
 
-int launch_ins_refit(Context* c, const InsArgs& a, bool sizes) {
+int launch_ins_refit(Context* c, const InsArgs& a) {
     const int64_t n = a.n;
     if (n < 2) return HX_OK;
     HX_TRY(launch_fill_i32(c, a.counters, 0, n - 1));
-    if (sizes)
-        hipLaunchKernelGGL(k_ins_refit<true>, dim3(grid_for(n)), dim3(kBlock), 0, c->stream, a);
-    else
-        hipLaunchKernelGGL(k_ins_refit<false>, dim3(grid_for(n)), dim3(kBlock), 0, c->stream, a);
+    hipLaunchKernelGGL(k_ins_refit<true>, dim3(grid_for(n)), dim3(kBlock), 0, c->stream, a);
     return check_launch("ins_refit");
 }
 
 int launch_insertion(Context* c, const InsArgs& a, int64_t* steps_out, int64_t* reinserted_out) {
     const int64_t n = a.n;
     const int N = (int)(2 * n - 1);
-    int steps = 0, mod_cur = std::max(a.mod, 1);
-    int64_t total = 0;
-    double cost = 3.402823466e+38, best = 3.402823466e+38, prev;
-    bool best_is_current = true;
     LaunchScope ls(c, "insertion");
-    HX_TRY(copy_tree(c, a.left, a.right, a.parent, a.best_left, a.best_right, a.best_parent, N));
-    const unsigned cost_grid = std::min<unsigned>(grid_for(N), 1024u);
-    while (steps < kInsMaxSteps) {
-        prev = cost;
-        const int rem = steps % mod_cur;
-        const int count = (N - rem + mod_cur - 1) / mod_cur;
-        const unsigned g = grid_for(count);
-        hipLaunchKernelGGL(k_ins_zero, dim3(1), dim3(64), 0, c->stream, a.acc, 4);
-        HX_TRY(check_launch("ins_zero"));
-        hipLaunchKernelGGL(k_ins_pack, dim3(grid_for(N)), dim3(kBlock), 0, c->stream, a);
-        HX_TRY(check_launch("ins_pack"));
-        hipLaunchKernelGGL(k_ins_find, dim3(g), dim3(kBlock), 0, c->stream, a, mod_cur, rem, count);
-        HX_TRY(check_launch("ins_find"));
-        HX_TRY(launch_fill_i32(c, reinterpret_cast<int32_t*>(a.locks), 0, 2 * (int64_t)N));
-        hipLaunchKernelGGL(k_ins_lock, dim3(g), dim3(kBlock), 0, c->stream, a, mod_cur, rem, count);
-        HX_TRY(check_launch("ins_lock"));
-        hipLaunchKernelGGL(k_ins_check, dim3(g), dim3(kBlock), 0, c->stream, a, mod_cur, rem, count);
-        HX_TRY(check_launch("ins_check"));
-        hipLaunchKernelGGL(k_ins_reinsert, dim3(g), dim3(kBlock), 0, c->stream, a, mod_cur, rem, count);
-        HX_TRY(check_launch("ins_reinsert"));
-        HX_TRY(launch_ins_refit(c, a, false));
-        hipLaunchKernelGGL(k_ins_cost, dim3(cost_grid), dim3(kBlock), 0, c->stream, a);
-        HX_TRY(check_launch("ins_cost"));
-        unsigned long long h[4] = {0, 0, 0, 0};
-        HX_HIP(hipMemcpyAsync(h, a.acc, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-        HX_HIP(hipStreamSynchronize(c->stream));
-        cost = (double)h[0] * (1.0 / 4294967296.0);
-        const int64_t inserted = (int64_t)h[2];
-        total += inserted;
-        best_is_current = false;
-        if (best > cost) {
-            best = cost;
-            HX_TRY(copy_tree(c, a.left, a.right, a.parent, a.best_left, a.best_right, a.best_parent, N));
-            best_is_current = true;
+    const dim3 nodes(grid_for(N)), leaves(grid_for(n)), block(kBlock);
+    const dim3 cost_blocks(std::min<unsigned>(grid_for(N), 256u));
+    hipLaunchKernelGGL(k_ins_step, dim3(1), dim3(64), 0, c->stream, a, std::max(a.mod, 1));
+    HX_TRY(check_launch("ins_start"));
+    InsCtrl h{};
+    do {
+        for (int k = 0; k < kInsBatch; ++k) {
+            hipLaunchKernelGGL(k_ins_pack, nodes, block, 0, c->stream, a);
+            HX_TRY(check_launch("ins_pack"));
+            hipLaunchKernelGGL(k_ins_find, nodes, block, 0, c->stream, a);
+            HX_TRY(check_launch("ins_find"));
+            hipLaunchKernelGGL(k_ins_lock, nodes, block, 0, c->stream, a);
+            HX_TRY(check_launch("ins_lock"));
+            hipLaunchKernelGGL(k_ins_check, nodes, block, 0, c->stream, a);
+            HX_TRY(check_launch("ins_check"));
+            hipLaunchKernelGGL(k_ins_reinsert, nodes, block, 0, c->stream, a);
+            HX_TRY(check_launch("ins_reinsert"));
+            hipLaunchKernelGGL(k_ins_refit<false>, leaves, block, 0, c->stream, a);
+            HX_TRY(check_launch("ins_refit"));
+            hipLaunchKernelGGL(k_ins_cost, cost_blocks, block, 0, c->stream, a);
+            HX_TRY(check_launch("ins_cost"));
+            hipLaunchKernelGGL(k_ins_step, dim3(1), dim3(64), 0, c->stream, a, 0);
+            HX_TRY(check_launch("ins_step"));
         }
-        ++steps;
-        const bool stalled = std::fabs(prev - cost) <= 0.01;
-        if ((stalled || inserted == 0) && mod_cur == 1) break;
-        if (stalled) mod_cur = std::max(1, mod_cur - 1);
-    }
-    if (!best_is_current)
-        HX_TRY(copy_tree(c, a.best_left, a.best_right, a.best_parent, a.left, a.right, a.parent, N));
-    HX_TRY(launch_ins_refit(c, a, true));
-    if (steps_out) *steps_out = steps;
-    if (reinserted_out) *reinserted_out = total;
+        HX_HIP(hipMemcpyAsync(&h, a.ctrl, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+        HX_HIP(hipStreamSynchronize(c->stream));
+    } while (!h.done);
+    hipLaunchKernelGGL(k_ins_restore, nodes, block, 0, c->stream, a);
+    HX_TRY(check_launch("ins_restore"));
+    HX_TRY(launch_ins_refit(c, a));
+    if (steps_out) *steps_out = h.steps;
+    if (reinserted_out) *reinserted_out = h.total;
     return HX_OK;
 }
 

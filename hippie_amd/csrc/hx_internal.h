@@ -368,6 +368,17 @@ int launch_refs_to_tris(Context* c, int32_t* ids, const int32_t* ref_tri, int64_
 // return the tree is the best one seen, refitted, with refs and heights of
 // its internal nodes.  n >= 2.
 constexpr int kInsMaxSteps = 1000;
+constexpr int kInsAcc = 33;   // words of InsArgs::acc
+// The loop's state, on the device.
+struct InsCtrl {
+    double best, prev;        // SAH cost of the best tree and of the last step's
+    long long total;          // moves applied
+    int steps, mod;
+    int done;                 // converged: later launches do nothing
+    int best_is_current;      // the last step's tree is the best one
+    int odd;                  // a node box is inverted (NaN vertices)
+    int pad;
+};
 struct InsArgs {
     int64_t n;
     int mod;
@@ -384,13 +395,14 @@ struct InsArgs {
     int32_t* best_left;       // 2n-1 each: the best tree so far
     int32_t* best_right;
     int32_t* best_parent;
-    unsigned long long* acc;  // [0] cost (2^-32 units), [1] moves found, [2] moves applied
+    unsigned long long* acc;  // [0] cost (2^-32 units), [1..] moves applied
+    InsCtrl* ctrl;
     int32_t* refs;            // n-1 leaf counts (filled by the final refit)
     int32_t* height;          // n-1 heights
     int4* rec;                // 2n-1 packed walk records, 4 int4 each
 };
 int launch_insertion(Context* c, const InsArgs& a, int64_t* steps_out, int64_t* reinserted_out);
-int launch_ins_refit(Context* c, const InsArgs& a, bool sizes);
+int launch_ins_refit(Context* c, const InsArgs& a);  // with sizes and heights
 
 // hx_hlbvh.hip: clusters of equal top-sah_bits Morton prefixes (Karras
 // subtrees), binned-SAH upper levels over them, depth-first relabelling.
