@@ -406,6 +406,160 @@ __global__ __launch_bounds__(kSortBlock) void k_sort_local(const uint64_t* __res
     }
 }
 
+// Sorts of up to kBlockSortKeys keys in one workgroup: keys (in LDS and
+// registers) and their input positions go through every digit pass without
+// leaving the CU.  A digit pass of the tiled sort is latency bound there (a
+// launch, a tile counter, loads, look-back and stores, 9 to 12 us whatever the
+// size, and three launches before the first): 4099 60-bit keys took 98 us, now
+// 29 us.  Ranking as in k_onesweep (ballot peers, wave counters in LDS).
+// With `split` (Morton keys of more than 40 bits) the digit passes cover the 32
+// high bits and each run of equal high bits is ranked by the rest, as
+// k_sort_local does; a run longer than `limit` makes every pass run instead.
+constexpr int kBlockSortThreads = 1024;
+constexpr int kBlockSortItems = 8;
+constexpr int kBlockSortKeys = kBlockSortThreads * kBlockSortItems;
+constexpr int kBlockSortWaves = kBlockSortThreads / kWave;
+constexpr int kBlockSortBits = 8;
+
+template <class K, bool IDENT>
+__global__ __launch_bounds__(kBlockSortThreads) void k_sort_block(const K* keys_in, const int32_t* vals_in, K* keys_out,
+                                                                  int32_t* vals_out, int n, int end_bit, int lo_bit,
+                                                                  int limit) {
+    constexpr int IT = kBlockSortItems, R = 1 << kBlockSortBits;
+    __shared__ K s_key[kBlockSortKeys];
+    __shared__ uint16_t s_pos[kBlockSortKeys];   // input positions
+    __shared__ uint32_t s_hist[kBlockSortWaves][R];
+    __shared__ uint32_t s_start[R];
+    __shared__ uint32_t s_wt[R / kWave];
+    __shared__ int s_long;
+    const int tid = threadIdx.x, w = tid / kWave, lane = lane_id();
+    // Every wave takes the same number of 64-key items, so that none idles.
+    const int items = (n + kBlockSortThreads - 1) / kBlockSortThreads;
+    const int base = w * kWave * items;
+    auto in = [&](int i) { return i < items && base + i * kWave + lane < n; };
+    K key[IT];
+    int at[IT];
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+        const int idx = base + i * kWave + lane;
+        at[i] = idx;
+        key[i] = in(i) ? keys_in[idx] : (K)0;
+    }
+    if (tid == 0) s_long = 0;
+    int dst[IT];
+    int from = lo_bit, shift = lo_bit;
+    while (true) {
+        const int nbits = min(kBlockSortBits, end_bit - shift);
+        const uint32_t mask = (1u << nbits) - 1u;
+        for (int k = tid; k < kBlockSortWaves * R; k += kBlockSortThreads) (&s_hist[0][0])[k] = 0u;
+        __syncthreads();
+        uint32_t packed[IT], rank[IT];
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            packed[i] = 0xFFFFFFFFu;
+            if (i >= items) continue;
+            const bool valid = in(i);
+            const uint32_t d = digit_of(key[i], shift, mask);
+            uint64_t peers = ballot64(valid);
+            for (int b = 0; b < nbits; ++b) {
+                const bool bit = (d >> b) & 1u;
+                const uint64_t bb = ballot64(bit);
+                peers &= bit ? bb : ~bb;
+            }
+            packed[i] = valid ? (uint32_t)count_below(peers) | (uint32_t)__builtin_ctzll(peers | (1ull << 63)) << 8 |
+                                    (uint32_t)__popcll(peers) << 16
+                              : 0xFFFFFFFFu;
+        }
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            rank[i] = 0u;
+            if (packed[i] != 0xFFFFFFFFu && (packed[i] & 0xFFu) == 0u)
+                rank[i] = atomicAdd(&s_hist[w][digit_of(key[i], shift, mask)], packed[i] >> 16);
+        }
+#pragma unroll
+        for (int i = 0; i < IT; ++i)
+            rank[i] = __shfl(rank[i], (int)((packed[i] >> 8) & 0x3Fu), kWave) + (packed[i] & 0xFFu);
+        __syncthreads();
+        // Digit starts: the first R threads own a digit each.
+        uint32_t tot = 0;
+        if (tid < R) {
+#pragma unroll
+            for (int ww = 0; ww < kBlockSortWaves; ++ww) {
+                const uint32_t c = s_hist[ww][tid];
+                s_hist[ww][tid] = tot;
+                tot += c;
+            }
+        }
+        const uint32_t inc = wave_inclusive_scan(tot, [](uint32_t x, uint32_t y) { return x + y; });
+        if (tid < R && lane == kWave - 1) s_wt[w] = inc;
+        __syncthreads();
+        if (tid < R) {
+            uint32_t pre = 0;
+            for (int k = 0; k < w; ++k) pre += s_wt[k];
+            s_start[tid] = pre + inc - tot;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            if (!in(i)) continue;
+            const uint32_t d = digit_of(key[i], shift, mask);
+            const uint32_t p = s_start[d] + s_hist[w][d] + rank[i];
+            s_key[p] = key[i];
+            s_pos[p] = (uint16_t)at[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const int idx = base + i * kWave + lane;
+            if (!in(i)) continue;
+            key[i] = s_key[idx];
+            at[i] = s_pos[idx];
+        }
+        shift += kBlockSortBits;
+        if (shift < end_bit) continue;
+#pragma unroll
+        for (int i = 0; i < IT; ++i) dst[i] = base + i * kWave + lane;
+        if (from == 0) break;
+        const K low_mask = ((K)1 << lo_bit) - 1;
+        const K key_mask = end_bit >= 8 * (int)sizeof(K) ? ~(K)0 : ((K)1 << end_bit) - 1;
+        auto high = [&](K k) { return (k & key_mask) >> lo_bit; };
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const int p = base + i * kWave + lane;
+            if (!in(i)) continue;
+            const K h = high(key[i]), lk = key[i] & low_mask;
+            int ls = p, le = p + 1;
+            while (ls > 0 && p - ls <= limit && high(s_key[ls - 1]) == h) --ls;
+            while (le < n && le - p <= limit && high(s_key[le]) == h) ++le;
+            if (le - ls > limit) {
+                s_long = 1;
+                continue;
+            }
+            int r = ls;
+            for (int q = ls; q < le; ++q) {
+                const K kq = s_key[q] & low_mask;
+                r += (kq < lk) || (kq == lk && q < p);
+            }
+            dst[i] = r;
+        }
+        __syncthreads();
+        if (!s_long) break;
+        // A stable LSD sort of this order gives the same result.
+        from = shift = 0;
+    }
+    int32_t val[IT];
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+        val[i] = in(i) ? (IDENT ? at[i] : vals_in[at[i]]) : 0;
+    __syncthreads();  // every input value is read before the output (which may be the input) is written
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+        if (!in(i)) continue;
+        keys_out[dst[i]] = key[i];
+        vals_out[dst[i]] = val[i];
+    }
+}
+
 __global__ void k_sort_flag_clear(int32_t* flag) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *flag = 0;
 }
@@ -545,6 +699,15 @@ int sort_split(Context* c, void* keys[2], int32_t* vals[2], int64_t n, int lo_bi
     return HX_OK;
 }
 
+// Keys per thread of a digit pass: the tunable, but at most 8 while 16 would not
+// give every CU two tiles.  A tile's latency grows with its keys per thread and
+// nothing else fills the chip there: 65,536 60-bit keys 119 -> 91 us, 262,143
+// 136 -> 117 us; above, the fewer and longer digit runs win (1,048,576: 151
+// against 158 us, 16.7M: 869 against 1044 us).
+int sort_items_for(const Context* c, int64_t n) {
+    return n < (int64_t)c->cu_count * 2 * kSortBlock * 8 ? std::min(c->tune.sort_items, 8) : c->tune.sort_items;
+}
+
 }  // namespace
 
 int sort_pass_count(const Context* c, int end_bit, int64_t n, bool keys64) {
@@ -555,7 +718,7 @@ int sort_pass_count(const Context* c, int end_bit, int64_t n, bool keys64) {
 }
 
 int sort_status_words_max(const Context* c, int64_t n, int end_bit) {
-    const int rb = c->tune.sort_digit_bits, it = c->tune.sort_items;
+    const int rb = c->tune.sort_digit_bits, it = sort_items_for(c, n);
     const int passes = sort_passes(end_bit, rb);
     return (int)((int64_t)passes * sort_tiles(n, it) * (1 << rb) + (int64_t)passes * (1 << rb) + kMaxPasses);
 }
@@ -566,7 +729,7 @@ int launch_sort_pairs(Context* c, void* keys[2], int32_t* vals[2], int64_t n, in
         set_error("radix sort: n = %lld exceeds 2^30 - 1", (long long)n);
         return HX_ERR_INVALID_ARG;
     }
-    const int bits = c->tune.sort_digit_bits, items = c->tune.sort_items, lb = c->tune.sort_lookback;
+    const int bits = c->tune.sort_digit_bits, items = sort_items_for(c, n), lb = c->tune.sort_lookback;
     // Long keys, many of them: four digit passes over the high bits leave runs
     // of equal high bits that are short for Morton codes (at most 19 keys for
     // the 16.7M-triangle benchmark scene at 32 high bits), which one pass
@@ -574,6 +737,24 @@ int launch_sort_pairs(Context* c, void* keys[2], int32_t* vals[2], int64_t n, in
     const int lo_bit = end_bit - 4 * bits;
     const bool split = allow_split && ws == nullptr && keys64 && c->tune.sort_local_run > 0 && n >= kLocalMinKeys &&
                        lo_bit >= bits;
+    if (n > 1 && n <= kBlockSortKeys && end_bit > 0) {
+        LaunchScope ls(c, "sort_block");
+        *result_index = sort_pass_count(c, end_bit, n, keys64) & 1;
+        const int in_block_lo = end_bit - 4 * kBlockSortBits;
+        const int lo = allow_split && keys64 && c->tune.sort_local_run > 0 && in_block_lo >= kBlockSortBits ? in_block_lo : 0;
+        const int limit = std::min(c->tune.sort_local_run, kLocalMaxRun);
+        auto launch = [&](auto kernel, auto* kin, auto* kout) {
+            hipLaunchKernelGGL(kernel, dim3(1), dim3(kBlockSortThreads), 0, c->stream, kin, vals[0], kout,
+                               vals[*result_index], (int)n, end_bit, lo, limit);
+        };
+        if (keys64)
+            launch(vals_identity ? k_sort_block<uint64_t, true> : k_sort_block<uint64_t, false>,
+                   static_cast<const uint64_t*>(keys[0]), static_cast<uint64_t*>(keys[*result_index]));
+        else
+            launch(vals_identity ? k_sort_block<uint32_t, true> : k_sort_block<uint32_t, false>,
+                   static_cast<const uint32_t*>(keys[0]), static_cast<uint32_t*>(keys[*result_index]));
+        return check_launch("sort_block");
+    }
 #define HX_SORT_CASE(RB, IT, LB)                                                                                   \
     if (bits == RB && items == IT && lb == LB) {                                                                  \
         if (split) return sort_split<RB, IT, LB>(c, keys, vals, n, lo_bit, end_bit, vals_identity, result_index); \
