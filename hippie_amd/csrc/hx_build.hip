@@ -712,10 +712,13 @@ __global__ __launch_bounds__(kBlock) void k_climb_top(ClimbArgs a, const int32_t
 //   k_lbvh_local: one workgroup per 512 leaves; deltas of its range in LDS;
 //     each arrival at an in-block parent leaves its id and range end in LDS,
 //     the second arrival combines.  A child whose parent straddles the block
-//     (split outside the block, or only one child arrived) joins the frontier.
-//   k_lbvh_top: the frontier climbs with the same rule on global memory, each
-//     arrival writing its side (child id, range end) with sc1 stores that
-//     complete before the parent's counter is bumped.
+//     (split outside the block, or only one child arrived) joins the block's
+//     frontier, a list in position order.
+//   k_lbvh_merge: the frontiers of neighbouring blocks, which cover their
+//     leaves without gaps, climb the same way in LDS, the boundaries between
+//     consecutive entries in the place of the split positions; what straddles
+//     the workgroup's lists is its own frontier for the next merge, until one
+//     workgroup holds the root.
 // ---------------------------------------------------------------------------
 
 // One leaf per thread, 512 leaves per block: measured at 16.7M triangles,
@@ -725,7 +728,7 @@ constexpr int kLbvhThreads = 512;
 constexpr int kLbvhLeaves = 512;
 
 template <bool K64>
-__global__ __launch_bounds__(kLbvhThreads) void k_lbvh_local(ClimbArgs a) {
+__global__ __launch_bounds__(kLbvhThreads) __attribute__((amdgpu_num_sgpr(80))) void k_lbvh_local(ClimbArgs a) {
     constexpr int T = kLbvhLeaves;
     // Slots: internal node s -> s - base, leaf p -> T + p - base.  Every link
     // kept in LDS stays inside the block -- range ends, child slots, parent
@@ -739,13 +742,12 @@ __global__ __launch_bounds__(kLbvhThreads) void k_lbvh_local(ClimbArgs a) {
     __shared__ int16_t s_first[T], s_last[T], s_left[T], s_right[T];  // offsets; children as slots
     __shared__ int8_t s_state[T];
     __shared__ uint8_t s_delta[T + 1];  // delta(base - 1 + k) + 1
-    __shared__ int16_t s_front[T];
+    __shared__ int16_t s_front[T];      // frontier slot whose range starts at this offset, or -1
     __shared__ int s_end[T];
-    __shared__ int s_nfront, s_fbase;
+    __shared__ int s_wfront[T / kWave];
     const int n = (int)a.n;
     const int base = blockIdx.x * T;
     const int last_leaf = min(base + T, n) - 1;
-    if (threadIdx.x == 0) s_nfront = 0;
     for (int i = threadIdx.x; i < T; i += kLbvhThreads) {
         s_cnt[i] = 0;
         s_end[i] = -1;
@@ -753,6 +755,7 @@ __global__ __launch_bounds__(kLbvhThreads) void k_lbvh_local(ClimbArgs a) {
         s_right[i] = -1;
         s_par[i] = -1;
         s_par[T + i] = -1;
+        s_front[i] = -1;
     }
     for (int k = threadIdx.x; k <= T; k += kLbvhThreads) {
         const int q = base - 1 + k;
@@ -787,7 +790,7 @@ __global__ __launch_bounds__(kLbvhThreads) void k_lbvh_local(ClimbArgs a) {
             const bool as_left = s_delta[r - base + 1] > s_delta[l - base];
             const int sp = as_left ? r : l - 1;
             if (sp < base || sp >= last_leaf) {
-                s_front[atomicAdd(&s_nfront, 1)] = (int16_t)ns;
+                s_front[l - base] = (int16_t)ns;
                 break;
             }
             const int li = sp - base;
@@ -823,16 +826,30 @@ __global__ __launch_bounds__(kLbvhThreads) void k_lbvh_local(ClimbArgs a) {
     // In-block parents with one arrival: the other child lies (partly)
     // outside the block, so the arrived child continues at the top level.
     for (int i = threadIdx.x; i < T; i += kLbvhThreads)
-        if (s_cnt[i] == 1) s_front[atomicAdd(&s_nfront, 1)] = s_left[i] >= 0 ? s_left[i] : s_right[i];
+        if (s_cnt[i] == 1) {
+            const int16_t ns = s_left[i] >= 0 ? s_left[i] : s_right[i];
+            s_front[ns < T ? s_first[ns] : ns - T] = ns;
+        }
     __syncthreads();
-    if (threadIdx.x == 0) s_fbase = atomicAdd(a.frontier_count, s_nfront);
-    __syncthreads();
-    for (int i = threadIdx.x; i < s_nfront; i += kLbvhThreads) a.frontier[s_fbase + i] = node_of(s_front[i]);
-    // Boxes and costs go out only where the top level reads them (nodes whose
-    // parent it completes); the emit reads the Bin rows each state-1 or root
-    // node gets from its children's boxes here.  Parents outside the block are
-    // written -1 here and set by the top level, which climbs from every
-    // frontier node.
+    // The frontier in position order: the list of this block.
+    static_assert(kLbvhThreads == T, "one position per thread");
+    {
+        const int16_t ns = s_front[threadIdx.x];
+        const uint64_t m = ballot64(ns >= 0);
+        if (lane_id() == 0) s_wfront[threadIdx.x / kWave] = __popcll(m);
+        __syncthreads();
+        int rank = count_below(m), total = 0;
+        for (int w = 0; w < T / kWave; ++w) {
+            if (w == (int)threadIdx.x / kWave) rank += total;
+            total += s_wfront[w];
+        }
+        if (ns >= 0) a.frontier[base + rank] = node_of(ns);
+        if (threadIdx.x == 0) a.list_count[blockIdx.x] = total;
+    }
+    // Boxes and costs go out only where a merge reads them (nodes whose parent
+    // it completes); the emit reads the Bin rows each state-1 or root node gets
+    // from its children's boxes here.  Parents outside the block are written -1
+    // here and set by the merges, which climb from every frontier node.
     auto store_box = [&](int node, int sl) {
         const int po = s_par[sl];
         const bool parent_here = po >= 0 && s_cnt[po] == 2;
@@ -854,8 +871,8 @@ __global__ __launch_bounds__(kLbvhThreads) void k_lbvh_local(ClimbArgs a) {
         store_box(n - 1 + base + i, T + i);
     }
     // Internal nodes of the block's split range: the finished ones written
-    // out coalesced; the others are completed by the top level, whose
-    // arrival words start cleared.
+    // out coalesced; the others are completed by the merges (or by k_lbvh_top,
+    // whose arrival words start cleared).
     for (int i = threadIdx.x; i < T; i += kLbvhThreads) {
         const int node = base + i;
         if (node >= n - 1) break;
@@ -891,12 +908,14 @@ __global__ __launch_bounds__(kLbvhThreads) void k_lbvh_local(ClimbArgs a) {
 // the sibling and the parent's range from the atomic's result.  A node's box
 // travels in registers up the chain and through nmin/nmax (sc1 stores that
 // complete before the arrival) to the sibling.
+// Only lists that do not fit the merges' LDS come here (k_lbvh_merge's last
+// workgroup), so a key order in which hundreds of nodes straddle a block still
+// builds; the chains are bound by the ~3 us of a level's round trips.
 template <bool K64>
-__global__ __launch_bounds__(kBlock) void k_lbvh_top(ClimbArgs a) {
-    const int count = *a.frontier_count;
+HX_DEV void lbvh_top(const ClimbArgs& a, const int32_t* list, int count) {
     const int n = (int)a.n;
-    for (int e = blockIdx.x * kBlock + threadIdx.x; e < count; e += gridDim.x * kBlock) {
-        int node = a.frontier[e];
+    for (int e = threadIdx.x; e < count; e += blockDim.x) {
+        int node = list[e];
         int l, r;
         if (node >= n - 1) {
             l = r = node - (n - 1);
@@ -966,6 +985,192 @@ __global__ __launch_bounds__(kBlock) void k_lbvh_top(ClimbArgs a) {
             node = sp;
         }
     }
+}
+
+// One workgroup merges `lists` consecutive frontier lists of `stride` slots each
+// (list k at a.frontier + k * stride, its length in_count[k]): entry e of their
+// concatenation is a node, entries are consecutive leaf ranges, and a node over
+// entries [i, j] joins the boundary right of j or left of i, whichever has the
+// longer common prefix, so a merge is the climb of k_lbvh_local with entries
+// for leaves.  Boxes, costs and links stay in LDS; a level costs ~0.25 us
+// against ~3 us for the round trips between XCDs of a climb on global memory
+// (arrival words by device atomics, boxes by sc1 stores and loads), which bound
+// the whole top: 4,099 triangles 29 -> 13 us, 65,536 56 -> 34 us, 16.7M 320 ->
+// 257 us (what is left there is the latency of cold scattered reads).  The frontier that is left goes to the workgroup's
+// first list slot and out_count.  LAST: one workgroup holds every list and
+// finishes the tree.  More entries than kMergeCap (a block has ~8, but a skewed
+// key order can have hundreds) are passed on unmerged; LAST climbs them on
+// global memory.
+constexpr int kMergeThreads = 256;
+constexpr int kMergeCap = 640;
+
+template <bool K64, bool LAST>
+__global__ __launch_bounds__(kMergeThreads) void k_lbvh_merge(ClimbArgs a, const int32_t* __restrict__ in_count,
+                                                              int nlists, int lists, int64_t stride,
+                                                              int32_t* __restrict__ out_count) {
+    constexpr int C = kMergeCap;
+    // Slots: entry e -> C + e, the node at the boundary right of entry e -> e.
+    __shared__ float s_box[6][2 * C];
+    __shared__ float s_cost[2 * C];
+    __shared__ int s_id[C], s_end[C];   // entry: node, last leaf
+    __shared__ int s_cnt[C];
+    __shared__ int16_t s_left[C], s_right[C], s_lo[C], s_hi[C], s_par[2 * C], s_out[C];
+    __shared__ int8_t s_state[C];
+    __shared__ uint8_t s_delta[C + 1];  // delta left of entry k, plus one
+    __shared__ int s_off[kMergeThreads + 1];
+    __shared__ int s_wt[kMergeThreads / kWave];
+    const int n = (int)a.n, tid = threadIdx.x;
+    const int l0 = blockIdx.x * lists, l1 = min(l0 + lists, nlists);
+    int32_t* const out = a.frontier + l0 * stride;
+    // Offsets of the lists in the concatenation (at most kMergeThreads of them).
+    {
+        const int c = l0 + tid < l1 ? in_count[l0 + tid] : 0;
+        int tot;
+        const int inc = block_inclusive_scan<kMergeThreads / kWave>(c, [](int x, int y) { return x + y; }, s_wt, tot);
+        s_off[tid + 1] = inc;
+        if (tid == 0) s_off[0] = 0;
+    }
+    __syncthreads();
+    const int E = s_off[l1 - l0];
+    auto source = [&](int e) {   // entry e's place in a.frontier
+        int lo = 0, hi = l1 - l0 - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (s_off[mid] <= e) lo = mid;
+            else hi = mid - 1;
+        }
+        return out + lo * stride + (e - s_off[lo]);
+    };
+    if (E > C) {
+        // In place: an entry never moves right, and a chunk is read before it is written.
+        for (int b = 0; b < E; b += kMergeThreads) {
+            const int e = b + tid;
+            const int v = e < E ? *source(e) : 0;
+            __syncthreads();
+            if (e < E) out[e] = v;
+            __syncthreads();
+        }
+        if (LAST) lbvh_top<K64>(a, out, E);
+        else if (tid == 0) out_count[blockIdx.x] = E;
+        return;
+    }
+    for (int e = tid; e < E; e += kMergeThreads) {
+        const int node = *source(e);
+        const int first = node >= n - 1 ? node - (n - 1) : a.first[node];
+        const int last = node >= n - 1 ? node - (n - 1) : a.last[node];
+        const float4 mn = a.nmin[node], mx = a.nmax[node];
+        s_id[e] = node;
+        s_end[e] = last;
+        const int sl = C + e;
+        s_box[0][sl] = mn.x; s_box[1][sl] = mn.y; s_box[2][sl] = mn.z;
+        s_box[3][sl] = mx.x; s_box[4][sl] = mx.y; s_box[5][sl] = mx.z;
+        s_cost[sl] = a.adaptive ? a.cost[node] : 0.0f;
+        s_delta[e] = (uint8_t)(first == 0 ? 0 : 1 + kdelta<K64>(first - 1, first, n, a.keys, a.mesh_of, a.mesh_off));
+        if (e == E - 1)
+            s_delta[E] = (uint8_t)(last == n - 1 ? 0 : 1 + kdelta<K64>(last, last + 1, n, a.keys, a.mesh_of, a.mesh_off));
+        s_cnt[e] = 0;
+        s_left[e] = s_right[e] = -1;
+        s_par[e] = s_par[C + e] = -1;
+        s_out[e] = -1;
+    }
+    __syncthreads();
+    const int leaf0 = E > 0 ? (s_id[0] >= n - 1 ? s_id[0] - (n - 1) : a.first[s_id[0]]) : 0;
+    auto first_leaf = [&](int i) { return i == 0 ? leaf0 : s_end[i - 1] + 1; };
+    auto box_mn = [&](int sl) { return make_float3(s_box[0][sl], s_box[1][sl], s_box[2][sl]); };
+    auto box_mx = [&](int sl) { return make_float3(s_box[3][sl], s_box[4][sl], s_box[5][sl]); };
+    // The node of slot sl: a boundary's node is numbered by its split position.
+    auto node_of = [&](int sl) { return sl < C ? s_end[sl] : s_id[sl - C]; };
+    for (int e = tid; e < E; e += kMergeThreads) {
+        int ns = C + e, i = e, j = e;
+        while (true) {
+            const bool as_left = s_delta[j + 1] > s_delta[i];
+            const int b = as_left ? j : i - 1;
+            if (b < 0 || b >= E - 1) {   // outside these lists, or the root
+                s_out[i] = (int16_t)ns;
+                break;
+            }
+            s_par[ns] = (int16_t)b;
+            if (as_left) {
+                s_left[b] = (int16_t)ns;
+                s_lo[b] = (int16_t)i;
+            } else {
+                s_right[b] = (int16_t)ns;
+                s_hi[b] = (int16_t)j;
+            }
+            if (__hip_atomic_fetch_add(&s_cnt[b], 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) == 0) break;
+            i = s_lo[b];
+            j = s_hi[b];
+            const int ls = s_left[b], rs = s_right[b];
+            const int l = first_leaf(i), r = s_end[j];
+            const Combined c = combine(a, l, r, box_mn(ls), box_mx(ls), s_cost[ls], box_mn(rs), box_mx(rs), s_cost[rs]);
+            s_box[0][b] = c.mn.x; s_box[1][b] = c.mn.y; s_box[2][b] = c.mn.z;
+            s_box[3][b] = c.mx.x; s_box[4][b] = c.mx.y; s_box[5][b] = c.mx.z;
+            s_cost[b] = c.cost;
+            s_state[b] = (int8_t)c.state;
+            if (c.state == 0 && !seg_top(a.mesh_of, a.mesh_off, n, l, r)) atomicMax(&a.end_at[l], r);
+            ns = b;
+        }
+    }
+    __syncthreads();
+    // Boundaries with one arrival: the arrived child stays on the frontier.
+    for (int b = tid; b < E; b += kMergeThreads)
+        if (s_cnt[b] == 1) {
+            const int ns = s_left[b] >= 0 ? s_left[b] : s_right[b];
+            s_out[ns < C ? s_lo[ns] : ns - C] = (int16_t)ns;
+            s_par[ns] = -1;
+        }
+    __syncthreads();
+    for (int k = tid; k < 2 * E; k += kMergeThreads) {
+        const int e = k < E ? k : k - E;
+        const int sl = k < E ? e : C + e;
+        if (sl < C && s_cnt[e] != 2) continue;   // no node at this boundary
+        const int node = node_of(sl);
+        const int po = s_par[sl];
+        a.parent[node] = po >= 0 ? s_end[po] : -1;
+        if (sl >= C) continue;
+        const int l = first_leaf(s_lo[e]), r = s_end[s_hi[e]];
+        const int ls = s_left[e], rs = s_right[e];
+        a.first[node] = l;
+        a.last[node] = r;
+        a.left[node] = node_of(ls);
+        a.right[node] = node_of(rs);
+        a.state[node] = s_state[e];
+        if (a.all_boxes || po < 0) {
+            a.nmin[node] = make_float4(s_box[0][sl], s_box[1][sl], s_box[2][sl], 0.0f);
+            a.nmax[node] = make_float4(s_box[3][sl], s_box[4][sl], s_box[5][sl], 0.0f);
+            if (a.adaptive) a.cost[node] = s_cost[sl];
+        }
+        if (s_state[e] == 1 || seg_top(a.mesh_of, a.mesh_off, n, l, r)) {
+            auto row = [&](int q, int x) { return make_float4(s_box[q][x], s_box[q + 1][x], s_box[q + 2][x], 0.0f); };
+            int4 r0, r1, r2;
+            bin_rows(row(0, ls), row(3, ls), row(0, rs), row(3, rs), r0, r1, r2);
+            int4* pr = reinterpret_cast<int4*>(a.proto + 3 * (int64_t)node);
+            pr[0] = r0;
+            pr[1] = r1;
+            pr[2] = r2;
+        }
+    }
+    if (LAST) {
+        // One node is left: the root.
+        if (tid == 0) *a.root_id = node_of(s_out[0]);
+        return;
+    }
+    int total = 0;
+    for (int b = 0; b < E; b += kMergeThreads) {
+        const int e = b + tid;
+        const int ns = e < E ? s_out[e] : -1;
+        const uint64_t m = ballot64(ns >= 0);
+        __syncthreads();
+        if (lane_id() == 0) s_wt[tid / kWave] = __popcll(m);
+        __syncthreads();
+        int rank = total + count_below(m);
+        for (int w = 0; w < kMergeThreads / kWave; ++w) {
+            if (w < tid / kWave) rank += s_wt[w];
+            total += s_wt[w];
+        }
+        if (ns >= 0) out[rank] = node_of(ns);
+    }
+    if (tid == 0) out_count[blockIdx.x] = total;
 }
 
 // ---------------------------------------------------------------------------
@@ -1640,24 +1845,48 @@ int launch_climb(Context* c, const ClimbArgs& a) {
     return check_launch("climb_top");
 }
 
-int launch_lbvh_climb(Context* c, const ClimbArgs& a) {
+int launch_lbvh_climb(Context* c, const ClimbArgs& args) {
     LaunchScope ls(c, "climb");
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, a.frontier_count, 0, (int64_t)1);
-    HX_TRY(check_launch("frontier_reset"));
-    const unsigned blocks = (unsigned)((a.n + kLbvhLeaves - 1) / kLbvhLeaves);
+    ClimbArgs a = args;
+    const int blocks = (int)((a.n + kLbvhLeaves - 1) / kLbvhLeaves);
+    // List lengths of every merge level behind each other.
+    HX_TRY(c->scan_partials.reserve(sizeof(int32_t) * (2 * (size_t)blocks + 64)));
+    a.list_count = c->scan_partials.as<int32_t>();
     if (a.keys64)
         hipLaunchKernelGGL(k_lbvh_local<true>, dim3(blocks), dim3(kLbvhThreads), 0, c->stream, a);
     else
         hipLaunchKernelGGL(k_lbvh_local<false>, dim3(blocks), dim3(kLbvhThreads), 0, c->stream, a);
     HX_TRY(check_launch("lbvh_local"));
-    // Every wave slot, as for the general climb (measured 1.483 -> 1.455 ms
-    // for the two climb kernels at 16.7M triangles against 4 blocks per CU).
-    const unsigned top = (unsigned)std::max(1, std::min<int>(c->cu_count * 8, (int)((a.n + kBlock - 1) / kBlock)));
-    if (a.keys64)
-        hipLaunchKernelGGL(k_lbvh_top<true>, dim3(top), dim3(kBlock), 0, c->stream, a);
-    else
-        hipLaunchKernelGGL(k_lbvh_top<false>, dim3(top), dim3(kBlock), 0, c->stream, a);
-    return check_launch("lbvh_top");
+    if (blocks == 1) return HX_OK;
+    // Each merge joins up to 16 lists a workgroup, the same
+    // number at every level.
+    constexpr int kMaxLists = 16;
+    static_assert(kMaxLists <= kMergeThreads, "one list per thread");
+    int levels = 1;
+    for (int64_t cover = kMaxLists; cover < blocks; cover *= kMaxLists) ++levels;
+    int per = 1;
+    auto covers = [&](int64_t g) {
+        int64_t cover = 1;
+        for (int k = 0; k < levels; ++k) cover *= g;
+        return cover >= blocks;
+    };
+    while (!covers(per)) ++per;
+    const int32_t* in = a.list_count;
+    int32_t* out = a.list_count + blocks;
+    int nlists = blocks;
+    int64_t stride = kLbvhLeaves;
+    while (true) {
+        const int groups = (nlists + per - 1) / per;
+        auto kernel = groups == 1 ? (a.keys64 ? k_lbvh_merge<true, true> : k_lbvh_merge<false, true>)
+                                  : (a.keys64 ? k_lbvh_merge<true, false> : k_lbvh_merge<false, false>);
+        hipLaunchKernelGGL(kernel, dim3(groups), dim3(kMergeThreads), 0, c->stream, a, in, nlists, per, stride, out);
+        HX_TRY(check_launch("lbvh_merge"));
+        if (groups == 1) return HX_OK;
+        in = out;
+        out += groups;
+        nlists = groups;
+        stride *= per;
+    }
 }
 
 int launch_collapse_emit(Context* c, const EmitArgs& a) {

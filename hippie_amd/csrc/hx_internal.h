@@ -156,6 +156,7 @@ struct ClimbArgs {
     float4* woop;
     int32_t* frontier;        // n entries: nodes whose parent straddles a climb block
     int32_t* frontier_count;  // zeroed by launch_construct (or launch_refit_reset)
+    int32_t* list_count;      // LBVH: frontier length of each block (set by launch_lbvh_climb)
     // ATRBVH preparation outputs (Karras trees only; NULL otherwise): 2n-1
     // areas and binary SAH costs, n-1 subtree sizes and heights.
     float* atr_area;
@@ -183,8 +184,8 @@ struct ClimbArgs {
 int launch_climb(Context* c, const ClimbArgs& a);
 // Binary radix tree of the sorted keys built bottom-up together with the
 // climb (boxes, Woop rows, costs, collapse states); internal nodes are
-// numbered by split position.  frontier_count must be zero on entry.
-int launch_lbvh_climb(Context* c, const ClimbArgs& a);
+// numbered by split position.
+int launch_lbvh_climb(Context* c, const ClimbArgs& args);
 struct EmitArgs {
     int64_t n;
     const int32_t* left;

@@ -376,3 +376,73 @@ def test_validate_single_triangle(ctx):
     t = np.array([[0, 1, 2]], np.int32)
     bvh = hx.LBVHBuilder(ctx).build(hx.Scene(v, t))
     assert bvh.validate() == 0
+
+
+@pytest.mark.parametrize("n", [2, 63, 64, 65, 1023, 1024, 1025, 4099, 8191, 8192, 8193])
+@pytest.mark.parametrize("bits", [1, 8, 9, 30, 39, 40, 41, 60, 64])
+def test_sort_pairs_one_workgroup(ctx, n, bits):
+    """Sorts of up to 8192 keys run in one workgroup (8193: the tiled passes):
+    random keys, few distinct keys and keys whose bits above `bits` differ."""
+    rng = np.random.default_rng(n * 100 + bits)
+    for k in (rng.integers(0, 1 << 63, n, dtype=np.uint64) * np.uint64(2) + np.uint64(1),
+              rng.integers(0, 7, n, dtype=np.uint64) << np.uint64(max(bits - 3, 0)), np.zeros(n, np.uint64)):
+        vals = rng.permutation(n).astype(np.int32)
+        kt = torch.from_numpy(k.view(np.int64).copy()).cuda()
+        vt = torch.from_numpy(vals.copy()).cuda()
+        hx.sort_pairs(ctx, kt, vt, bits)
+        mask = np.uint64((1 << bits) - 1)
+        order = np.argsort(k & mask, kind="stable")
+        assert np.array_equal(kt.cpu().numpy().view(np.uint64), k[order])
+        assert np.array_equal(vt.cpu().numpy(), vals[order])
+
+
+def _edge_heavy_blocks(clusters):
+    """Triangles whose sorted 60-bit codes agree in ever fewer bits from the
+    edges of every 512-leaf block to its middle, so that ~57 nodes straddle
+    each block (a random order has ~10)."""
+    top = 60 - max(int(clusters).bit_length(), 5)
+    alt = sum(1 << b for b in range(0, top, 2))
+    keys = []
+    for j in range(clusters + 1):
+        c = (j << top) | alt
+        below = [c & ~(1 << b) for b in range(0, top, 2)]
+        above = [c | (1 << b) for b in range(1, top, 2)]
+        per = 256 // (len(below) + 1)
+        if j > 0:
+            keys += below * per + [c] * (256 - per * len(below))
+        if j < clusters:
+            keys += above * per + [c] * (256 - per * len(above))
+    k = np.array(keys, np.uint64)
+    xyz = np.zeros((len(k), 3), np.int64)
+    for b in range(20):
+        for a in range(3):
+            xyz[:, a] |= ((k >> np.uint64(3 * b + a)) & np.uint64(1)).astype(np.int64) << b
+    v = np.repeat(((xyz + 0.5) / 1048575.0)[:, None, :], 3, 1)
+    v[:, 1, 0] += 1e-7
+    v[:, 2, 1] += 1e-7
+    v[0, :], v[-1, :] = 0.0, 1.0  # the unit box
+    return v.astype(np.float32).reshape(-1, 3), np.arange(3 * len(v), dtype=np.int32).reshape(-1, 3)
+
+
+# 16 and 31 blocks fit one and two merge levels, 200 clusters overflow the first
+# level's workgroups, 16 the last one's (640 entries; 16 x 57 of them).
+@pytest.mark.parametrize("clusters", [1, 2, 16, 30, 200])
+def test_lbvh_merge_of_straddling_nodes(oracle, ctx, clusters):
+    v, t = _edge_heavy_blocks(clusters)
+    bvh = hx.LBVHBuilder(ctx, morton_bits=60).build(hx.Scene(v, t))
+    ref = oracle.build_lbvh(v, t, bits=60)
+    a = oracle.bin_canonical(bvh.nodes_host(), bvh.n_interior, bvh.n_leaves, bvh.tri_indices_host())
+    b = oracle.bin_canonical(ref["nodes"], ref["n_interior"], ref["n_leaves"], ref["tri_idx"])
+    assert np.array_equal(a, b)
+
+
+# Blocks of 512 leaves, merges of up to 16 lists (one level up to 8192 leaves).
+@pytest.mark.parametrize("n", [2, 511, 512, 513, 1025, 8191, 8192, 8193, 131073])
+@pytest.mark.parametrize("adaptive", [0, 1])
+def test_lbvh_merge_level_edges(oracle, ctx, n, adaptive):
+    v, t = scenes.uniform_soup(n, seed=n)
+    bvh = hx.LBVHBuilder(ctx, morton_bits=60, adaptive_leaf_size=adaptive, max_leaf_size=3).build(hx.Scene(v, t))
+    ref = oracle.build_lbvh(v, t, bits=60, adaptive=bool(adaptive), max_leaf_size=3)
+    a = oracle.bin_canonical(bvh.nodes_host(), bvh.n_interior, bvh.n_leaves, bvh.tri_indices_host())
+    b = oracle.bin_canonical(ref["nodes"], ref["n_interior"], ref["n_leaves"], ref["tri_idx"])
+    assert np.array_equal(a, b)
