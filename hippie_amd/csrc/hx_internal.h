@@ -577,6 +577,7 @@ struct TraceArgs {
     int fetch_threshold;    // dynamic fetch: busy lanes below which a wave refills
     int lanes;              // rays per wave, and the run length's divisor (set by the launch)
     int run_shift;
+    int share_busy;         // lanes share rays while at most this many of a wave are busy
     // Batched trace (else NULL): each ray traverses its own mesh's BVH.
     const int32_t* ray_mesh;
     const int4* mesh_tab;   // per mesh {node base, ...}

@@ -118,6 +118,39 @@ struct TraversalStack {
     }
 };
 
+// Lanes that share a ray (SHARE).  When a wave's rays are all handed out, its
+// idle lanes take stack entries of its busy lanes and traverse them for the same
+// ray; the ray's best hit lives in the owner lane's slot.  (t, id) packs into
+// one word whose order is "smaller t, then smaller id", the tie rule, so an LDS
+// atomic minimum merges hits, and every lane adopts the best one once a round.
+// The closest hit does not depend on which lane tests what.
+// A ray is a serial chain of ~0.4 us a visit, hundreds of visits for the longest
+// ones, so small ray sets and the end of every launch last as long as their
+// longest rays: 4,096 rays 40 -> 26 us, 16,384 147 -> 49 us, 65,536 340 -> 182 us,
+// 262,144 268 -> 225 us, 1,048,576 399 -> 365 us, 4.2M camera rays 1216 -> 1039 us.
+// What is taken: while few lanes are busy the lowest entry, the largest subtree,
+// which spreads the work fastest; else the top one, the next the lane would
+// visit, since far subtrees are mostly culled once the near ones are done (always
+// the lowest: 262,144 rays 332 us; always the top: 16,384 rays 77 us).
+struct ShareSlot {
+    uint64_t key;
+    float2 uv;
+};
+// Orders this wave's LDS accesses (no instruction: the wave runs in lockstep).
+HX_DEV void wave_fence() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); }
+constexpr int kShareLow = 16;     // busy lanes up to which the lowest entry is taken
+constexpr int kShareVisits = 8;   // node visits between two rounds of sharing
+HX_DEV uint64_t share_key(float t, int32_t id) {
+    const uint32_t b = __float_as_uint(t);
+    return (uint64_t)(b ^ (b >> 31 ? 0xFFFFFFFFu : 0x80000000u)) << 32 | (uint32_t)id;
+}
+HX_DEV void share_adopt(uint64_t key, float& t, int32_t& id, bool always = false) {
+    if (!always && key >= share_key(t, id == -1 ? 0 : id)) return;
+    const uint32_t b = (uint32_t)(key >> 32);
+    t = __uint_as_float(b ^ (b >> 31 ? 0x80000000u : 0xFFFFFFFFu));
+    id = (int32_t)(uint32_t)key;
+}
+
 // POSTPONE: leaves a lane may hold back while its wave still traverses (1, as
 // HipTracerBinKernels.cu:169-177; 2 is the reference's commented variant,
 // :171-173, 255; up to 4 here).  Held leaves wait in leafAddr (newest) ..
@@ -133,9 +166,10 @@ struct TraversalStack {
 // one node paid for themselves only while the ray counter set the pace; with
 // RayPool they cost 1,048,576 primaries 3 % and 16,384 rays 10 % (the check and
 // the scalar cache's latency) and gave sorted primaries nothing.
-template <bool STATS, bool ORDERED, int LDS_DEPTH, int POSTPONE, int AHEAD>
+template <bool STATS, bool ORDERED, int LDS_DEPTH, int POSTPONE, int AHEAD, bool SHARE>
 HX_TRACE_KERNEL __attribute__((amdgpu_waves_per_eu(LDS_DEPTH <= 16 ? 8 : 1))) void k_trace(TraceArgs a) {
     __shared__ int32_t s_stack[LDS_DEPTH > 0 ? LDS_DEPTH * kTraceBlock : 1];
+    __shared__ ShareSlot s_share[SHARE ? kTraceBlock : 1];
     TraversalStack<LDS_DEPTH> stack;
     stack.col = (lds_i32*)(s_stack + threadIdx.x);
     int sp = 0;
@@ -144,65 +178,150 @@ HX_TRACE_KERNEL __attribute__((amdgpu_waves_per_eu(LDS_DEPTH <= 16 ? 8 : 1))) vo
     float hitT = 0.f, hitU = 0.f, hitV = 0.f;
     int32_t nodeAddr = kSentinel, leafAddr = 0, leafAddr2 = 0, leafAddr3 = 0, leafAddr4 = 0, hitIndex = -1,
             hitId = -1;
-    int64_t rayidx = 0;
+    int32_t rayidx = -1;
     int32_t nNodes = 0, nTris = 0;
     // Batched trace: this lane's mesh (node base, first triangle position).
-    int64_t nodeBase = 0, triBase = 0;
-    if (lane_id() >= a.lanes) return;
+    int32_t nodeBase = 0, triBase = 0;
+    const int lane = lane_id();
+    if (!SHARE && lane >= a.lanes) return;
     RayPool pool;
     pool.start(a);
+    // SHARE, once the rays are handed out: lane whose ray this lane works on,
+    // its slot, and this lane's lowest stack entry that may be given away.
+    ShareSlot* const wave_slots = s_share + (SHARE ? threadIdx.x - lane : 0);
+    bool sharing = false;
+    int share = lane | 1 << 8;   // owner lane, lowest entry << 8
 
     while (true) {
         // Fetch new rays for the terminated lanes of this wave.
-        const bool terminated = nodeAddr == kSentinel;
-        const uint64_t tmask = ballot64(terminated);
-        const int slot = pool.take(terminated, tmask, __popcll(tmask), a.control);
-        if (terminated) {
-            rayidx = slot;
-            if (rayidx >= a.n_rays) break;
-            if (ORDERED) rayidx = a.order[rayidx];
-            if (a.ray_mesh) {
-                const int m = a.ray_mesh[rayidx];
-                if ((unsigned)m >= (unsigned)a.n_meshes) {  // no such mesh: a miss
-                    reinterpret_cast<int2*>(a.results)[2 * rayidx] =
-                        make_int2(-1, __float_as_int(a.rays[2 * rayidx + 1].w));
+        const bool terminated = nodeAddr == kSentinel && (!SHARE || lane < a.lanes);
+        if (!sharing) {
+            const uint64_t tmask = ballot64(terminated);
+            const int slot = pool.take(terminated, tmask, __popcll(tmask), a.control);
+            if (terminated && (!SHARE || slot < (int)a.n_rays)) {
+                if (!SHARE && slot >= (int)a.n_rays) break;
+                rayidx = ORDERED ? a.order[slot] : slot;
+                const int m = a.ray_mesh ? a.ray_mesh[rayidx] : 0;
+                if (a.ray_mesh && (unsigned)m >= (unsigned)a.n_meshes) {  // no such mesh: a miss
+                    reinterpret_cast<int2*>(a.results)[2 * (int64_t)rayidx] =
+                        make_int2(-1, __float_as_int(a.rays[2 * (int64_t)rayidx + 1].w));
                     if (STATS) a.stats[rayidx] = make_int2(0, 0);
-                    continue;
+                    rayidx = -1;
+                } else {
+                    if (a.ray_mesh) {
+                        nodeBase = a.mesh_tab[m].x;
+                        triBase = a.mesh_off[m];
+                    }
+                    const float4 o = a.rays[2 * (int64_t)rayidx + 0];
+                    const float4 d = a.rays[2 * (int64_t)rayidx + 1];
+                    ox = o.x; oy = o.y; oz = o.z; tmin = o.w;
+                    dx = d.x; dy = d.y; dz = d.z; hitT = d.w;
+                    const float ooeps = 8.2718061255302767e-25f;  // exp2f(-80)
+                    idx = 1.0f / (fabsf(dx) > ooeps ? dx : copysignf(ooeps, dx));
+                    idy = 1.0f / (fabsf(dy) > ooeps ? dy : copysignf(ooeps, dy));
+                    idz = 1.0f / (fabsf(dz) > ooeps ? dz : copysignf(ooeps, dz));
+                    oodx = ox * idx;
+                    oody = oy * idy;
+                    oodz = oz * idz;
+                    stack.put(0, kSentinel);
+                    sp = 0;
+                    leafAddr = 0;
+                    leafAddr2 = 0;
+                    leafAddr3 = 0;
+                    leafAddr4 = 0;
+                    nodeAddr = 0;
+                    hitIndex = -1;
+                    hitId = -1;
+                    if (STATS) { nNodes = 0; nTris = 0; }
                 }
-                nodeBase = a.mesh_tab[m].x;
-                triBase = a.mesh_off[m];
             }
-            const float4 o = a.rays[2 * rayidx + 0];
-            const float4 d = a.rays[2 * rayidx + 1];
-            ox = o.x; oy = o.y; oz = o.z; tmin = o.w;
-            dx = d.x; dy = d.y; dz = d.z; hitT = d.w;
-            const float ooeps = 8.2718061255302767e-25f;  // exp2f(-80)
-            idx = 1.0f / (fabsf(dx) > ooeps ? dx : copysignf(ooeps, dx));
-            idy = 1.0f / (fabsf(dy) > ooeps ? dy : copysignf(ooeps, dy));
-            idz = 1.0f / (fabsf(dz) > ooeps ? dz : copysignf(ooeps, dz));
-            oodx = ox * idx;
-            oody = oy * idy;
-            oodz = oz * idz;
-            stack.put(0, kSentinel);
-            sp = 0;
-            leafAddr = 0;
-            leafAddr2 = 0;
-            leafAddr3 = 0;
-            leafAddr4 = 0;
-            nodeAddr = 0;
-            hitIndex = -1;
-            hitId = -1;
-            if (STATS) { nNodes = 0; nTris = 0; }
+        }
+        int visits = 0x7fffffff;
+        if (SHARE && (sharing || (pool.next >= pool.end && pool.base >= pool.n))) {
+            if (!sharing) {
+                sharing = true;
+                wave_slots[lane].key = share_key(hitT, hitIndex == -1 ? 0 : hitId);
+                wave_slots[lane].uv = make_float2(hitU, hitV);
+                hitIndex = -1;
+            }
+            ShareSlot* const mine = wave_slots + (share & 0xFF);
+            wave_fence();
+            if (hitIndex != -1) {   // a hit since the last round
+                const uint64_t key = share_key(hitT, hitId);
+                // A ray that may hit at t <= 0 is not shared: -0 and 0 tie, but
+                // not as keys.
+                if (tmin >= 0.0f) __hip_atomic_fetch_min(&mine->key, key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                else mine->key = key;
+                wave_fence();
+                if (mine->key == key) mine->uv = make_float2(hitU, hitV);
+                hitIndex = -1;
+            }
+            wave_fence();
+            const uint64_t busy = ballot64(nodeAddr != kSentinel);
+            if (!busy) break;
+            // The best hit of the ray so far, whoever found it.
+            if (nodeAddr != kSentinel) share_adopt(mine->key, hitT, hitId);
+            // The k-th idle lane takes the lowest stack entry of the k-th lane that has one.
+            const bool low = __popcll(busy) <= kShareLow;
+            const bool gives = nodeAddr != kSentinel && (share >> 8) <= sp && (low ? share >> 8 : sp) < LDS_DEPTH && tmin >= 0.0f;
+            const uint64_t gm = ballot64(gives);
+            const uint64_t im = ~busy;
+            const int pairs = min(__popcll(gm), __popcll(im));
+            if (pairs > 0 && __popcll(busy) <= a.share_busy) {
+                const int grank = count_below(gm), irank = count_below(im);
+                // Lane k learns the k-th giving lane.
+                const int kth = __builtin_amdgcn_ds_permute((gives ? grank : 63) << 2, lane);
+                const bool takes = nodeAddr == kSentinel && irank < pairs;
+                const int from = __shfl(kth, takes ? irank : 0, kWave);
+                const int e = __shfl(low ? share >> 8 : sp, from, kWave);
+                lds_i32* const src = stack.col - lane + from + e * kTraceBlock;
+                int32_t got = 0;
+                if (takes) {
+                    got = *src;
+                    if (low) *src = kSentinel;
+                }
+                if (gives && grank < pairs) {
+                    if (low) share += 1 << 8;
+                    else --sp;
+                }
+                auto copy = [&](auto& v) {
+                    const auto x = __shfl(v, from, kWave);
+                    if (takes) v = x;
+                };
+                copy(ox); copy(oy); copy(oz); copy(tmin);
+                copy(dx); copy(dy); copy(dz);
+                copy(idx); copy(idy); copy(idz);
+                copy(oodx); copy(oody); copy(oodz);
+                copy(hitT); copy(hitId); copy(share);
+                if (a.ray_mesh) {
+                    copy(nodeBase);
+                    copy(triBase);
+                }
+                if (takes) {
+                    nodeAddr = got;
+                    leafAddr = leafAddr2 = leafAddr3 = leafAddr4 = 0;
+                    stack.put(0, kSentinel);
+                    sp = 0;
+                    share = (share & 0xFF) | 1 << 8;
+                }
+            }
+            wave_fence();
+            visits = kShareVisits;
         }
 
         while (nodeAddr != kSentinel) {
+            if (SHARE && nodeAddr < 0) {   // a leaf that was handed over: nothing else is on the stack
+                leafAddr = nodeAddr;
+                nodeAddr = kSentinel;
+            }
             const int half = __popcll(ballot64(true)) >> 1;
+            int left = visits;
             while ((uint32_t)nodeAddr < (uint32_t)kSentinel) {
                 if (STATS) ++nNodes;
                 float c0min, c0max, c1min, c1max;
                 int2 cn;
                 {
-                    const int64_t na = nodeBase + nodeAddr;
+                    const int64_t na = (uint32_t)(nodeBase + nodeAddr);
                     const float4* np = reinterpret_cast<const float4*>(a.nodes + 4 * na);
                     const float4 n0xy = np[0];
                     const float4 n1xy = np[1];
@@ -270,15 +389,16 @@ HX_TRACE_KERNEL __attribute__((amdgpu_waves_per_eu(LDS_DEPTH <= 16 ? 8 : 1))) vo
                     nodeAddr = stack.get(sp--);
                 }
                 if (!__any(leafAddr >= 0) || __popcll(ballot64(true)) <= half) break;
+                if (SHARE && --left == 0) break;
             }
 
             while (leafAddr < 0) {
-                const int4 lb = a.nodes[4 * (nodeBase + ~leafAddr) + 3];
+                const int4 lb = a.nodes[4 * (int64_t)(uint32_t)(nodeBase + ~leafAddr) + 3];
                 // The next triangle's first Woop row (AHEAD = 1), or its first
                 // two (AHEAD = 2), are read while this one is tested: leaves of
                 // long thin triangles test hundreds per ray, and most of those
                 // tests pass the plane test and need the second row.
-                const float4* wrow = a.woop + 3 * (triBase + lb.x);
+                const float4* wrow = a.woop + 3 * (int64_t)(triBase + lb.x);
                 float4 vnext = lb.x < lb.y ? wrow[0] : make_float4(0.f, 0.f, 0.f, 0.f);
                 float4 vnext1 = AHEAD >= 2 && lb.x < lb.y ? wrow[1] : make_float4(0.f, 0.f, 0.f, 0.f);
                 for (int tri = lb.x; tri < lb.y; ++tri, wrow += 3) {
@@ -332,16 +452,29 @@ HX_TRACE_KERNEL __attribute__((amdgpu_waves_per_eu(LDS_DEPTH <= 16 ? 8 : 1))) vo
                 }
             }
 
-            if (__popcll(ballot64(true)) < a.fetch_threshold) break;
+            if (__popcll(ballot64(true)) < a.fetch_threshold || (SHARE && sharing)) break;
         }
 
-        if (nodeAddr == kSentinel) {
+        if (nodeAddr == kSentinel && rayidx >= 0 && !(SHARE && sharing)) {
             if (hitIndex == -1)
-                reinterpret_cast<int2*>(a.results)[2 * rayidx] = make_int2(-1, __float_as_int(hitT));
+                reinterpret_cast<int2*>(a.results)[2 * (int64_t)rayidx] = make_int2(-1, __float_as_int(hitT));
             else
                 a.results[rayidx] =
                     make_int4(hitId, __float_as_int(hitT), __float_as_int(hitU), __float_as_int(hitV));
             if (STATS) a.stats[rayidx] = make_int2(nNodes, nTris);
+            rayidx = -1;
+        }
+    }
+    if (SHARE && rayidx >= 0) {
+        const ShareSlot r = wave_slots[lane];
+        const float tmax = a.rays[2 * (int64_t)rayidx + 1].w;
+        if (r.key == share_key(tmax, 0)) {
+            reinterpret_cast<int2*>(a.results)[2 * (int64_t)rayidx] = make_int2(-1, __float_as_int(tmax));
+        } else {
+            float t = 0.0f;
+            int32_t id = 0;
+            share_adopt(r.key, t, id, true);
+            a.results[rayidx] = make_int4(id, __float_as_int(t), __float_as_int(r.uv.x), __float_as_int(r.uv.y));
         }
     }
 }
@@ -653,12 +786,17 @@ __global__ void k_zero_control(int32_t* control) {
 // over more of them: half as many rays per wave while that still leaves waves
 // idle, down to 16 (65,536 rays over 1M triangles 500 -> 357 us, 16,384 over
 // 64k 187 -> 157 us; 8 or 4 rays per wave were slower, 484 us, since the address
-// units take 4 lanes a cycle and neighbouring rays share nodes).
-unsigned trace_shape(Context* c, int occ, TraceArgs& a) {
+// units take 4 lanes a cycle and neighbouring rays share nodes), or 8 where the
+// other lanes share the rays (16,384 rays 60 -> 49 us).  While every wave has
+// such lanes from the start they join at once; later, when the chip is full,
+// only once half a wave is idle (262,144 rays 259 -> 225 us).
+unsigned trace_shape(Context* c, int occ, bool share, TraceArgs& a) {
     const int per_cu = c->tune.trace_blocks_per_cu > 0 ? std::min(c->tune.trace_blocks_per_cu, occ) : occ;
     const int64_t waves = (int64_t)c->cu_count * per_cu * (kTraceBlock / kWave);
     a.lanes = kWave;
-    while (a.lanes > 16 && a.n_rays <= waves * (a.lanes / 2)) a.lanes /= 2;
+    const int least = share ? 8 : 16;
+    while (a.lanes > least && a.n_rays <= waves * (a.lanes / 2)) a.lanes /= 2;
+    a.share_busy = a.n_rays <= waves * 16 ? kWave : kWave / 2;
     a.run_shift = 2;
     while (((int64_t)1 << (a.run_shift - 2)) < waves) ++a.run_shift;
     a.fetch_threshold = std::max(1, a.fetch_threshold * a.lanes / kWave);
@@ -667,19 +805,28 @@ unsigned trace_shape(Context* c, int occ, TraceArgs& a) {
                                                             (a.n_rays + per_block - 1) / per_block));
 }
 
-template <bool STATS, bool ORDERED, int LDS_DEPTH, int POSTPONE, int AHEAD>
+// Sharing pays where the longest rays show: up to 16 rays a lane slot.  Above
+// (16.7M rays and more) the tail is too short a part of the launch (sorted
+// primaries 3.19 -> 3.23 ms).  Batched rays lose by it (1.37M: 1131 -> 1187 us or
+// more): they are short and hit early.  An any-hit trace reports the first hit of
+// one lane's traversal order, and the counts of a stats trace are per ray.
+bool share_pays(const Context* c, const TraceArgs& a) {
+    return !a.any_hit && !a.stats && !a.ray_mesh && a.n_rays <= (int64_t)c->cu_count * 8 * kTraceBlock * 16;
+}
+
+template <bool STATS, bool ORDERED, int LDS_DEPTH, int POSTPONE, int AHEAD, bool SHARE>
 int launch_trace_t(Context* c, const TraceArgs& a) {
     // Occupancy limit of this instantiation, queried once per process.
     static int occ = 0;
     if (occ == 0) {
         int q = 0;
-        HX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&q, k_trace<STATS, ORDERED, LDS_DEPTH, POSTPONE, AHEAD>,
+        HX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&q, k_trace<STATS, ORDERED, LDS_DEPTH, POSTPONE, AHEAD, SHARE>,
                                                              kTraceBlock, 0));
         occ = std::max(q, 1);
     }
     TraceArgs t = a;
-    const unsigned blocks = trace_shape(c, occ, t);
-    hipLaunchKernelGGL((k_trace<STATS, ORDERED, LDS_DEPTH, POSTPONE, AHEAD>), dim3(blocks), dim3(kTraceBlock), 0,
+    const unsigned blocks = trace_shape(c, occ, SHARE, t);
+    hipLaunchKernelGGL((k_trace<STATS, ORDERED, LDS_DEPTH, POSTPONE, AHEAD, SHARE>), dim3(blocks), dim3(kTraceBlock), 0,
                        c->stream, t);
     return check_launch("trace");
 }
@@ -687,11 +834,14 @@ int launch_trace_t(Context* c, const TraceArgs& a) {
 template <bool STATS, bool ORDERED, int POSTPONE, int AHEAD>
 int launch_trace_depth(Context* c, const TraceArgs& a) {
     switch (c->tune.trace_lds_stack) {
-        case 0: return launch_trace_t<STATS, ORDERED, 0, POSTPONE, AHEAD>(c, a);
-        case 16: return launch_trace_t<STATS, ORDERED, 16, POSTPONE, AHEAD>(c, a);
-        case 24: return launch_trace_t<STATS, ORDERED, 24, POSTPONE, AHEAD>(c, a);
-        case 32: return launch_trace_t<STATS, ORDERED, 32, POSTPONE, AHEAD>(c, a);
-        default: return launch_trace_t<STATS, ORDERED, 64, POSTPONE, AHEAD>(c, a);
+        case 0: return launch_trace_t<STATS, ORDERED, 0, POSTPONE, AHEAD, false>(c, a);
+        case 16:
+            if (!STATS && share_pays(c, a))
+                return launch_trace_t<false, ORDERED, 16, POSTPONE, AHEAD, true>(c, a);
+            return launch_trace_t<STATS, ORDERED, 16, POSTPONE, AHEAD, false>(c, a);
+        case 24: return launch_trace_t<STATS, ORDERED, 24, POSTPONE, AHEAD, false>(c, a);
+        case 32: return launch_trace_t<STATS, ORDERED, 32, POSTPONE, AHEAD, false>(c, a);
+        default: return launch_trace_t<STATS, ORDERED, 64, POSTPONE, AHEAD, false>(c, a);
     }
 }
 
@@ -723,7 +873,7 @@ int launch_trace_wide_t(Context* c, const TraceArgs& a) {
         occ = std::max(q, 1);
     }
     TraceArgs t = a;
-    const unsigned blocks = trace_shape(c, occ, t);
+    const unsigned blocks = trace_shape(c, occ, false, t);
     hipLaunchKernelGGL((k_trace_wide<N, STATS, ORDERED, LDS_DEPTH>), dim3(blocks), dim3(kTraceBlock), 0, c->stream, t);
     return check_launch("trace_wide");
 }

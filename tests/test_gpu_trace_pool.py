@@ -58,3 +58,56 @@ def test_wide_ray_counts(ctx, scene_data, layout, count):
         rb.launch = {"trace_blocks_per_cu": 1}
         out.append(hx.HipTracer(ctx, bvh).trace(rb).cpu().numpy())
     assert np.array_equal(*out)
+
+
+def _odd_rays(n, seed):
+    """Random rays with the limits a merge of hits has to keep: negative tmin
+    (hits behind the origin), empty, infinite and NaN intervals, dead rays."""
+    rng = np.random.default_rng(seed)
+    r = scenes.random_rays(n, seed=seed).copy()
+    k = n // 8
+    r[:k, 3] = -2.0
+    r[k:2 * k, 7] = np.inf
+    r[2 * k:3 * k, 7] = rng.uniform(0.0, 0.6, k)
+    r[3 * k:3 * k + 40, 7] = np.nan
+    r[3 * k + 40:3 * k + 80, 3] = np.nan
+    r[4 * k:4 * k + 100, 7] = -1.0
+    r[5 * k:5 * k + 100, 4:7] = 0.0
+    return r
+
+
+# Lanes share rays in the kernel with 16 stack entries in LDS; the one with 24
+# does not.  Every triangle is there three times, so equal distances are common.
+@pytest.mark.parametrize("n_rays", [1, 8, 65, 1000, 5000, 70000, 150000])
+@pytest.mark.parametrize("postpone", [1, 2, 4])
+def test_shared_rays_keep_hits(oracle, ctx, n_rays, postpone):
+    v, t = scenes.merge(*[scenes.uniform_soup(700, seed=5)] * 3, scenes.ground_grid(12))
+    bvh = hx.LBVHBuilder(ctx, morton_bits=60).build(hx.Scene(v, t))
+    rays = _odd_rays(n_rays, seed=n_rays)
+    out = []
+    for depth in (16, 24):
+        rb = hx.RayBuffer(rays)
+        rb.launch = {"trace_lds_stack": depth, "trace_postpone": postpone}
+        rb.results.fill_(0x7F7F7F7F)
+        out.append(hx.HipTracer(ctx, bvh).trace(rb).cpu().numpy())
+    assert np.array_equal(*out)
+    ref, _ = oracle.trace(bvh.nodes_host(), bvh.woop_host(), bvh.tri_indices_host(), rays)
+    assert np.array_equal(out[0][:, 0], ref[:, 0])
+
+
+@pytest.mark.parametrize("sort", [False, True])
+def test_shared_rays_deep_tree(oracle, ctx, sort):
+    """A tree deeper than the stack's LDS part: entries beyond it are not given away."""
+    n = 4000
+    v, t = scenes.uniform_soup(n, seed=9)
+    v = (v * np.exp2(-np.repeat(np.arange(n) % 19, 3)).astype(np.float32)[:, None]).astype(np.float32)
+    bvh = hx.LBVHBuilder(ctx, morton_bits=60, adaptive_leaf_size=0, max_leaf_size=1).build(hx.Scene(v, t))
+    rays = scenes.random_rays(20000, seed=10)
+    rays[:10000, 4:7] = -rays[:10000, 0:3] / np.linalg.norm(rays[:10000, 0:3], axis=1, keepdims=True)
+    rb = hx.RayBuffer(rays)
+    tr = hx.HipTracer(ctx, bvh)
+    res = (tr.trace_sort(rb) if sort else tr.trace(rb)).cpu().numpy()
+    ref, ov = oracle.trace(bvh.nodes_host(), bvh.woop_host(), bvh.tri_indices_host(), rays)
+    assert ov == 0 and ctx.overflow_count() == 0
+    hit = ref[:, 0] >= 0
+    assert np.array_equal(res[:, :2], ref[:, :2]) and np.array_equal(res[hit], ref[hit])
