@@ -22,7 +22,7 @@
 // reproduced exactly: findLeafToExpand over 2+i lanes and findMinimumDistance
 // (per-lane strided minimum over 32 lanes, then a 32-lane tree).  The
 // distance matrix lives in LDS; the treelet leaves live in the lanes'
-// registers and move by cross-lane permutes.
+// registers while it is formed and in LDS while it is merged.
 #include <algorithm>
 #include <vector>
 
@@ -49,10 +49,12 @@ inline unsigned grid_for(int64_t n, int block) { return (unsigned)((n + block - 
 // ATRBuilderKernels.cu:11-20; the row comes from a float square root, as in
 // the reference).
 HX_DEV int trm_index(int row, int col) { return ((row - 1) * row) / 2 + col; }
-HX_DEV int trm_row(int index) { return (int)((-1.0f + sqrtf(8.0f * (float)index + 1.0f)) / 2.0f) + 1; }
-HX_DEV int trm_col(int index) {
-    const int y = trm_row(index);
-    return index - (y * (y - 1)) / 2;
+// (row << 8 | col) of an index below kTrm.  sqrt(8 index + 2) lies at least
+// 0.008 above 2 row - 1 and 0.05 below 2 row + 1 there, so the hardware's square root
+// (1 ulp) gives the same row as the correctly rounded one.
+HX_DEV int trm_row_col(int index) {
+    const int row = (int)(0.5f * __builtin_amdgcn_sqrtf(8.0f * (float)index + 2.0f) - 0.5f) + 1;
+    return row << 8 | (index - (row * (row - 1)) / 2);
 }
 
 // TRBuilderUtil.h:100-130 (x*y + x*z + y*z, no validity test).
@@ -71,107 +73,164 @@ template <class T>
 HX_DEV T gshfl(T v, int src) { return __shfl(v, src, kG); }
 template <class T>
 HX_DEV T gshfl_down(T v, int d) { return __shfl_down(v, d, kG); }
-HX_DEV float3 gshfl3(float3 v, int src) { return make_float3(gshfl(v.x, src), gshfl(v.y, src), gshfl(v.z, src)); }
 
 // Orders this wave's LDS accesses (no instruction: the wave runs in lockstep).
 HX_DEV void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); }
 
+// Maximum over the 32 lanes of a group, in every lane, in VALU moves: rotations
+// inside the rows of 16 lanes, then a swap of the two rows.
+constexpr int kDppRowRor1 = 0x121, kDppRowRor2 = 0x122, kDppRowRor4 = 0x124, kDppRowRor8 = 0x128;
+HX_DEV float group_max(float v) {
+    v = fmaxf(v, dpp_move<kDppRowRor8, 0xF>(v));
+    v = fmaxf(v, dpp_move<kDppRowRor4, 0xF>(v));
+    v = fmaxf(v, dpp_move<kDppRowRor2, 0xF>(v));
+    v = fmaxf(v, dpp_move<kDppRowRor1, 0xF>(v));
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+    return fmaxf(__int_as_float((int)rows[0]), __int_as_float((int)rows[1]));
+}
+
+// v of lane `lane0` of the wave's first group to its lanes and of lane `lane1`
+// of the wave to the second group's.
+HX_DEV int group_pick(int v, int lane0, int lane1) {
+    const int v0 = __builtin_amdgcn_readlane(v, lane0), v1 = __builtin_amdgcn_readlane(v, lane1);
+    return lane_id() < kG ? v0 : v1;
+}
+
+// Lane of each group's largest value if no group of the wave has a tie or a
+// NaN: then every order of comparisons finds the same one.  Otherwise false,
+// and the caller takes the reference's shuffle tree, which decides ties.
+// `in`: the lane takes part.
+HX_DEV bool group_argmax(float v, bool in, int& lane0, int& lane1) {
+    const float top = group_max(in ? v : -__builtin_inff());
+    const uint64_t nan = ballot64(in && v != v), eq = ballot64(in && v == top);
+    const uint32_t lo = (uint32_t)eq, hi = (uint32_t)(eq >> 32);
+    lane0 = lo ? __builtin_ctz(lo) : 0;
+    lane1 = kG + (hi ? __builtin_ctz(hi) : 0);
+    return nan == 0 && (lo & (lo - 1)) == 0 && (hi & (hi - 1)) == 0;
+}
+
+HX_DEV int4 child_record(int l, int r, float al, float ar) {
+    return make_int4(l, r, __float_as_int(al), __float_as_int(ar));
+}
+
 // formTreelet (TRBuilderUtil.h:171-226): expand the treelet leaf of largest
 // area that is an internal node, t-2 times.  Lane i < t ends with treelet leaf
 // i in tl, lane i < t-1 with the treelet's internal node i in inode (lane 0:
-// the root X).
-HX_DEV void form_treelet(const AtrArgs& a, int X, int xl, int xr, int t, int lane, int& tl, int& inode) {
+// the root X, whose record is root).  The steps are a chain of dependent reads;
+// a node's record holds its children and their areas, so a step is one read.
+HX_DEV void form_treelet(const AtrArgs& a, int X, int4 root, int t, int lane, int& tl, int& inode) {
     const int n = (int)a.n;
     tl = -1;
     inode = -1;
     float tl_area = 0.0f;
     if (lane == 0) {
-        tl = xl;
-        tl_area = a.area[xl];
+        tl = root.x;
+        tl_area = __int_as_float(root.z);
         inode = X;
     }
     if (lane == 1) {
-        tl = xr;
-        tl_area = a.area[xr];
+        tl = root.y;
+        tl_area = __int_as_float(root.w);
     }
     for (int it = 0; it < t - 2; ++it) {
-        int idx = lane;
         float val = (tl >= n - 1) ? -kMaxFloat : tl_area;
-        for (int k = 2 + it; k > 1; k = (k + 1) / 2) {  // findLeafToExpand
-            const int s = k / 2;
-            const int oi = gshfl_down(idx, s);
-            const float ov = gshfl_down(val, s);
-            if (ov > val) {
-                val = ov;
-                idx = oi;
+        int e, rep, e0, e1;
+        if (group_argmax(val, lane < 2 + it, e0, e1)) {
+            e = (lane_id() < kG ? e0 : e1) & (kG - 1);
+            rep = group_pick(tl, e0, e1);
+        } else {
+            int idx = lane;
+            for (int k = 2 + it; k > 1; k = (k + 1) / 2) {  // findLeafToExpand
+                const int s = k / 2;
+                const int oi = gshfl_down(idx, s);
+                const float ov = gshfl_down(val, s);
+                if (ov > val) {
+                    val = ov;
+                    idx = oi;
+                }
             }
+            e = gshfl(idx, 0);
+            rep = gshfl(tl, e);
         }
-        const int e = gshfl(idx, 0);
-        const int rep = gshfl(tl, e);
-        const int cl = a.left[rep], cr = a.right[rep];
-        const float al = a.area[cl], ar = a.area[cr];
+        const int4 rec = a.children[rep];
         if (lane == it + 1) inode = rep;
         if (lane == e) {
-            tl = cl;
-            tl_area = al;
+            tl = rec.x;
+            tl_area = __int_as_float(rec.z);
         }
         if (lane == it + 2) {
-            tl = cr;
-            tl_area = ar;
+            tl = rec.y;
+            tl_area = __int_as_float(rec.w);
         }
     }
 }
 
-// One treelet per 32-lane group; task = index into the height bucket.
-__global__ __launch_bounds__(kAtrBlock) void k_atr_level(AtrArgs a, const int32_t* __restrict__ list, int count) {
-    __shared__ float s_d[kGroups][kTrm];
-    const int grp = threadIdx.x / kG;
-    const int lane = threadIdx.x & (kG - 1);
-    const int task = blockIdx.x * kGroups + grp;
-    if (task >= count) return;  // whole 32-lane groups leave together
-    float* D = s_d[grp];
+// LDS of one 32-lane group: the distance matrix and the state of the rows
+// (box, cost, node, size, height), read by every lane as broadcasts.
+struct AtrGroup {
+    float4 lo[kG];  // box minimum, SAH cost
+    float4 hi[kG];  // box maximum, node
+    int2 rh[kG];    // references, height
+    float d[kTrm + 1];
+};
+
+// The treelet of X by 32 lanes.  A wave holds two treelets and the levels of
+// the upper tree have fewer treelets than the chip has waves, so a level takes
+// what one treelet takes, a serial chain of t - 2 expansions and t - 1 joins
+// (9 leaves: 3.5 + 6.2 us of a 14 us level).  So a join is short: the minimum
+// by row rotations, ties alone by the reference's tree; the rows' state in LDS,
+// read as broadcasts together; no square root to the last bit.  1M triangles:
+// the 66 levels of a build 1941 us, now 34 and the two of k_atr_top 1609 us.
+HX_DEV void atr_treelet(const AtrArgs& a, int X, int lane, AtrGroup& g) {
     const int n = (int)a.n;
     const int t = a.treelet_size;
-    const int X = list[task];
+    float* const D = g.d;
 
     // The climb step at X (ATRBuilderKernels.cu:293-310): children are final.
-    const int xl = a.left[X], xr = a.right[X];
+    const int4 root = a.children[X];
+    const int xl = root.x, xr = root.y;
     const float costX = a.ct * a.area[X] + a.cost[xl] + a.cost[xr];
     const int hl = xl >= n - 1 ? 0 : a.height[xl];
     const int hr = xr >= n - 1 ? 0 : a.height[xr];
     const int heightX = 1 + max(hl, hr);
 
     int tl, inode;
-    form_treelet(a, X, xl, xr, t, lane, tl, inode);
+    form_treelet(a, X, root, t, lane, tl, inode);
 
     // Treelet leaves: node, box, cost, size, height per lane.
-    int node = tl, rnode = -1, refs = 1, hgt = 0, mrefs = 0, mh = 0;
-    float sah = 0.0f, mcost = 0.0f;
+    int node = tl, rnode = -1, mrefs = 0, mh = 0;
+    float mcost = 0.0f, larea = 0.0f, rarea = 0.0f;
     float3 mn = make_float3(0.0f, 0.0f, 0.0f), mx = mn;
     if (lane < t) {
         const float4 bmn = a.nmin[tl], bmx = a.nmax[tl];
-        mn = make_float3(bmn.x, bmn.y, bmn.z);
-        mx = make_float3(bmx.x, bmx.y, bmx.z);
-        sah = a.cost[tl];
+        const float sah = a.cost[tl];
+        int refs = 1, hgt = 0;
         if (tl < n - 1) {
             refs = a.refs[tl];
             hgt = a.height[tl];
         }
+        mn = make_float3(bmn.x, bmn.y, bmn.z);
+        mx = make_float3(bmx.x, bmx.y, bmx.z);
+        g.lo[lane] = make_float4(mn.x, mn.y, mn.z, sah);
+        g.hi[lane] = make_float4(mx.x, mx.y, mx.z, __int_as_float(tl));
+        g.rh[lane] = make_int2(refs, hgt);
     }
+    wave_lds_fence();
 
     // calculateDistancesMatrix (ATRBuilderKernels.cu:22-64): every pair.
     const int pairs = t * (t - 1) / 2;
-    for (int base = 0; base < pairs; base += kG) {
-        const int e = base + lane;
-        const int row = e < pairs ? trm_row(e) : 0;
-        const int col = e < pairs ? e - (row * (row - 1)) / 2 : 0;
-        const float3 amn = gshfl3(mn, row), amx = gshfl3(mx, row);
-        const float3 bmn = gshfl3(mn, col), bmx = gshfl3(mx, col);
-        if (e < pairs) D[e] = atr_union_area(amn, amx, bmn, bmx);
+    for (int e = lane; e < pairs; e += kG) {
+        const int rc = trm_row_col(e), row = rc >> 8, col = rc & 0xFF;
+        D[e] = atr_union_area(xyz(g.lo[row]), xyz(g.hi[row]), xyz(g.lo[col]), xyz(g.hi[col]));
     }
     wave_lds_fence();
 
     for (int lastRow = t - 1; lastRow > 0; --lastRow) {
+        // What does not hang on the join is read first.
+        const float dLast = D[trm_index(lastRow, min(lane, lastRow - 1))];
+        const float4 lastLo = g.lo[lastRow], lastHi = g.hi[lastRow];
+        const int2 lastRh = g.rh[lastRow];
+        const int newId = group_pick(inode, lastRow - 1, kG + lastRow - 1);
         // findMinimumDistance (:81-94): strided minimum, then a 32-lane tree.
         const int msize = lastRow * (lastRow + 1) / 2;
         int mi = 0;
@@ -183,73 +242,65 @@ __global__ __launch_bounds__(kAtrBlock) void k_atr_level(AtrArgs a, const int32_
                 mi = j;
             }
         }
-        for (int s = kG / 2; s >= 1; s >>= 1) {
-            const int oi = gshfl_down(mi, s);
-            const float od = gshfl_down(md, s);
-            if (od < md) {
-                md = od;
-                mi = oi;
+        int e0, e1;
+        if (group_argmax(-md, true, e0, e1)) {
+            mi = group_pick(mi, e0, e1);
+        } else {
+            for (int s = kG / 2; s >= 1; s >>= 1) {
+                const int oi = gshfl_down(mi, s);
+                const float od = gshfl_down(md, s);
+                if (od < md) {
+                    md = od;
+                    mi = oi;
+                }
             }
+            mi = gshfl(mi, 0);
         }
-        const int minIndex = gshfl(mi, 0);
-        const int joinCol = trm_col(minIndex), joinRow = trm_row(minIndex);
+        const int join = trm_row_col(mi), joinCol = join & 0xFF, joinRow = join >> 8;
 
-        // updateState (:96-158).
-        const float ssum = gshfl(sah, joinRow) + gshfl(sah, joinCol);
-        const int leftIndex = gshfl(node, joinRow), rightIndex = gshfl(node, joinCol);
-        float3 amn = gshfl3(mn, joinRow), amx = gshfl3(mx, joinRow);
-        const float3 bmn = gshfl3(mn, joinCol), bmx = gshfl3(mx, joinCol);
-        amn = make_float3(fminf(bmn.x, amn.x), fminf(bmn.y, amn.y), fminf(bmn.z, amn.z));
-        amx = make_float3(fmaxf(bmx.x, amx.x), fmaxf(bmx.y, amx.y), fmaxf(bmx.z, amx.z));
-        const int refsNew = gshfl(refs, joinRow) + gshfl(refs, joinCol);
-        const int hNew = 1 + max(gshfl(hgt, joinRow), gshfl(hgt, joinCol));
-        const int newId = gshfl(inode, lastRow - 1);
+        // updateState (:96-158): the merged node takes row joinCol, row
+        // lastRow moves to joinRow.
+        const float4 rLo = g.lo[joinRow], rHi = g.hi[joinRow], cLo = g.lo[joinCol], cHi = g.hi[joinCol];
+        const int2 rRh = g.rh[joinRow], cRh = g.rh[joinCol];
+        const float ssum = rLo.w + cLo.w;
+        const float la = atr_area3(xyz(rLo), xyz(rHi)), ra = atr_area3(xyz(cLo), xyz(cHi));
+        const float3 amn = make_float3(fminf(cLo.x, rLo.x), fminf(cLo.y, rLo.y), fminf(cLo.z, rLo.z));
+        const float3 amx = make_float3(fmaxf(cHi.x, rHi.x), fmaxf(cHi.y, rHi.y), fmaxf(cHi.z, rHi.z));
+        const int refsNew = rRh.x + cRh.x;
+        const int hNew = 1 + max(rRh.y, cRh.y);
         const float c = ssum + a.ct * atr_area3(amn, amx);
-        if (lane == joinCol) {
-            node = newId;
-            mn = amn;
-            mx = amx;
-            sah = c;
-            refs = refsNew;
-            hgt = hNew;
-        }
-        const int lastIndex = gshfl(node, lastRow);
-        const float sahLast = gshfl(sah, lastRow);
-        const float3 lmn = gshfl3(mn, lastRow), lmx = gshfl3(mx, lastRow);
-        const int refsLast = gshfl(refs, lastRow), hLast = gshfl(hgt, lastRow);
-        if (lane == joinRow) {
-            node = lastIndex;
-            sah = sahLast;
-            mn = lmn;
-            mx = lmx;
-            refs = refsLast;
-            hgt = hLast;
-        }
         if (lane == lastRow) {
-            node = leftIndex;
-            rnode = rightIndex;
-            mn = amn;
-            mx = amx;
+            node = __float_as_int(rHi.w);
+            rnode = __float_as_int(cHi.w);
+            larea = la;
+            rarea = ra;
             mcost = c;
             mrefs = refsNew;
             mh = hNew;
         }
+        const bool isCol = lane == joinCol;
+        if (lane == joinRow) {
+            mn = xyz(lastLo);
+            mx = xyz(lastHi);
+        }
+        if (isCol || lane == lastRow) {
+            mn = amn;
+            mx = amx;
+        }
 
         if (lastRow > 1) {
-            // updateDistancesMatrix (:160-196): row lastRow moves to joinRow,
-            // then row/column joinCol is recomputed from the merged box.
-            if (lane < lastRow && lane != joinRow) {
-                const float d = D[trm_index(lastRow, lane)];
-                D[trm_index(max(joinRow, lane), min(joinRow, lane))] = d;
+            if (isCol || lane == joinRow) {
+                g.lo[lane] = isCol ? make_float4(amn.x, amn.y, amn.z, c) : lastLo;
+                g.hi[lane] = isCol ? make_float4(amx.x, amx.y, amx.z, __int_as_float(newId)) : lastHi;
+                g.rh[lane] = isCol ? make_int2(refsNew, hNew) : lastRh;
             }
+            // updateDistancesMatrix (:160-196): row lastRow moves to joinRow,
+            // then row/column joinCol is recomputed from the merged box (a
+            // union's area does not depend on the order of its two boxes).
+            if (lane < lastRow && lane != joinRow) D[trm_index(max(joinRow, lane), min(joinRow, lane))] = dLast;
             wave_lds_fence();
-            const bool upd = lane < lastRow && lane != joinCol;
-            const int dr = upd ? max(joinCol, lane) : lane;
-            const int dc = upd ? min(joinCol, lane) : lane;
-            const float3 pmn = gshfl3(mn, dr), pmx = gshfl3(mx, dr);
-            const float3 qmn = gshfl3(mn, dc), qmx = gshfl3(mx, dc);
-            const float d = atr_union_area(pmn, pmx, qmn, qmx);
-            if (upd) D[trm_index(dr, dc)] = d;
+            if (lane < lastRow && lane != joinCol)
+                D[trm_index(max(joinCol, lane), min(joinCol, lane))] = atr_union_area(mn, mx, amn, amx);
             wave_lds_fence();
         }
     }
@@ -261,6 +312,7 @@ __global__ __launch_bounds__(kAtrBlock) void k_atr_level(AtrArgs a, const int32_
         if (lane >= 1 && lane < t) {
             a.left[vid] = node;
             a.right[vid] = rnode;
+            a.children[vid] = child_record(node, rnode, larea, rarea);
             a.parent[node] = vid;
             a.parent[rnode] = vid;
             a.cost[vid] = mcost;
@@ -280,11 +332,55 @@ __global__ __launch_bounds__(kAtrBlock) void k_atr_level(AtrArgs a, const int32_
 // The cost climb step for a node that is not restructured (ATRBuilderKernels.cu
 // :293-310): every iteration recomputes it, which matters for interior nodes a
 // kept treelet gave a cost in merge order.
+HX_DEV void atr_climb_cost(const AtrArgs& a, int v) {
+    a.cost[v] = a.ct * a.area[v] + a.cost[a.left[v]] + a.cost[a.right[v]];
+}
+
+// One treelet per 32-lane group; task = index into the height bucket.
+__global__ __launch_bounds__(kAtrBlock) void k_atr_level(AtrArgs a, const int32_t* __restrict__ list, int count) {
+    __shared__ AtrGroup s_group[kGroups];
+    const int grp = threadIdx.x / kG;
+    const int task = blockIdx.x * kGroups + grp;
+    if (task >= count) return;  // whole 32-lane groups leave together
+    atr_treelet(a, list[task], threadIdx.x & (kG - 1), s_group[grp]);
+}
+
+// The remaining heights, none with more than kTopTasks nodes in a bucket, by
+// one workgroup: what a height wrote is in this CU's cache when the next one
+// reads it, and there are no launches between them.  A height takes 12 us here and 14 us
+// as a launch of its own.
+constexpr int kTopThreads = 1024;
+constexpr int kTopTasks = 64;
+__global__ __launch_bounds__(kTopThreads) void k_atr_top(AtrArgs a, int bucket, int buckets, int offset, bool costs) {
+    constexpr int G = kTopThreads / kG;
+    __shared__ AtrGroup s_group[G];
+    const int grp = threadIdx.x / kG;
+    for (int b = bucket; b < buckets; ++b) {
+        const int count = a.hist[b];
+        if (count == 0) continue;
+        const int32_t* list = a.list + offset;
+        if (b & 1) {
+            for (int k = grp; k < count; k += G) atr_treelet(a, list[k], threadIdx.x & (kG - 1), s_group[grp]);
+        } else if (costs) {
+            for (int k = threadIdx.x; k < count; k += kTopThreads) atr_climb_cost(a, list[k]);
+        }
+        offset += count;
+        __syncthreads();  // this height's nodes before the next one's reads
+    }
+}
+
+// The records of form_treelet, from the prepared hierarchy.
+__global__ __launch_bounds__(kBlock) void k_atr_children(AtrArgs a) {
+    const int v = blockIdx.x * kBlock + threadIdx.x;
+    if (v >= (int)a.n - 1) return;
+    const int l = a.left[v], r = a.right[v];
+    a.children[v] = child_record(l, r, a.area[l], a.area[r]);
+}
+
 __global__ __launch_bounds__(kBlock) void k_atr_small(AtrArgs a, const int32_t* __restrict__ list, int count) {
     const int k = blockIdx.x * kBlock + threadIdx.x;
     if (k >= count) return;
-    const int v = list[k];
-    a.cost[v] = a.ct * a.area[v] + a.cost[a.left[v]] + a.cost[a.right[v]];
+    atr_climb_cost(a, list[k]);
 }
 
 // ---- TR: optimal treelet restructuring (TRBuilderKernels.cu:11-476) ----
@@ -364,7 +460,8 @@ __global__ __launch_bounds__(kAtrBlock) void k_tr_level(AtrArgs a, const int32_t
     const float ct = a.ct, ci = a.ci;
 
     // The climb step at X (TRBuilderKernels.cu:391-407): children are final.
-    const int xl = a.left[X], xr = a.right[X];
+    const int4 root = a.children[X];
+    const int xl = root.x, xr = root.y;
     const float costX = ct * a.area[X] + a.cost[xl] + a.cost[xr];
     const int hl = xl >= n - 1 ? 0 : a.height[xl];
     const int hr = xr >= n - 1 ? 0 : a.height[xr];
@@ -372,7 +469,7 @@ __global__ __launch_bounds__(kAtrBlock) void k_tr_level(AtrArgs a, const int32_t
     const float R = (float)a.refs[X];
 
     int tl, inode;
-    form_treelet(a, X, xl, xr, kTrT, lane, tl, inode);
+    form_treelet(a, X, root, kTrT, lane, tl, inode);
     float leafCost = 0.0f;
     if (lane < kTrT) {
         const float4 bmn = a.nmin[tl], bmx = a.nmax[tl];
@@ -536,16 +633,27 @@ __global__ __launch_bounds__(kAtrBlock) void k_tr_level(AtrArgs a, const int32_t
         a.parent[l] = node;
         a.parent[r] = node;
         int refs = 0;
-        float3 mn = make_float3(kMaxFloat, kMaxFloat, kMaxFloat);
-        float3 mx = make_float3(-kMaxFloat, -kMaxFloat, -kMaxFloat);
-        for (int i = 0; i < kTrT; ++i) {
-            if (v >> i & 1) {
-                const float* b = s_box[grp][i];
-                mn = make_float3(fminf(b[0], mn.x), fminf(b[1], mn.y), fminf(b[2], mn.z));
-                mx = make_float3(fmaxf(b[3], mx.x), fmaxf(b[4], mx.y), fmaxf(b[5], mx.z));
-                refs += s_leaf[grp][1][i];
+        for (int i = 0; i < kTrT; ++i)
+            if (v >> i & 1) refs += s_leaf[grp][1][i];
+        // Box of a set of treelet leaves; a child's record area is the area
+        // that its own lane stores.
+        auto box_of = [&](int set, float3& mn, float3& mx) {
+            mn = make_float3(kMaxFloat, kMaxFloat, kMaxFloat);
+            mx = make_float3(-kMaxFloat, -kMaxFloat, -kMaxFloat);
+            for (int i = 0; i < kTrT; ++i) {
+                if (set >> i & 1) {
+                    const float* b = s_box[grp][i];
+                    mn = make_float3(fminf(b[0], mn.x), fminf(b[1], mn.y), fminf(b[2], mn.z));
+                    mx = make_float3(fmaxf(b[3], mx.x), fmaxf(b[4], mx.y), fmaxf(b[5], mx.z));
+                }
             }
-        }
+        };
+        float3 mn, mx;
+        box_of(M[v], mn, mx);
+        const float larea = atr_area3(mn, mx);
+        box_of(M[v] ^ v, mn, mx);
+        a.children[node] = child_record(l, r, larea, atr_area3(mn, mx));
+        box_of(v, mn, mx);
         a.refs[node] = refs;
         a.height[node] = rec[5][lane];
         if (lane > 0) {  // the root keeps its box and its climb cost
@@ -679,15 +787,30 @@ int launch_treelets(Context* c, const AtrArgs& a, const PlocArgs& relabel, int64
     const int64_t n = a.n;
     hipLaunchKernelGGL(k_atr_zero, dim3(1), dim3(64), 0, c->stream, a.accepted, 1);
     HX_TRY(check_launch("atr_zero"));
+    if (n > 1 && a.iterations > 0) {
+        hipLaunchKernelGGL(k_atr_children, dim3(grid_for(n - 1, kBlock)), dim3(kBlock), 0, c->stream, a);
+        HX_TRY(check_launch("atr_children"));
+    }
     std::vector<int> counts;
     int64_t gamma = a.treelet_size;
     {
         LaunchScope ls(c, tr ? "tr_optimize" : "atr_optimize");
         for (int i = 0; i < a.iterations; ++i) {
             HX_TRY(bucket_by_height(c, a, (int)std::min<int64_t>(gamma, INT32_MAX), counts));
+            int buckets = kBuckets;
+            while (buckets > 0 && counts[buckets - 1] == 0) --buckets;
+            int top = buckets;  // first bucket of k_atr_top
+            if (!tr)
+                while (top > 0 && counts[top - 1] <= kTopTasks) --top;
             int off = 0;
-            for (int b = 0; b < kBuckets; ++b) {
+            for (int b = 0; b < buckets; ++b) {
                 const int cnt = counts[b];
+                if (b == top) {
+                    hipLaunchKernelGGL(k_atr_top, dim3(1), dim3(kTopThreads), 0, c->stream, a, top, buckets, off,
+                                       i > 0);
+                    HX_TRY(check_launch("atr_top"));
+                    break;
+                }
                 if (cnt > 0 && (b & 1)) {
                     if (tr) {
                         hipLaunchKernelGGL(k_tr_level, dim3(grid_for(cnt, kGroups)), dim3(kAtrBlock), 0,

@@ -359,8 +359,6 @@ HX_DEV Combined combine(const ClimbArgs& a, int first, int last, float3 lmn, flo
     return c;
 }
 
-HX_DEV float3 xyz(float4 v) { return make_float3(v.x, v.y, v.z); }
-
 // A node that must stay an interior whatever its SAH state: the root (of each
 // mesh, in a batched build) and, in a batched build, the separator nodes
 // above the mesh roots (ranges spanning meshes), which are never emitted.

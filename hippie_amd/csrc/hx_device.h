@@ -108,6 +108,8 @@ HX_DEV int wave_sum_i32(int v) {
     return v;
 }
 
+HX_DEV float3 xyz(float4 v) { return make_float3(v.x, v.y, v.z); }
+
 // DPP move of every 32-bit word of v (GFX9 controls: row_shr:n = 0x110 + n,
 // row_bcast:15 = 0x142, row_bcast:31 = 0x143).  Lanes of rows outside
 // ROW_MASK, or whose source lies outside the pattern, keep their own value;

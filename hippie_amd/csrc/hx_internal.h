@@ -301,6 +301,7 @@ struct AtrArgs {
     int32_t* parent;
     float4* nmin;
     float4* nmax;
+    int4* children;      // n-1: left, right and the bits of their areas (filled by launch_atr / launch_tr)
     float* area;         // 2n-1
     float* cost;         // 2n-1
     int32_t* refs;       // n-1

@@ -86,3 +86,17 @@ def test_atr_trace_and_refit(oracle, ctx):
     bvh.update(hx.Scene(v2, t))
     exp_nodes = oracle.refit_final(nodes0, bvh.n_interior, bvh.n_leaves, bvh.tri_indices_host(), v2, t)
     assert np.array_equal(bvh.nodes_host(), exp_nodes), "refit nodes"
+
+
+@pytest.mark.parametrize("ts", [4, 7, 9, 17, 30])
+@pytest.mark.parametrize("n", [31, 130, 520, 2100])
+def test_atr_upper_heights(oracle, ctx, n, ts):
+    """Buckets of up to 64 nodes are restructured by one workgroup (several passes over
+    its 32 groups, odd counts included), the fuller ones below by a launch a height."""
+    v, t = scenes.gaussian_mixture_soup(n, seed=n + ts)
+    _check(oracle, ctx, v, t, ts=ts, iters=3)
+
+
+def test_atr_upper_heights_ties(oracle, ctx):
+    v, t = scenes.ground_grid(24)
+    _check(oracle, ctx, v, t, ts=9, iters=3)
