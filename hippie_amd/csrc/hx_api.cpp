@@ -265,7 +265,8 @@ size_t ploc_work_bytes(int64_t n) { return (size_t)n * (2 * 4 + 2 * 16 + 2 * 8 +
 // ATR workspace: area, cost (2n-1 floats), refs, height, list (n ints), children (n int4),
 // hist, cursor (levels + 1 ints), accepted.
 size_t atr_work_bytes(int64_t n) {
-    return (size_t)(2 * n) * 8 + (size_t)n * (12 + 16) + 2 * sizeof(int32_t) * (2 * hx::kAtrMaxLevels + 1) + 4096;
+    return (size_t)(2 * n) * 8 + (size_t)n * (12 + 16) + 2 * sizeof(int32_t) * (2 * hx::kAtrMaxLevels + 1) +
+           4 * (size_t)(hx::kAtrCounters * hx::kAtrCounterStride) + 4096;
 }
 
 // HLBVH workspace: two n-int arrays, cluster arrays of up to 2^15 entries.
@@ -651,7 +652,7 @@ int run_atr(hx_bvh* b) {
     a.list = reinterpret_cast<int32_t*>(carve(4 * (size_t)n));
     a.hist = reinterpret_cast<int32_t*>(carve(4 * (size_t)(2 * hx::kAtrMaxLevels + 1)));
     a.cursor = reinterpret_cast<int32_t*>(carve(4 * (size_t)(2 * hx::kAtrMaxLevels + 1)));
-    a.accepted = reinterpret_cast<int32_t*>(carve(16));
+    a.accepted = reinterpret_cast<int32_t*>(carve(4 * (size_t)(hx::kAtrCounters * hx::kAtrCounterStride)));
     a.children = reinterpret_cast<int4*>(carve(16 * (size_t)n));
     hx::ClimbArgs ca = climb_args(b, false);
     ca.split = nullptr;  // still a Karras tree

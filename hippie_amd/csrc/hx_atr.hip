@@ -109,6 +109,14 @@ HX_DEV bool group_argmax(float v, bool in, int& lane0, int& lane1) {
     return nan == 0 && (lo & (lo - 1)) == 0 && (hi & (hi - 1)) == 0;
 }
 
+// Counts a kept treelet.  Adds to one address are served one after another
+// (about 10 ns each), which bound the full heights: 52k treelets took 186 us with
+// one counter and take 88 us with 256 on lines of their own.
+HX_DEV void count_kept(const AtrArgs& a) {
+    const unsigned k = (blockIdx.x * blockDim.x + threadIdx.x) / kG % kAtrCounters;
+    atomicAdd(a.accepted + k * kAtrCounterStride, 1);
+}
+
 HX_DEV int4 child_record(int l, int r, float al, float ar) {
     return make_int4(l, r, __float_as_int(al), __float_as_int(ar));
 }
@@ -180,7 +188,8 @@ struct AtrGroup {
 // (9 leaves: 3.5 + 6.2 us of a 14 us level).  So a join is short: the minimum
 // by row rotations, ties alone by the reference's tree; the rows' state in LDS,
 // read as broadcasts together; no square root to the last bit.  1M triangles:
-// the 66 levels of a build 1941 us, now 34 and the two of k_atr_top 1609 us.
+// the 66 levels of a build took 1941 us; 34 of them and the two launches of
+// k_atr_top now take 1241 us (count_kept included).
 HX_DEV void atr_treelet(const AtrArgs& a, int X, int lane, AtrGroup& g) {
     const int n = (int)a.n;
     const int t = a.treelet_size;
@@ -322,7 +331,7 @@ HX_DEV void atr_treelet(const AtrArgs& a, int X, int lane, AtrGroup& g) {
             a.refs[vid] = mrefs;
             a.height[vid] = mh;
         }
-        if (lane == 0) atomicAdd(a.accepted, 1);
+        if (lane == 0) count_kept(a);
     } else if (lane == 0) {
         a.cost[X] = costX;
         a.height[X] = heightX;
@@ -665,7 +674,7 @@ __global__ __launch_bounds__(kAtrBlock) void k_tr_level(AtrArgs a, const int32_t
     }
     if (lane == 0) {
         a.cost[X] = costX;
-        if (keep) atomicAdd(a.accepted, 1);
+        if (keep) count_kept(a);
         else a.height[X] = heightX;
     }
 }
@@ -721,6 +730,16 @@ __global__ __launch_bounds__(kBlock) void k_atr_scatter(const int32_t* __restric
 #pragma unroll
     for (int k = 0; k < kItems; ++k)
         if (lvl[k] >= 0) list[s_base[lvl[k]] + loc[k]] = (int)(base + k * kBlock + threadIdx.x);
+}
+
+// Sum of the counters into the first one.
+__global__ __launch_bounds__(kAtrCounters) void k_atr_kept(int32_t* __restrict__ accepted) {
+    static_assert(kAtrCounters == 256, "four waves");
+    __shared__ int s_sum[kAtrCounters / kWave];
+    const int v = wave_sum_i32(accepted[threadIdx.x * kAtrCounterStride]);
+    if (lane_id() == 0) s_sum[threadIdx.x / kWave] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) accepted[0] = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
 }
 
 __global__ void k_atr_zero(int32_t* __restrict__ p, int count) {
@@ -785,7 +804,7 @@ namespace {
 // doubles per iteration, stopping once it exceeds the reference count.
 int launch_treelets(Context* c, const AtrArgs& a, const PlocArgs& relabel, int64_t* accepted_out, bool tr) {
     const int64_t n = a.n;
-    hipLaunchKernelGGL(k_atr_zero, dim3(1), dim3(64), 0, c->stream, a.accepted, 1);
+    hipLaunchKernelGGL(k_atr_zero, dim3(8), dim3(kBlock), 0, c->stream, a.accepted, kAtrCounters * kAtrCounterStride);
     HX_TRY(check_launch("atr_zero"));
     if (n > 1 && a.iterations > 0) {
         hipLaunchKernelGGL(k_atr_children, dim3(grid_for(n - 1, kBlock)), dim3(kBlock), 0, c->stream, a);
@@ -835,6 +854,8 @@ int launch_treelets(Context* c, const AtrArgs& a, const PlocArgs& relabel, int64
     }
     HX_TRY(launch_relabel_by_height(c, a, relabel));
     if (accepted_out) {
+        hipLaunchKernelGGL(k_atr_kept, dim3(1), dim3(kAtrCounters), 0, c->stream, a.accepted);
+        HX_TRY(check_launch("atr_kept"));
         int32_t acc = 0;
         HX_HIP(hipMemcpyAsync(&acc, a.accepted, sizeof(acc), hipMemcpyDeviceToHost, c->stream));
         HX_HIP(hipStreamSynchronize(c->stream));

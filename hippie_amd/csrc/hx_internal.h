@@ -309,9 +309,10 @@ struct AtrArgs {
     int32_t* list;       // n-1: internal nodes grouped by height
     int32_t* hist;       // bucket counts / cursors (2 * kAtrMaxLevels + 1 each)
     int32_t* cursor;
-    int32_t* accepted;   // 1: treelets whose restructuring was kept
+    int32_t* accepted;   // kAtrCounters partial counts of the kept treelets, kAtrCounterStride words apart
 };
 constexpr int kAtrMaxLevels = 1024;
+constexpr int kAtrCounters = 256, kAtrCounterStride = 32;
 // relabel: fields of a PLOC argument block used by launch_tree_down.
 int launch_atr(Context* c, const AtrArgs& a, const PlocArgs& relabel, int64_t* accepted_out);
 // TR (TRBuilder.cpp:140-191): the same level driver with the optimal 7-leaf
