@@ -13,7 +13,8 @@
 //                      wins (strict '>' over a left-to-right scan);
 //   k_ploc_tile_counts merges (mutual pair, lower index) and survivors
 //                      (everything but the higher index of a mutual pair) per
-//                      1024-cluster tile;
+//                      512-cluster tile; k_ploc_pairs does both in one
+//                      launch for small radii;
 //   k_ploc_scan        (rounds of more than kDirectTiles tiles) exclusive scan
 //                      of the tile counts, totals for the host;
 //   k_ploc_merge       new node = (m-2) - (merge rank in cluster order): the
@@ -43,12 +44,14 @@ constexpr int kBlock = 256;
 // thread with a block scan each left 244 workgroups of 4 waves for 1,000,003
 // clusters; one workgroup of 16 waves per 1024 clusters and ballots instead of
 // scans took a round's counts, scan and merge from 43 to 10 us (mean of the 48
-// rounds there).
-constexpr int kTile = 1024;
+// rounds there).  512 for the sake of k_ploc_pairs, whose small rounds then
+// spread over more CUs (2310 us with 1024, 2160 with 512, 2175 with 256 for the whole
+// build at r = 25; the other radii and 200,003 clusters likewise).
+constexpr int kTile = 512;
 constexpr int kTileWaves = kTile / kWave;
 // Up to this many tiles a merge workgroup adds up the counts before its own
-// (at most 32 KB from L2); above it one workgroup scans them first.
-constexpr int kDirectTiles = 4096;
+// (at most 64 KB from L2); above it one workgroup scans them first.
+constexpr int kDirectTiles = 8192;
 constexpr int kPlocBatch = 16;  // rounds launched between host reads
 constexpr int kMaxLdsRadius = 1024;   // window of 256 + 2r boxes, 6 floats each, in LDS
 
@@ -169,6 +172,36 @@ HX_DEV bool ploc_pair_round(int m, const int32_t* cmesh, int n_meshes, int i, in
     return true;
 }
 
+// Place of the cluster nearest to the one at place `me` among the r places on
+// either side (the lowest on ties), -1 without one; sa, sb: boxes, sm: meshes.
+template <bool MESH>
+HX_DEV int scan_window(const float4* sa, const float2* sb, const int32_t* sm, int me, int r) {
+    const Box3 own = cluster_box(sa[me], sb[me]);
+    const float3 lo = make_float3(vmin(own.mn.x, own.mx.x), vmin(own.mn.y, own.mx.y), vmin(own.mn.z, own.mx.z));
+    const float3 hi = make_float3(vmax(own.mn.x, own.mx.x), vmax(own.mn.y, own.mx.y), vmax(own.mn.z, own.mx.z));
+    const int mine = MESH ? sm[me] : 0;
+    int best = -1;
+    float bestD = kHalfMax;
+    auto step = [&](int q) {
+        const float d = half_union_area(sa[q], sb[q], lo, hi);
+        const bool better = bestD > d && (!MESH || sm[q] == mine);
+        bestD = better ? d : bestD;
+        best = better ? q : best;
+    };
+    auto scan = [&](int q, int q1) {
+        for (; q + 4 <= q1; q += 4) {
+            step(q);
+            step(q + 1);
+            step(q + 2);
+            step(q + 3);
+        }
+        for (; q < q1; ++q) step(q);
+    };
+    scan(me - r, me);
+    scan(me + 1, me + r + 1);
+    return best;
+}
+
 // The window [b0 - r, b0 + kBlock + r) of a workgroup's clusters in LDS, places
 // outside [0, m) filled with far boxes, so that every lane scans the same 2r
 // places with no bounds tests.  VALU bound: 17 instructions and two LDS reads
@@ -199,30 +232,7 @@ __global__ __launch_bounds__(kBlock) void k_ploc_neighbours(const float4* __rest
     }
     __syncthreads();
     if (i >= m) return;
-    const int me = threadIdx.x + r;
-    const Box3 own = cluster_box(sa[me], sb[me]);
-    const float3 lo = make_float3(vmin(own.mn.x, own.mx.x), vmin(own.mn.y, own.mx.y), vmin(own.mn.z, own.mx.z));
-    const float3 hi = make_float3(vmax(own.mn.x, own.mx.x), vmax(own.mn.y, own.mx.y), vmax(own.mn.z, own.mx.z));
-    const int mine = MESH ? sm[me] : 0;
-    int best = -1;
-    float bestD = kHalfMax;
-    auto step = [&](int q) {
-        const float d = half_union_area(sa[q], sb[q], lo, hi);
-        const bool better = bestD > d && (!MESH || sm[q] == mine);
-        bestD = better ? d : bestD;
-        best = better ? q : best;
-    };
-    auto scan = [&](int q, int q1) {
-        for (; q + 4 <= q1; q += 4) {
-            step(q);
-            step(q + 1);
-            step(q + 2);
-            step(q + 3);
-        }
-        for (; q < q1; ++q) step(q);
-    };
-    scan(me - r, me);
-    scan(me + 1, me + r + 1);
+    const int best = scan_window<MESH>(sa, sb, sm, threadIdx.x + r, r);
     nb[i] = best < 0 ? -1 : best + b0 - r;
 }
 
@@ -256,6 +266,67 @@ HX_DEV void tile_ballots(int2 f, uint64_t& bm, uint64_t& bs, int2* ws) {
     __syncthreads();
 }
 
+// The sum of the waves' counts of tile_ballots, by one thread.
+HX_DEV int2 tile_sum(const int2* ws) {
+    int2 s = ws[0];
+    for (int w = 1; w < kTileWaves; ++w) s = make_int2(s.x + ws[w].x, s.y + ws[w].y);
+    return s;
+}
+
+// Neighbours and tile counts in one launch.  The kTile threads find the
+// neighbours of the tile's kTile - 2r clusters and of the r clusters on either
+// side, so that the tile's mutual pairs are known from LDS alone.  Most rounds
+// are too small to take longer than a launch, and this saves one of three;
+// the work grows by kTile / (kTile - 2r), so larger radii and rounds keep two
+// kernels.  Builds of 1,000,003 triangles, two kernels and one: r = 8 1725 and
+// 1624 us, r = 25 2290 and 2165, r = 48 2745 and 2675, r = 64 3033 and 3021;
+// 16.7M triangles at r = 25 18.50 and 18.64 ms.
+constexpr int kFusedRadius = 48;
+constexpr int kFusedClusters = 1 << 22;
+template <bool MESH>
+__global__ __launch_bounds__(kTile) void k_ploc_pairs(const float4* __restrict__ ca, const float2* __restrict__ cb,
+                                                      const int4* __restrict__ round, int r,
+                                                      int32_t* __restrict__ nb, const int32_t* __restrict__ cmesh,
+                                                      int n_meshes, int2* __restrict__ partial) {
+    extern __shared__ float4 s_win[];
+    __shared__ int s_nb[kTile];
+    __shared__ int2 ws[kTileWaves];
+    const int W = kTile + 2 * r;
+    float4* sa = s_win;
+    float2* sb = reinterpret_cast<float2*>(sa + W);
+    int32_t* sm = reinterpret_cast<int32_t*>(sb + W);
+    const int m = round->x;
+    const int b0 = blockIdx.x * (kTile - 2 * r);
+    if (m <= 1 || b0 >= m) return;
+    const int t = threadIdx.x;
+    const int i = b0 - r + t;  // this thread's cluster, if 0 <= i < m
+    int j = -1;
+    if (MESH && m <= n_meshes) {
+        if (i >= 0 && i < m && (i ^ 1) < m) j = i ^ 1;  // ploc_pair_round
+    } else {
+        for (int k = t; k < W; k += kTile) {
+            const int q = b0 - 2 * r + k;
+            const bool in = q >= 0 && q < m;
+            sa[k] = in ? ca[q] : far_box_a();
+            sb[k] = in ? cb[q] : far_box_b();
+            if (MESH) sm[k] = in ? cmesh[q] : -1;
+        }
+        __syncthreads();
+        if (i >= 0 && i < m) {
+            const int best = scan_window<MESH>(sa, sb, sm, t + r, r);
+            j = best < 0 ? -1 : best + b0 - 2 * r;
+        }
+    }
+    s_nb[t] = j;
+    __syncthreads();
+    const bool own = t >= r && t < kTile - r && i < m;
+    const bool mutual = own && j >= 0 && s_nb[j - (b0 - r)] == i;
+    if (own) nb[i] = j;
+    uint64_t bm, bs;
+    tile_ballots(make_int2(mutual && i < j ? 1 : 0, own && !(mutual && i > j) ? 1 : 0), bm, bs, ws);
+    if (t == 0) partial[blockIdx.x] = tile_sum(ws);
+}
+
 __global__ __launch_bounds__(kTile) void k_ploc_tile_counts(const int32_t* __restrict__ nb,
                                                             const int4* __restrict__ round,
                                                             int2* __restrict__ partial) {
@@ -265,11 +336,7 @@ __global__ __launch_bounds__(kTile) void k_ploc_tile_counts(const int32_t* __res
     if (m <= 1 || base >= m) return;
     uint64_t bm, bs;
     tile_ballots(ploc_flags(nb, m, base + threadIdx.x), bm, bs, ws);
-    if (threadIdx.x == 0) {
-        int2 s = ws[0];
-        for (int w = 1; w < kTileWaves; ++w) s = make_int2(s.x + ws[w].x, s.y + ws[w].y);
-        partial[blockIdx.x] = s;
-    }
+    if (threadIdx.x == 0) partial[blockIdx.x] = tile_sum(ws);
 }
 
 // The round's totals (merged, surviving) to its record, whose cluster count
@@ -284,14 +351,15 @@ HX_DEV void close_round(int4* round, int2 tot) {
 // Single block: exclusive scan of the tile counts in place; the round's
 // (merged, surviving) totals go to its record and the survivors become the
 // next round's cluster count.
-__global__ __launch_bounds__(kTile) void k_ploc_scan(int2* __restrict__ partial, int4* __restrict__ round) {
+__global__ __launch_bounds__(kTile) void k_ploc_scan(int2* __restrict__ partial, int4* __restrict__ round,
+                                                     int tile_size) {
     __shared__ int2 wt[kTileWaves];
     const int m = round->x;
     if (m <= 1) {
         if (threadIdx.x == 0) close_round(round, make_int2(0, m));
         return;
     }
-    const int ntiles = (m + kTile - 1) / kTile;
+    const int ntiles = (m + tile_size - 1) / tile_size;
     int2 carry = make_int2(0, 0);
     for (int base = 0; base < ntiles; base += kTile) {
         const int t = base + threadIdx.x;
@@ -348,20 +416,20 @@ HX_DEV void merge_cluster(const PlocArgs& a, int src, int i, int2 f, int mrank, 
 // of a zero); its subtree size goes to last[node] for the relabelling.
 // SCANNED: partial holds exclusive prefixes (k_ploc_scan); else the counts, which
 // the workgroup adds up itself, and the workgroup of the last tile closes the
-// round.
+// round.  tile_size: clusters of a tile, as the counts were taken.
 template <bool SCANNED>
 __global__ __launch_bounds__(kTile) void k_ploc_merge(PlocArgs a, int src, int4* __restrict__ round,
-                                                      const int2* __restrict__ partial) {
+                                                      const int2* __restrict__ partial, int tile_size) {
     __shared__ int2 ws[kTileWaves], pre[kTileWaves];
     const int m = round->x;
     const int tile = blockIdx.x;
-    const int64_t base = tile * (int64_t)kTile;
+    const int64_t base = tile * (int64_t)tile_size;
     if (m <= 1) {
         if (!SCANNED && tile == 0 && threadIdx.x == 0) close_round(round, make_int2(0, m));
         return;
     }
     if (base >= m) return;
-    const int64_t i = base + threadIdx.x;
+    const int64_t i = (int)threadIdx.x < tile_size ? base + threadIdx.x : m;
     const int2 f = ploc_flags(a.nb, m, i);
     const int w = threadIdx.x / kWave;
     int2 carry = make_int2(0, 0);
@@ -384,7 +452,7 @@ __global__ __launch_bounds__(kTile) void k_ploc_merge(PlocArgs a, int src, int4*
     }
     if (i < m)
         merge_cluster(a, src, (int)i, f, carry.x + below.x + count_below(bm), carry.y + below.y + count_below(bs), m - 2);
-    if (!SCANNED && base + kTile >= m && threadIdx.x == 0)
+    if (!SCANNED && base + tile_size >= m && threadIdx.x == 0)
         close_round(round, make_int2(carry.x + tot.x, carry.y + tot.y));
 }
 
@@ -629,7 +697,8 @@ int launch_ploc(Context* c, const PlocArgs& a, int* rounds_out) {
         hipLaunchKernelGGL(k_ploc_leaves, dim3(grid_for(n)), dim3(kBlock), 0, c->stream, a);
         HX_TRY(check_launch("ploc_leaves"));
     }
-    const int64_t max_tiles = (n + kTile - 1) / kTile;
+    constexpr int kMinTile = kTile - 2 * kFusedRadius;
+    const int64_t max_tiles = (n + kMinTile - 1) / kMinTile;
     HX_TRY(c->scan_partials.reserve(sizeof(int2) * (size_t)max_tiles + sizeof(int4) * (kPlocBatch + kTailClusters + 2) +
                                     64));
     int2* partial = c->scan_partials.as<int2>();
@@ -673,31 +742,43 @@ int launch_ploc(Context* c, const PlocArgs& a, int* rounds_out) {
             }
             break;
         }
-        const int ntiles = (m + kTile - 1) / kTile;
         for (int b = 0; b < kPlocBatch; ++b) {
             if (a.adaptive) r = std::min(r + 1, a.max_radius);
+            const int32_t* cmesh = batched ? a.cm[src] : nullptr;
+            const bool fused = r <= kFusedRadius && m <= kFusedClusters;
+            const int tile_size = fused ? kTile - 2 * r : kTile;
+            const int ntiles = (m + tile_size - 1) / tile_size;
             {
                 LaunchScope ls(c, "ploc_neighbours");
-                const size_t lds = sizeof(float) * (batched ? 7 : 6) * (size_t)(kBlock + 2 * r);
-                const int32_t* cmesh = batched ? a.cm[src] : nullptr;
-                auto kernel = r > kMaxLdsRadius ? k_ploc_neighbours_far
-                                                : batched ? k_ploc_neighbours<true> : k_ploc_neighbours<false>;
-                hipLaunchKernelGGL(kernel, dim3(grid_for(m)), dim3(kBlock), r > kMaxLdsRadius ? 0 : lds, c->stream,
-                                   a.ca[src], a.cb[src], rounds + b, r, a.nb, cmesh, a.n_meshes);
-                HX_TRY(check_launch("ploc_neighbours"));
+                const size_t lds = sizeof(float) * (batched ? 7 : 6) * (size_t)((fused ? kTile : kBlock) + 2 * r);
+                if (fused) {
+                    hipLaunchKernelGGL((batched ? k_ploc_pairs<true> : k_ploc_pairs<false>), dim3(ntiles), dim3(kTile),
+                                       lds, c->stream, a.ca[src], a.cb[src], rounds + b, r, a.nb, cmesh, a.n_meshes,
+                                       partial);
+                    HX_TRY(check_launch("ploc_pairs"));
+                } else {
+                    auto kernel = r > kMaxLdsRadius ? k_ploc_neighbours_far
+                                                    : batched ? k_ploc_neighbours<true> : k_ploc_neighbours<false>;
+                    hipLaunchKernelGGL(kernel, dim3(grid_for(m)), dim3(kBlock), r > kMaxLdsRadius ? 0 : lds, c->stream,
+                                       a.ca[src], a.cb[src], rounds + b, r, a.nb, cmesh, a.n_meshes);
+                    HX_TRY(check_launch("ploc_neighbours"));
+                }
             }
             {
                 LaunchScope ls(c, "ploc_merge");
-                hipLaunchKernelGGL(k_ploc_tile_counts, dim3(ntiles), dim3(kTile), 0, c->stream, a.nb, rounds + b,
-                                   partial);
-                HX_TRY(check_launch("ploc_tile_counts"));
+                if (!fused) {
+                    hipLaunchKernelGGL(k_ploc_tile_counts, dim3(ntiles), dim3(kTile), 0, c->stream, a.nb, rounds + b,
+                                       partial);
+                    HX_TRY(check_launch("ploc_tile_counts"));
+                }
                 const bool direct = ntiles <= kDirectTiles;
                 if (!direct) {
-                    hipLaunchKernelGGL(k_ploc_scan, dim3(1), dim3(kTile), 0, c->stream, partial, rounds + b);
+                    hipLaunchKernelGGL(k_ploc_scan, dim3(1), dim3(kTile), 0, c->stream, partial, rounds + b,
+                                       tile_size);
                     HX_TRY(check_launch("ploc_scan"));
                 }
                 hipLaunchKernelGGL((direct ? k_ploc_merge<false> : k_ploc_merge<true>), dim3(ntiles), dim3(kTile), 0,
-                                   c->stream, a, src, rounds + b, partial);
+                                   c->stream, a, src, rounds + b, partial, tile_size);
                 HX_TRY(check_launch("ploc_merge"));
             }
             src ^= 1;

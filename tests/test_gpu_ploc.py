@@ -120,3 +120,18 @@ def test_ploc_rebuild_reuses_handle(oracle, ctx):
 def test_ploc_tile_and_window_edges(oracle, ctx, n, radius):
     v, t = scenes.merge(scenes.uniform_soup(n - n // 2, seed=n), scenes.gaussian_mixture_soup(n // 2, seed=radius))
     _check(oracle, ctx, v, t, radius, max_radius=2048)
+
+
+# Radii up to 48 find neighbours and count pairs in one launch over tiles of 512 - 2r
+# clusters; from 49 on they take two.  Sizes around whole tiles above the tail.
+@pytest.mark.parametrize("n", [2049, 2080, 2081, 2310, 2311, 5101])
+@pytest.mark.parametrize("radius", [1, 25, 48, 49])
+def test_ploc_pair_tiles(oracle, ctx, n, radius):
+    v, t = scenes.merge(scenes.uniform_soup(n - n // 2, seed=n), scenes.gaussian_mixture_soup(n // 2, seed=radius))
+    _check(oracle, ctx, v, t, radius)
+
+
+def test_ploc_pair_tiles_grow(oracle, ctx):
+    """An adaptive radius crosses from one form to the other between two rounds."""
+    v, t = scenes.uniform_soup(20000, seed=5)
+    _check(oracle, ctx, v, t, 44, ploc_adaptive=True, max_radius=60)
