@@ -153,12 +153,13 @@ int hx_context_profile_reset(hx_context* ctx);
  *   "trace_lds_stack"      traversal-stack entries held in LDS (0,16,24,32,64)
  *   "trace_fetch"          refill a wave when fewer of its 64 lanes are busy
  *   "trace_blocks_per_cu"  persistent trace workgroups per CU (0 = occupancy)
- *   "trace_postpone"       leaves a lane holds back while its wave traverses (1 to 4; Bin layout,
- *                          closest hit; any-hit traces keep 1)
+ *   "trace_postpone"       leaves a lane holds back while its wave traverses (1 to 4; Bin layout;
+ *                          any-hit rays test theirs oldest first, so their hits stay the same)
  *   "trace_woop_ahead"     Woop rows of a leaf's next triangle read while the current one is
  *                          tested (1 or 2; Bin layout)
  *   "sort_digit_bits"      radix digit width of every sort (8 or 10)
- *   "sort_items"           keys per thread in a sort pass (8, 16 or 32)
+ *   "sort_items"           keys per thread in a sort pass (8, 16 or 32; 8 while the tiles do not
+ *                          fill the chip twice)
  *   "sort_lookback"        tiles read per sort look-back round trip (4, 8, 16)
  *   "sort_local_run"       the builds' Morton sorts and hx_sort_pairs_u64 of
  *                          > 40-bit keys with at least 2^18 keys run four
