@@ -45,18 +45,22 @@ HX_DEV float span_end(float a0, float a1, float b0, float b1, float c0, float c1
 // finish together: a fixed run of 1/2 of a wave's share cost 15 % on 16.7M
 // diffuse rays, runs of 1024 rays cost 10 % on sorted primaries (3.51 against
 // 3.19 ms) since the waves of a CU then work far apart.
-constexpr int kRunMax = 256;
+// Batched rays keep to runs of 64: the rays in flight belong to few meshes then,
+// whose trees the caches hold (67.1M rays into 512 meshes 280 -> 226 ms, 241 with
+// a refill at a time; with 1M atomics in that time the counter does not bound it).
+constexpr int kRunMax = 256, kRunMaxBatch = 64;
 struct RayPool {
     int next, end;   // this wave's rays
     int base;        // first ray of the latest run: the rays left start about here
     int dyn0;        // first ray that is handed out by the counter
-    int n, lanes, shift;
+    int n, lanes, shift, most;
 
-    HX_DEV int run() const { return max(lanes, min((n - base) >> shift, kRunMax)); }
+    HX_DEV int run() const { return max(lanes, min((n - base) >> shift, most)); }
     HX_DEV void start(const TraceArgs& a) {
         n = (int)a.n_rays;
         lanes = a.lanes;
         shift = a.run_shift;
+        most = a.ray_mesh ? kRunMaxBatch : kRunMax;
         base = 0;
         const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kTraceBlock / kWave) + threadIdx.x / kWave);
         const int r = run();
