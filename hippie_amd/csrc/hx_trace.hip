@@ -169,7 +169,9 @@ HX_DEV void share_adopt(uint64_t key, float& t, int32_t& id, bool always = false
 // Nodes are always read by vector loads.  Scalar loads when a whole wave visits
 // one node paid for themselves only while the ray counter set the pace; with
 // RayPool they cost 1,048,576 primaries 3 % and 16,384 rays 10 % (the check and
-// the scalar cache's latency) and gave sorted primaries nothing.
+// the scalar cache's latency).  Large coherent sets miss them: 16.7M sorted
+// primaries over 16.7M triangles 4.64 -> 6.2 ms, the diffuse rays of that scene
+// 10.95 -> 9.88 ms.
 template <bool STATS, bool ORDERED, int LDS_DEPTH, int POSTPONE, int AHEAD, bool SHARE>
 HX_TRACE_KERNEL __attribute__((amdgpu_waves_per_eu(LDS_DEPTH <= 16 ? 8 : 1))) void k_trace(TraceArgs a) {
     __shared__ int32_t s_stack[LDS_DEPTH > 0 ? LDS_DEPTH * kTraceBlock : 1];
