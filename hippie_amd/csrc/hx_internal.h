@@ -575,7 +575,7 @@ struct TraceArgs {
     const int32_t* tri_idx;
     int2* stats;            // optional
     const int32_t* order;   // optional: ray slot -> ray index (sorted trace)
-    int32_t* control;       // [0] ray counter, [1] overflow counter
+    int32_t* control;       // [0] ray counter, [1] overflow counter, [2] rays from one point
     int fetch_threshold;    // dynamic fetch: busy lanes below which a wave refills
     int lanes;              // rays per wave, and the run length's divisor (set by the launch)
     int run_shift;

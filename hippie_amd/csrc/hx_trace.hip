@@ -43,27 +43,36 @@ HX_DEV float span_end(float a0, float a1, float b0, float b1, float c0, float c1
 // and 1,000,000 diffuse rays from 900 to 704 us.  Runs shrink with the rays left
 // (1 / (4 x waves) of them, at least one ray per lane) so that the last waves
 // finish together: a fixed run of 1/2 of a wave's share cost 15 % on 16.7M
-// diffuse rays, runs of 1024 rays cost 10 % on sorted primaries (3.51 against
-// 3.19 ms) since the waves of a CU then work far apart.
+// diffuse rays.
 // Batched rays keep to runs of 64: the rays in flight belong to few meshes then,
 // whose trees the caches hold (67.1M rays into 512 meshes 280 -> 226 ms, 241 with
 // a refill at a time; with 1M atomics in that time the counter does not bound it).
+//
+// Rays from one point (`alike`, see alike_pays) are handed out a refill at a time.
+// Neighbours among them cost alike, so a wave that stays on its own run in a
+// costly place carries several groups of long-lived rays, each at another depth;
+// when all waves take the next rays in turn it carries one such group among short
+// ones.  16.7M sorted primaries over as many triangles: 2.93 -> 2.57 G VALU and
+// 170 -> 124 M vector-load instructions.
+constexpr int kControlAlike = 2;   // word of TraceArgs::control
 constexpr int kRunMax = 256, kRunMaxBatch = 64;
 struct RayPool {
     int next, end;   // this wave's rays
     int base;        // first ray of the latest run: the rays left start about here
     int dyn0;        // first ray that is handed out by the counter
     int n, lanes, shift, most;
+    bool alike;
 
     HX_DEV int run() const { return max(lanes, min((n - base) >> shift, most)); }
-    HX_DEV void start(const TraceArgs& a) {
+    HX_DEV void start(const TraceArgs& a, bool one_point) {
         n = (int)a.n_rays;
         lanes = a.lanes;
         shift = a.run_shift;
         most = a.ray_mesh ? kRunMaxBatch : kRunMax;
         base = 0;
+        alike = one_point;
         const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kTraceBlock / kWave) + threadIdx.x / kWave);
-        const int r = run();
+        const int r = alike ? lanes : run();
         next = wave * r;
         end = min(next + r, n);
         dyn0 = base = (int)gridDim.x * (kTraceBlock / kWave) * r;
@@ -76,7 +85,7 @@ struct RayPool {
         int mine = next + below;
         if (count > avail) {
             int first = n;
-            const int r = run();
+            const int r = alike ? count : run();
             if (base < n) {
                 if (want && below == 0) first = atomicAdd(counter, r);
                 first = dyn0 + __builtin_amdgcn_readlane(first, __ffsll((unsigned long long)mask) - 1);
@@ -106,6 +115,9 @@ struct RayPool {
 // LDS and private accesses apart: through a generic pointer it merges the two
 // into one flat load, which waits on both memory counters.
 typedef __attribute__((address_space(3))) int32_t lds_i32;
+// Read by scalar loads where the address is the same in every lane.
+typedef const __attribute__((address_space(4))) float const_f32;
+typedef const __attribute__((address_space(4))) int32_t const_i32;
 
 template <int LDS_DEPTH, int SIZE = kStackSize>
 struct TraversalStack {
@@ -166,13 +178,13 @@ HX_DEV void share_adopt(uint64_t key, float& t, int32_t& id, bool always = false
 // which is traversal order, so that the hit they report is the same however
 // many are held.
 //
-// Nodes are always read by vector loads.  Scalar loads when a whole wave visits
-// one node paid for themselves only while the ray counter set the pace; with
-// RayPool they cost 1,048,576 primaries 3 % and 16,384 rays 10 % (the check and
-// the scalar cache's latency).  Large coherent sets miss them: 16.7M sorted
-// primaries over 16.7M triangles 4.64 -> 6.2 ms, the diffuse rays of that scene
-// 10.95 -> 9.88 ms.
-template <bool STATS, bool ORDERED, int LDS_DEPTH, int POSTPONE, int AHEAD, bool SHARE>
+// A node is read by vector loads, which cost the CU's texture address and data
+// units four 16-byte-per-lane instructions however many lanes share it.  With
+// rays from one point (ALIKE) a node that all active lanes of the wave visit is
+// read by scalar loads instead (constant address space: the trace never writes
+// the nodes).  For other rays the check costs more than the reads it saves (16,384
+// rays 10 %).
+template <bool STATS, bool ORDERED, int LDS_DEPTH, int POSTPONE, int AHEAD, bool SHARE, bool ALIKE>
 HX_TRACE_KERNEL __attribute__((amdgpu_waves_per_eu(LDS_DEPTH <= 16 ? 8 : 1))) void k_trace(TraceArgs a) {
     __shared__ int32_t s_stack[LDS_DEPTH > 0 ? LDS_DEPTH * kTraceBlock : 1];
     __shared__ ShareSlot s_share[SHARE ? kTraceBlock : 1];
@@ -190,8 +202,9 @@ HX_TRACE_KERNEL __attribute__((amdgpu_waves_per_eu(LDS_DEPTH <= 16 ? 8 : 1))) vo
     int32_t nodeBase = 0, triBase = 0;
     const int lane = lane_id();
     if (!SHARE && lane >= a.lanes) return;
+    const bool alike = ALIKE && __builtin_amdgcn_readfirstlane(a.control[kControlAlike]) != 0;
     RayPool pool;
-    pool.start(a);
+    pool.start(a, alike);
     // SHARE, once the rays are handed out: lane whose ray this lane works on,
     // its slot, and this lane's lowest stack entry that may be given away.
     ShareSlot* const wave_slots = s_share + (SHARE ? threadIdx.x - lane : 0);
@@ -299,10 +312,6 @@ HX_TRACE_KERNEL __attribute__((amdgpu_waves_per_eu(LDS_DEPTH <= 16 ? 8 : 1))) vo
                 copy(idx); copy(idy); copy(idz);
                 copy(oodx); copy(oody); copy(oodz);
                 copy(hitT); copy(hitId); copy(share);
-                if (a.ray_mesh) {
-                    copy(nodeBase);
-                    copy(triBase);
-                }
                 if (takes) {
                     nodeAddr = got;
                     leafAddr = leafAddr2 = leafAddr3 = leafAddr4 = 0;
@@ -326,17 +335,9 @@ HX_TRACE_KERNEL __attribute__((amdgpu_waves_per_eu(LDS_DEPTH <= 16 ? 8 : 1))) vo
                 if (STATS) ++nNodes;
                 float c0min, c0max, c1min, c1max;
                 int2 cn;
-                {
-                    const int64_t na = (uint32_t)(nodeBase + nodeAddr);
-                    const float4* np = reinterpret_cast<const float4*>(a.nodes + 4 * na);
-                    const float4 n0xy = np[0];
-                    const float4 n1xy = np[1];
-                    const float4 nz = np[2];
-                    const int4 links = a.nodes[4 * na + 3];
-                    // The child links share the node's cache line: keep their
-                    // load with the box loads instead of after the box test.
-                    asm volatile("" ::"v"(links.x), "v"(links.y));
-                    cn = make_int2(links.x, links.y);
+                // Written out in both branches below, so that a node of the whole
+                // wave is tested straight from the scalar registers.
+                auto box_test = [&](float4 n0xy, float4 n1xy, float4 nz) {
                     const float c0lox = fmaf(n0xy.x, idx, -oodx);
                     const float c0hix = fmaf(n0xy.y, idx, -oodx);
                     const float c0loy = fmaf(n0xy.z, idy, -oody);
@@ -353,6 +354,26 @@ HX_TRACE_KERNEL __attribute__((amdgpu_waves_per_eu(LDS_DEPTH <= 16 ? 8 : 1))) vo
                     const float c1hiy = fmaf(n1xy.w, idy, -oody);
                     c1min = span_begin(c1lox, c1hix, c1loy, c1hiy, c1loz, c1hiz, tmin);
                     c1max = span_end(c1lox, c1hix, c1loy, c1hiy, c1loz, c1hiz, hitT);
+                };
+                const uint32_t na = (uint32_t)(nodeBase + nodeAddr);
+                const uint32_t n0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)na);
+                if (alike && __all(na == n0)) {
+                    const_f32* f = (const_f32*)(a.nodes + 4 * (int64_t)n0);
+                    const_i32* w = (const_i32*)(a.nodes + 4 * (int64_t)n0);
+                    box_test(make_float4(f[0], f[1], f[2], f[3]), make_float4(f[4], f[5], f[6], f[7]),
+                             make_float4(f[8], f[9], f[10], f[11]));
+                    cn = make_int2(w[12], w[13]);
+                } else {
+                    const float4* np = reinterpret_cast<const float4*>(a.nodes + 4 * (int64_t)na);
+                    const float4 n0xy = np[0];
+                    const float4 n1xy = np[1];
+                    const float4 nz = np[2];
+                    const int4 links = a.nodes[4 * (int64_t)na + 3];
+                    // The child links share the node's cache line: keep their
+                    // load with the box loads instead of after the box test.
+                    asm volatile("" ::"v"(links.x), "v"(links.y));
+                    cn = make_int2(links.x, links.y);
+                    box_test(n0xy, n1xy, nz);
                 }
                 const bool swp = c1min < c0min;
                 const bool t0 = c0max >= c0min;
@@ -525,7 +546,7 @@ struct WideStackSize {
     static constexpr int kSize = N == 4 ? 96 : 160;
 };
 
-template <int N, bool STATS, bool ORDERED, int LDS_DEPTH>
+template <int N, bool STATS, bool ORDERED, int LDS_DEPTH, bool ALIKE>
 HX_TRACE_KERNEL void k_trace_wide(TraceArgs a) {
     constexpr int kSize = WideStackSize<N>::kSize;
     __shared__ int32_t s_stack[LDS_DEPTH > 0 ? LDS_DEPTH * kTraceBlock : 1];
@@ -540,8 +561,9 @@ HX_TRACE_KERNEL void k_trace_wide(TraceArgs a) {
     int32_t nNodes = 0, nTris = 0;
     const float4* nodes4 = reinterpret_cast<const float4*>(a.nodes);
     if (lane_id() >= a.lanes) return;
+    const bool alike = ALIKE && __builtin_amdgcn_readfirstlane(a.control[kControlAlike]) != 0;
     RayPool pool;
-    pool.start(a);
+    pool.start(a, alike);
 
     while (true) {
         const bool terminated = nodeAddr == kSentinel;
@@ -576,6 +598,7 @@ HX_TRACE_KERNEL void k_trace_wide(TraceArgs a) {
                 if (STATS) ++nNodes;
                 float dist[N];
                 int32_t link[N];
+                // Child c's test; written out in both node-read branches, as in k_trace.
                 auto child_test = [&](int c, float4 xy, float4 zl) {
                     const float lox = fmaf(xy.x, idx, -oodx);
                     const float hix = fmaf(xy.y, idx, -oodx);
@@ -589,15 +612,25 @@ HX_TRACE_KERNEL void k_trace_wide(TraceArgs a) {
                     dist[c] = hit ? cmin : __int_as_float(0x7f800000);
                     link[c] = hit ? __float_as_int(zl.z) : kSentinel;
                 };
-                const float4* np = nodes4 + (int64_t)nodeAddr * 2 * N;
-                float4 xys[N], zls[N];
+                const int32_t n0 = __builtin_amdgcn_readfirstlane(nodeAddr);
+                if (alike && __all(nodeAddr == n0)) {
+                    const_f32* f = (const_f32*)(nodes4 + (int64_t)n0 * 2 * N);
 #pragma unroll
-                for (int c = 0; c < N; ++c) {
-                    xys[c] = np[c];
-                    zls[c] = np[N + c];
+                    for (int c = 0; c < N; ++c)
+                        child_test(c, make_float4(f[4 * c], f[4 * c + 1], f[4 * c + 2], f[4 * c + 3]),
+                                   make_float4(f[4 * (N + c)], f[4 * (N + c) + 1], f[4 * (N + c) + 2],
+                                               f[4 * (N + c) + 3]));
+                } else {
+                    const float4* np = nodes4 + (int64_t)nodeAddr * 2 * N;
+                    float4 xys[N], zls[N];
+#pragma unroll
+                    for (int c = 0; c < N; ++c) {
+                        xys[c] = np[c];
+                        zls[c] = np[N + c];
+                    }
+#pragma unroll
+                    for (int c = 0; c < N; ++c) child_test(c, xys[c], zls[c]);
                 }
-#pragma unroll
-                for (int c = 0; c < N; ++c) child_test(c, xys[c], zls[c]);
 #pragma unroll
                 for (int q = 0; q < WideNet<N>::kPairs; ++q) {
                     const int2 pr = WideNet<N>::pair(q);
@@ -786,6 +819,57 @@ __global__ void k_zero_control(int32_t* control) {
     if (threadIdx.x < 2) control[threadIdx.x] = 0;
 }
 
+// k_zero_control of a launch that may hold rays from one point: kAlikeWindows
+// windows of 64 neighbouring rays, spread evenly over the set as it is traced.
+// control[kControlAlike] is set if in more than half of them every ray is live (a
+// dead one, with an empty interval, ends at once whatever its origin: the secondary
+// rays of misses) and starts at the same point.
+constexpr int kAlikeBlock = 1024, kAlikeWindows = 64;
+__global__ __launch_bounds__(kAlikeBlock) void k_zero_control_alike(TraceArgs a) {
+    __shared__ int s_alike[kAlikeBlock / kWave];
+    const int w = threadIdx.x / kWave;
+    int count = 0;
+    for (int k = w; k < kAlikeWindows; k += kAlikeBlock / kWave) {
+        const int64_t slot = (a.n_rays - kWave) * k / (kAlikeWindows - 1) + lane_id();
+        const int64_t ray = a.order ? a.order[slot] : slot;
+        const float4 o = a.rays[2 * ray], d = a.rays[2 * ray + 1];
+        auto first = [](float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); };
+        count += __all(o.x == first(o.x) && o.y == first(o.y) && o.z == first(o.z) && d.w > o.w) ? 1 : 0;
+    }
+    if (lane_id() == 0) s_alike[w] = count;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int k = 1; k < kAlikeBlock / kWave; ++k) count += s_alike[k];
+    a.control[0] = a.control[1] = 0;
+    a.control[kControlAlike] = 2 * count > kAlikeWindows ? 1 : 0;
+}
+
+// Large sets are looked over for rays from one point (k_zero_control_alike; RayPool
+// and k_trace say what they get): from 4 rays a
+// lane slot on (2.1M rays; the wide kernels and sorted sets), 12 in input order
+// (6.3M).  Below, and where half of the rays miss at the root, the one ray counter
+// would set the pace: unsorted 1,048,576 rays over 65,536 triangles 359 -> 370 us,
+// a step with 4.2M camera rays over 1.3M triangles 1.76 -> 1.81 ms.  Primaries of the Gaussian
+// mixture and ground grid, refill by refill with scalar reads against runs with
+// vector reads: 16.7M sorted rays over 16.7M / 1M / 65k triangles 6.39 -> 4.82,
+// 7.79 -> 6.46, 4.15 -> 3.49 ms (Quad, 16.7M and 65k: 6.79 -> 4.98, 4.51 -> 3.48;
+// Oct: 9.14 -> 7.01, 5.30 -> 4.30), 4.2M sorted 2.04 -> 1.53, 2.38 -> 2.02,
+// 1.27 -> 1.04 ms, 16.7M in input order 6.24 -> 5.15, 7.78 -> 7.02, 4.14 -> 3.52 ms.
+// Of the 1.6 ms at 16.7M triangles the hand-out gives 0.7 ms, the scalar reads 0.9.
+// The diffuse rays of these scenes take what they took (9.83, 10.4, 3.75 ms).  The
+// counts of a stats trace keep to one kernel.
+bool alike_pays(const Context* c, const TraceArgs& a, bool wide) {
+    return !a.stats && a.n_rays >= (int64_t)c->cu_count * 8 * kTraceBlock * (a.order || wide ? 4 : 12);
+}
+
+int zero_control(Context* c, const TraceArgs& a, bool wide) {
+    if (alike_pays(c, a, wide))
+        hipLaunchKernelGGL(k_zero_control_alike, dim3(1), dim3(kAlikeBlock), 0, c->stream, a);
+    else
+        hipLaunchKernelGGL(k_zero_control, dim3(1), dim3(64), 0, c->stream, a.control);
+    return check_launch("zero_control");
+}
+
 // Rays per wave, workgroups and run lengths of a launch.  A wave costs the same
 // whether 16 or 64 of its lanes carry rays, and lanes that diverge wait for each
 // other, so a launch that cannot fill the chip with full waves spreads its rays
@@ -813,28 +897,35 @@ unsigned trace_shape(Context* c, int occ, bool share, TraceArgs& a) {
 
 // Sharing pays where the longest rays show: up to 16 rays a lane slot.  Above
 // (16.7M rays and more) the tail is too short a part of the launch (sorted
-// primaries 3.19 -> 3.23 ms).  Batched rays lose by it (1.37M: 1131 -> 1187 us or
+// primaries over a Gaussian mixture of 16.7M triangles 3.19 -> 3.23 ms).  Batched rays lose by it (1.37M: 1131 -> 1187 us or
 // more): they are short and hit early.  An any-hit trace reports the first hit of
 // one lane's traversal order, and the counts of a stats trace are per ray.
 bool share_pays(const Context* c, const TraceArgs& a) {
     return !a.any_hit && !a.stats && !a.ray_mesh && a.n_rays <= (int64_t)c->cu_count * 8 * kTraceBlock * 16;
 }
 
-template <bool STATS, bool ORDERED, int LDS_DEPTH, int POSTPONE, int AHEAD, bool SHARE>
-int launch_trace_t(Context* c, const TraceArgs& a) {
+template <bool STATS, bool ORDERED, int LDS_DEPTH, int POSTPONE, int AHEAD, bool SHARE, bool ALIKE>
+int launch_trace_kernel(Context* c, const TraceArgs& a) {
     // Occupancy limit of this instantiation, queried once per process.
     static int occ = 0;
     if (occ == 0) {
         int q = 0;
-        HX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&q, k_trace<STATS, ORDERED, LDS_DEPTH, POSTPONE, AHEAD, SHARE>,
+        HX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&q, k_trace<STATS, ORDERED, LDS_DEPTH, POSTPONE, AHEAD, SHARE, ALIKE>,
                                                              kTraceBlock, 0));
         occ = std::max(q, 1);
     }
     TraceArgs t = a;
     const unsigned blocks = trace_shape(c, occ, SHARE, t);
-    hipLaunchKernelGGL((k_trace<STATS, ORDERED, LDS_DEPTH, POSTPONE, AHEAD, SHARE>), dim3(blocks), dim3(kTraceBlock), 0,
+    hipLaunchKernelGGL((k_trace<STATS, ORDERED, LDS_DEPTH, POSTPONE, AHEAD, SHARE, ALIKE>), dim3(blocks), dim3(kTraceBlock), 0,
                        c->stream, t);
     return check_launch("trace");
+}
+
+template <bool STATS, bool ORDERED, int LDS_DEPTH, int POSTPONE, int AHEAD, bool SHARE>
+int launch_trace_t(Context* c, const TraceArgs& a) {
+    if (!STATS && alike_pays(c, a, false))
+        return launch_trace_kernel<false, ORDERED, LDS_DEPTH, POSTPONE, AHEAD, SHARE, true>(c, a);
+    return launch_trace_kernel<STATS, ORDERED, LDS_DEPTH, POSTPONE, AHEAD, SHARE, false>(c, a);
 }
 
 template <bool STATS, bool ORDERED, int POSTPONE, int AHEAD>
@@ -869,19 +960,25 @@ int launch_trace_postpone(Context* c, const TraceArgs& a) {
     }
 }
 
-template <int N, bool STATS, bool ORDERED, int LDS_DEPTH>
-int launch_trace_wide_t(Context* c, const TraceArgs& a) {
+template <int N, bool STATS, bool ORDERED, int LDS_DEPTH, bool ALIKE>
+int launch_trace_wide_kernel(Context* c, const TraceArgs& a) {
     static int occ = 0;
     if (occ == 0) {
         int q = 0;
-        HX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&q, k_trace_wide<N, STATS, ORDERED, LDS_DEPTH>, kTraceBlock,
+        HX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&q, k_trace_wide<N, STATS, ORDERED, LDS_DEPTH, ALIKE>, kTraceBlock,
                                                              0));
         occ = std::max(q, 1);
     }
     TraceArgs t = a;
     const unsigned blocks = trace_shape(c, occ, false, t);
-    hipLaunchKernelGGL((k_trace_wide<N, STATS, ORDERED, LDS_DEPTH>), dim3(blocks), dim3(kTraceBlock), 0, c->stream, t);
+    hipLaunchKernelGGL((k_trace_wide<N, STATS, ORDERED, LDS_DEPTH, ALIKE>), dim3(blocks), dim3(kTraceBlock), 0, c->stream, t);
     return check_launch("trace_wide");
+}
+
+template <int N, bool STATS, bool ORDERED, int LDS_DEPTH>
+int launch_trace_wide_t(Context* c, const TraceArgs& a) {
+    if (!STATS && alike_pays(c, a, true)) return launch_trace_wide_kernel<N, false, ORDERED, LDS_DEPTH, true>(c, a);
+    return launch_trace_wide_kernel<N, STATS, ORDERED, LDS_DEPTH, false>(c, a);
 }
 
 template <int N, bool STATS, bool ORDERED>
@@ -906,8 +1003,7 @@ int launch_trace_wide_n(Context* c, const TraceArgs& a) {
 
 int launch_trace_wide(Context* c, int N, const TraceArgs& a) {
     if (a.n_rays <= 0) return HX_OK;
-    hipLaunchKernelGGL(k_zero_control, dim3(1), dim3(64), 0, c->stream, a.control);
-    HX_TRY(check_launch("zero_control"));
+    HX_TRY(zero_control(c, a, true));
     LaunchScope ls(c, a.order ? "trace_wide_sorted" : "trace_wide");
     if (N == 4) return launch_trace_wide_n<4>(c, a);
     if (N == 8) return launch_trace_wide_n<8>(c, a);
@@ -917,8 +1013,7 @@ int launch_trace_wide(Context* c, int N, const TraceArgs& a) {
 
 int launch_trace(Context* c, const TraceArgs& a) {
     if (a.n_rays <= 0) return HX_OK;
-    hipLaunchKernelGGL(k_zero_control, dim3(1), dim3(64), 0, c->stream, a.control);
-    HX_TRY(check_launch("zero_control"));
+    HX_TRY(zero_control(c, a, false));
     LaunchScope ls(c, a.order ? "trace_sorted" : "trace");
     if (a.stats)
         return a.order ? launch_trace_postpone<true, true>(c, a) : launch_trace_postpone<true, false>(c, a);

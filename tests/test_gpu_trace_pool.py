@@ -5,6 +5,7 @@ traversal order.  Hits are compared bit for bit with the one-lane CPU oracle.
 """
 import numpy as np
 import pytest
+import torch
 
 import hippie_amd as hx
 from hippie_amd import scenes
@@ -111,3 +112,40 @@ def test_shared_rays_deep_tree(oracle, ctx, sort):
     assert ov == 0 and ctx.overflow_count() == 0
     hit = ref[:, 0] >= 0
     assert np.array_equal(res[:, :2], ref[:, :2]) and np.array_equal(res[hit], ref[hit])
+
+
+def _point_rays(n, seed, kind):
+    """Rays from one point; "half": the second half from anywhere; "dead": every
+    second ray's interval is empty; "nan": one ray in 5000 has no origin."""
+    r = scenes.random_rays(n, seed=seed)
+    k = n // 2 + 1 if kind == "half" else n
+    r[:k, 0:3] = (0.5, 0.5, -0.8)
+    if kind == "dead":
+        r[::2, 7] = -1.0
+    if kind == "nan":
+        r[::5000, 0] = np.nan
+    return r
+
+
+# Sets from 4 rays a lane slot on (sorted ones and the wide layouts; 12 in input
+# order) are looked over for rays from one point, which are handed out refill by
+# refill and read nodes by scalar loads: sizes around both, and sets that are only
+# partly alike.
+@pytest.mark.parametrize("layout", ["bin", "quad", "oct"])
+@pytest.mark.parametrize("sort", [False, True])
+@pytest.mark.parametrize("kind, extra", [("point", -1), ("point", 0), ("point", 77), ("half", 1), ("dead", 1), ("nan", 1)])
+def test_rays_from_one_point(oracle, ctx, layout, sort, kind, extra):
+    slots = torch.cuda.get_device_properties(0).multi_processor_count * 8 * 256
+    n = slots * (4 if sort or layout != "bin" else 12) + extra
+    v, t = scenes.uniform_soup(700, seed=41)
+    bvh = hx.LBVHBuilder(ctx, morton_bits=60, layout=layout).build(hx.Scene(v, t))
+    rays = _point_rays(n, 42, kind)
+    rb = hx.RayBuffer(rays)
+    rb.results.fill_(0x7F7F7F7F)
+    tr = hx.HipTracer(ctx, bvh)
+    res = (tr.trace_sort(rb) if sort else tr.trace(rb)).cpu().numpy()
+    b = hx.LBVHBuilder(ctx, morton_bits=60).build(hx.Scene(v, t))
+    ref, _ = oracle.trace(b.nodes_host(), b.woop_host(), b.tri_indices_host(), rays)
+    assert np.array_equal(res[:, :2], ref[:, :2])
+    hit = ref[:, 0] >= 0
+    assert hit.any() and np.array_equal(res[hit], ref[hit])
