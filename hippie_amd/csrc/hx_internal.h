@@ -464,9 +464,6 @@ struct SortWorkspace {
     uint32_t* status;
     int64_t status_words;
 };
-// Status words a sort of n keys over [0, end_bit) needs with the context's
-// digit width and keys per thread (no split sort).
-int sort_status_words_max(const Context* c, int64_t n, int end_bit);
 // Stable LSD sort of (key, value) over bits [0, end_bit).  keys/vals ping-pong
 // between [0] and [1]; returns in *result_index which buffer holds the output.
 // vals_identity: the input values are 0..n-1 and are not read.  allow_split:

@@ -577,11 +577,10 @@ __global__ void k_sort_copy_gated(const uint64_t* __restrict__ ks, const int32_t
 }
 
 // Status words (look-back flags, digit histograms, tile counters) of an LSD
-// sort of n keys over `bits` key bits.
-template <int RB, int IT>
-int64_t sort_status_words(int64_t n, int bits) {
-    const int passes = sort_passes(bits, RB);
-    return (int64_t)passes * sort_tiles(n, IT) * (1 << RB) + (int64_t)passes * (1 << RB) + kMaxPasses;
+// sort of n keys over `bits` key bits, rb bits a pass, `items` keys per thread.
+int64_t sort_status_words(int rb, int items, int64_t n, int bits) {
+    const int passes = sort_passes(bits, rb);
+    return (int64_t)passes * sort_tiles(n, items) * (1 << rb) + (int64_t)passes * (1 << rb) + kMaxPasses;
 }
 
 // LSD passes over key bits [lo_bit, end_bit) from buffers 0; *result = the
@@ -668,7 +667,7 @@ template <int RB, int IT, int LB>
 int sort_split(Context* c, void* keys[2], int32_t* vals[2], int64_t n, int lo_bit, int end_bit, bool vals_identity,
                int* result) {
     // Every buffer the gated passes touch is reserved before anything runs.
-    const int64_t words = std::max(sort_status_words<RB, IT>(n, end_bit), sort_status_words<RB, IT>(n, end_bit - lo_bit));
+    const int64_t words = std::max(sort_status_words(RB, IT, n, end_bit), sort_status_words(RB, IT, n, end_bit - lo_bit));
     HX_TRY(c->sort_status.reserve(sizeof(uint32_t) * (size_t)words));
     HX_TRY(c->sort_flag.reserve(64));
     int32_t* flag = c->sort_flag.as<int32_t>();
@@ -703,9 +702,14 @@ int sort_split(Context* c, void* keys[2], int32_t* vals[2], int64_t n, int lo_bi
 // give every CU two tiles.  A tile's latency grows with its keys per thread and
 // nothing else fills the chip there: 65,536 60-bit keys 119 -> 91 us, 262,143
 // 136 -> 117 us; above, the fewer and longer digit runs win (1,048,576: 151
-// against 158 us, 16.7M: 869 against 1044 us).
-int sort_items_for(const Context* c, int64_t n) {
-    return n < (int64_t)c->cu_count * 2 * kSortBlock * 8 ? std::min(c->tune.sort_items, 8) : c->tune.sort_items;
+// against 158 us, 16.7M: 869 against 1044 us).  Twice the tiles need twice the
+// status words: a workspace of the caller that does not hold them (10-bit digits,
+// from 600,000 keys on in hx_trace_sorted_noalloc) gets the tunable's.
+int sort_items_for(const Context* c, int64_t n, int end_bit, const SortWorkspace* ws) {
+    const int items = n < (int64_t)c->cu_count * 2 * kSortBlock * 8 ? std::min(c->tune.sort_items, 8) : c->tune.sort_items;
+    if (ws != nullptr && sort_status_words(c->tune.sort_digit_bits, items, n, end_bit) > ws->status_words)
+        return c->tune.sort_items;
+    return items;
 }
 
 }  // namespace
@@ -717,19 +721,13 @@ int sort_pass_count(const Context* c, int end_bit, int64_t n, bool keys64) {
     return sort_passes(end_bit, bits);
 }
 
-int sort_status_words_max(const Context* c, int64_t n, int end_bit) {
-    const int rb = c->tune.sort_digit_bits, it = sort_items_for(c, n);
-    const int passes = sort_passes(end_bit, rb);
-    return (int)((int64_t)passes * sort_tiles(n, it) * (1 << rb) + (int64_t)passes * (1 << rb) + kMaxPasses);
-}
-
 int launch_sort_pairs(Context* c, void* keys[2], int32_t* vals[2], int64_t n, int end_bit, bool keys64,
                       bool vals_identity, int* result_index, bool allow_split, const SortWorkspace* ws) {
     if (n >= (int64_t)1 << 30) {
         set_error("radix sort: n = %lld exceeds 2^30 - 1", (long long)n);
         return HX_ERR_INVALID_ARG;
     }
-    const int bits = c->tune.sort_digit_bits, items = sort_items_for(c, n), lb = c->tune.sort_lookback;
+    const int bits = c->tune.sort_digit_bits, items = sort_items_for(c, n, end_bit, ws), lb = c->tune.sort_lookback;
     // Long keys, many of them: four digit passes over the high bits leave runs
     // of equal high bits that are short for Morton codes (at most 19 keys for
     // the 16.7M-triangle benchmark scene at 32 high bits), which one pass

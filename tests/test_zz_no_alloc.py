@@ -75,3 +75,20 @@ def test_noalloc_rejects_more_rays_than_its_scratch():
     with pytest.raises(_lib.HxError, match="exceed"):
         _sorted_trace("hx_trace_sorted_noalloc", ctx, bvh, rays, "aila", 60, res, order)
     assert int((res[:, 0] != -7).sum()) == 0   # nothing ran
+
+
+@pytest.mark.parametrize("n", [600_000, 700_001, 900_000, MAX_RAYS - 1, MAX_RAYS])
+@pytest.mark.parametrize("bits", [48, 60, 64])
+def test_noalloc_wide_digits(n, bits):
+    """10-bit digits need the most sort status words: every size up to the maximum fits
+    the fixed scratch, below the line where a sort takes 8 keys per thread as well."""
+    ctx = hx.Context(0)
+    ctx.set_tuning("sort_digit_bits", 10)
+    v, t = scenes.uniform_soup(4096, seed=3)
+    bvh = hx.LBVHBuilder(ctx, morton_bits=30).build(hx.Scene(v, t))
+    rays = torch.as_tensor(scenes.random_rays(n, seed=4), device="cuda")
+    got, want = _buffers(n), _buffers(n)
+    _sorted_trace("hx_trace_sorted_noalloc", ctx, bvh, rays, "aila", bits, *got)
+    _sorted_trace("hx_trace_sorted", ctx, bvh, rays, "aila", bits, *want)
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
