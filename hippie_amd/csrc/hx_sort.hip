@@ -583,6 +583,32 @@ int64_t sort_status_words(int rb, int items, int64_t n, int bits) {
     return (int64_t)passes * sort_tiles(n, items) * (1 << rb) + (int64_t)passes * (1 << rb) + kMaxPasses;
 }
 
+// Keys per thread of a digit pass: the tunable, but at most 8 while 16 would not
+// give every CU two tiles.  A tile's latency grows with its keys per thread and
+// nothing else fills the chip there: 65,536 60-bit keys 119 -> 91 us, 262,143
+// 136 -> 117 us; above, the fewer and longer digit runs win (1,048,576: 151
+// against 158 us, 16.7M: 869 against 1044 us).  Twice the tiles need twice the
+// status words: a workspace of the caller that does not hold them (10-bit digits,
+// from 600,000 keys on in hx_trace_sorted_noalloc) gets the tunable's.
+inline int64_t sort_few_keys(const Context* c) { return (int64_t)c->cu_count * 2 * kSortBlock * 8; }
+int sort_items_for(const Context* c, int64_t n, int end_bit, const SortWorkspace* ws) {
+    const int items = n < sort_few_keys(c) ? std::min(c->tune.sort_items, 8) : c->tune.sort_items;
+    if (ws != nullptr && sort_status_words(c->tune.sort_digit_bits, items, n, end_bit) > ws->status_words)
+        return c->tune.sort_items;
+    return items;
+}
+
+// The context's status words for a sort of n keys with `items` each: also what
+// any sort of fewer keys needs, which may have more tiles, so that a smaller sort
+// never grows (and so frees) a buffer that a captured graph refers to.
+int reserve_status(Context* c, int items, int64_t n, int bits) {
+    const int rb = c->tune.sort_digit_bits;
+    int64_t words = sort_status_words(rb, items, n, bits);
+    if (n >= sort_few_keys(c))
+        words = std::max(words, sort_status_words(rb, std::min(items, 8), sort_few_keys(c) - 1, bits));
+    return c->sort_status.reserve(sizeof(uint32_t) * (size_t)words);
+}
+
 // LSD passes over key bits [lo_bit, end_bit) from buffers 0; *result = the
 // buffer index holding the output.  With a gate every launch is enqueued and
 // does its work only if *gate is set (status must then be reserved already).
@@ -615,7 +641,7 @@ int sort_impl(Context* c, void* keys[2], int32_t* vals[2], int64_t n, int lo_bit
             set_error("radix sort: gated passes need their status words reserved in advance");
             return HX_ERR_INVALID_ARG;
         }
-        HX_TRY(c->sort_status.reserve(sizeof(uint32_t) * (size_t)words));
+        HX_TRY(reserve_status(c, IT, n, end_bit - lo_bit));
         status = c->sort_status.as<uint32_t>();
     }
     uint32_t* hist = status + status_words;
@@ -667,8 +693,7 @@ template <int RB, int IT, int LB>
 int sort_split(Context* c, void* keys[2], int32_t* vals[2], int64_t n, int lo_bit, int end_bit, bool vals_identity,
                int* result) {
     // Every buffer the gated passes touch is reserved before anything runs.
-    const int64_t words = std::max(sort_status_words(RB, IT, n, end_bit), sort_status_words(RB, IT, n, end_bit - lo_bit));
-    HX_TRY(c->sort_status.reserve(sizeof(uint32_t) * (size_t)words));
+    HX_TRY(reserve_status(c, IT, n, end_bit));
     HX_TRY(c->sort_flag.reserve(64));
     int32_t* flag = c->sort_flag.as<int32_t>();
     int hi_res = 0;
@@ -696,20 +721,6 @@ int sort_split(Context* c, void* keys[2], int32_t* vals[2], int64_t n, int lo_bi
     }
     *result = hi_res ^ 1;
     return HX_OK;
-}
-
-// Keys per thread of a digit pass: the tunable, but at most 8 while 16 would not
-// give every CU two tiles.  A tile's latency grows with its keys per thread and
-// nothing else fills the chip there: 65,536 60-bit keys 119 -> 91 us, 262,143
-// 136 -> 117 us; above, the fewer and longer digit runs win (1,048,576: 151
-// against 158 us, 16.7M: 869 against 1044 us).  Twice the tiles need twice the
-// status words: a workspace of the caller that does not hold them (10-bit digits,
-// from 600,000 keys on in hx_trace_sorted_noalloc) gets the tunable's.
-int sort_items_for(const Context* c, int64_t n, int end_bit, const SortWorkspace* ws) {
-    const int items = n < (int64_t)c->cu_count * 2 * kSortBlock * 8 ? std::min(c->tune.sort_items, 8) : c->tune.sort_items;
-    if (ws != nullptr && sort_status_words(c->tune.sort_digit_bits, items, n, end_bit) > ws->status_words)
-        return c->tune.sort_items;
-    return items;
 }
 
 }  // namespace

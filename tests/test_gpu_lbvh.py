@@ -446,3 +446,37 @@ def test_lbvh_merge_level_edges(oracle, ctx, n, adaptive):
     a = oracle.bin_canonical(bvh.nodes_host(), bvh.n_interior, bvh.n_leaves, bvh.tri_indices_host())
     b = oracle.bin_canonical(ref["nodes"], ref["n_interior"], ref["n_leaves"], ref["tri_idx"])
     assert np.array_equal(a, b)
+
+
+# Sorts of fewer keys than two 4096-key tiles a CU take smaller tiles and may need
+# more status words than a larger sort: those are reserved with the larger one's.
+@pytest.mark.parametrize("digits", [8, 10])
+def test_smaller_sort_keeps_the_status_buffer(digits):
+    c = hx.Context(0)
+    c.set_tuning("sort_digit_bits", digits)
+    line = torch.cuda.get_device_properties(0).multi_processor_count * 4096
+    rng = np.random.default_rng(digits)
+    src = [torch.from_numpy(rng.integers(0, 1 << 62, n, dtype=np.int64)).cuda() for n in (line, line - 1)]
+    keys = [k.clone() for k in src]
+    vals = [torch.arange(k.numel(), dtype=torch.int32, device="cuda") for k in src]
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    c.set_stream(s)
+    try:
+        with torch.cuda.stream(s):
+            hx.sort_pairs(c, keys[0], vals[0], 62)
+            s.synchronize()
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=s):
+                hx.sort_pairs(c, keys[1], vals[1], 62)
+    finally:
+        c.set_stream(torch.cuda.current_stream())
+    order = torch.argsort(src[1], stable=True)
+    for _ in range(3):
+        keys[1].copy_(src[1])
+        vals[1].copy_(torch.arange(src[1].numel(), dtype=torch.int32, device="cuda"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(keys[1].cpu().numpy(), src[1][order].cpu().numpy())
+        assert np.array_equal(vals[1].cpu().numpy(), order.int().cpu().numpy())
