@@ -142,7 +142,6 @@ struct hx_bvh {
     // clustering workspace (cluster ids, boxes and neighbours, ping-pong).
     DevBuf split, ploc_work, atr_work, hlbvh_work, ins_work;
     DevBuf node_at;  // general trees: internal node at each split position
-    DevBuf link;     // LBVH builds: arrival words of the climb's top level
     DevBuf proto;    // LBVH builds: Bin rows 0-2 of each internal node from the climb
     DevBuf leaf_stats;  // hx_bvh_leaf_stats: size counts and their sum
     int ploc_rounds = 0;
@@ -323,7 +322,6 @@ int reserve_bvh(hx_bvh* b, int64_t n) {
         HX_TRY(b->tri_local.reserve(4 * (size_t)n));
     }
     if (b->params.method == HX_METHOD_LBVH) {
-        HX_TRY(b->link.reserve(8 * (size_t)n));
         HX_TRY(b->proto.reserve(48 * (size_t)n));
     }
     if (b->params.method == HX_METHOD_PLOC) {
@@ -392,7 +390,6 @@ hx::ClimbArgs lbvh_climb_args(hx_bvh* b, const void* keys, bool keys64) {
     hx::ClimbArgs ca = climb_args(b, false);
     ca.keys = keys;
     ca.keys64 = keys64 ? 1 : 0;
-    ca.link = b->link.as<uint64_t>();
     ca.root_id = b->counts.as<int32_t>() + 3;
     ca.all_boxes = b->params.keep_debug || b->params.layout != HX_LAYOUT_BIN ? 1 : 0;
     ca.proto = b->proto.as<float4>();

@@ -869,15 +869,11 @@ __global__ __launch_bounds__(kLbvhThreads) __attribute__((amdgpu_num_sgpr(80))) 
         store_box(n - 1 + base + i, T + i);
     }
     // Internal nodes of the block's split range: the finished ones written
-    // out coalesced; the others are completed by the merges (or by k_lbvh_top,
-    // whose arrival words start cleared).
+    // out coalesced; the others are completed by the merges.
     for (int i = threadIdx.x; i < T; i += kLbvhThreads) {
         const int node = base + i;
         if (node >= n - 1) break;
-        if (s_cnt[i] != 2) {
-            a.link[node] = 0;
-            continue;
-        }
+        if (s_cnt[i] != 2) continue;
         const int first = base + s_first[i], last = base + s_last[i];
         a.first[node] = first;
         a.last[node] = last;
@@ -900,91 +896,6 @@ __global__ __launch_bounds__(kLbvhThreads) __attribute__((amdgpu_num_sgpr(80))) 
     }
 }
 
-// Each arrival at a parent ORs one 64-bit word: presence (bit 63), its node
-// id (bits 31-61) and its far range end (bits 0-30: first of the parent if
-// it is the left child, last if the right), so the second arrival learns
-// the sibling and the parent's range from the atomic's result.  A node's box
-// travels in registers up the chain and through nmin/nmax (sc1 stores that
-// complete before the arrival) to the sibling.
-// Only lists that do not fit the merges' LDS come here (k_lbvh_merge's last
-// workgroup), so a key order in which hundreds of nodes straddle a block still
-// builds; the chains are bound by the ~3 us of a level's round trips.
-template <bool K64>
-HX_DEV void lbvh_top(const ClimbArgs& a, const int32_t* list, int count) {
-    const int n = (int)a.n;
-    for (int e = threadIdx.x; e < count; e += blockDim.x) {
-        int node = list[e];
-        int l, r;
-        if (node >= n - 1) {
-            l = r = node - (n - 1);
-        } else {
-            l = a.first[node];
-            r = a.last[node];
-        }
-        int dl = l == 0 ? -1 : kdelta<K64>(l - 1, l, n, a.keys, a.mesh_of, a.mesh_off);
-        int dr = r == n - 1 ? -1 : kdelta<K64>(r, r + 1, n, a.keys, a.mesh_of, a.mesh_off);
-        float3 mn = xyz(a.nmin[node]), mx = xyz(a.nmax[node]);
-        float cost = a.adaptive ? a.cost[node] : 0.0f;
-        while (true) {
-            if (l == 0 && r == n - 1) {
-                a.parent[node] = -1;
-                *a.root_id = node;
-                break;
-            }
-            const bool as_left = dr > dl;
-            const int sp = as_left ? r : l - 1;
-            complete_stores();
-            const uint64_t mine = (1ull << 63) | ((uint64_t)(uint32_t)node << 31) | (uint32_t)(as_left ? l : r);
-            const uint64_t old = __hip_atomic_fetch_or(&a.link[sp], mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            a.parent[node] = sp;
-            if (as_left) {
-                a.left[sp] = node;
-                a.first[sp] = l;
-            } else {
-                a.right[sp] = node;
-                a.last[sp] = r;
-            }
-            if (old == 0) break;
-            const int sib = (int)((old >> 31) & 0x7fffffffu);
-            const int far = (int)(old & 0x7fffffffu);
-            const float4 smn = ld_agent(a.nmin + sib), smx = ld_agent(a.nmax + sib);
-            const float scost = a.adaptive ? ld_agent(a.cost + sib) : 0.0f;
-            Combined c;
-            if (as_left) {
-                r = far;
-                dr = r == n - 1 ? -1 : kdelta<K64>(r, r + 1, n, a.keys, a.mesh_of, a.mesh_off);
-                c = combine(a, l, r, mn, mx, cost, xyz(smn), xyz(smx), scost);
-            } else {
-                l = far;
-                dl = l == 0 ? -1 : kdelta<K64>(l - 1, l, n, a.keys, a.mesh_of, a.mesh_off);
-                c = combine(a, l, r, xyz(smn), xyz(smx), scost, mn, mx, cost);
-            }
-            st_agent(a.nmin + sp, make_float4(c.mn.x, c.mn.y, c.mn.z, 0.0f));
-            st_agent(a.nmax + sp, make_float4(c.mx.x, c.mx.y, c.mx.z, 0.0f));
-            if (a.adaptive) st_agent(a.cost + sp, c.cost);
-            a.state[sp] = c.state;
-            const bool top = seg_top(a.mesh_of, a.mesh_off, n, l, r);
-            if (c.state == 0 && !top) atomicMax(&a.end_at[l], r);
-            if (c.state == 1 || top) {
-                const float4 omn = make_float4(mn.x, mn.y, mn.z, 0.0f), omx = make_float4(mx.x, mx.y, mx.z, 0.0f);
-                int4 r0, r1, r2;
-                if (as_left)
-                    bin_rows(omn, omx, smn, smx, r0, r1, r2);
-                else
-                    bin_rows(smn, smx, omn, omx, r0, r1, r2);
-                int4* pr = reinterpret_cast<int4*>(a.proto + 3 * (int64_t)sp);
-                pr[0] = r0;
-                pr[1] = r1;
-                pr[2] = r2;
-            }
-            mn = c.mn;
-            mx = c.mx;
-            cost = c.cost;
-            node = sp;
-        }
-    }
-}
-
 // One workgroup merges `lists` consecutive frontier lists of `stride` slots each
 // (list k at a.frontier + k * stride, its length in_count[k]): entry e of their
 // concatenation is a node, entries are consecutive leaf ranges, and a node over
@@ -994,13 +905,21 @@ HX_DEV void lbvh_top(const ClimbArgs& a, const int32_t* list, int count) {
 // against ~3 us for the round trips between XCDs of a climb on global memory
 // (arrival words by device atomics, boxes by sc1 stores and loads), which bound
 // the whole top: 4,099 triangles 29 -> 13 us, 65,536 56 -> 34 us, 16.7M 320 ->
-// 257 us (what is left there is the latency of cold scattered reads).  The frontier that is left goes to the workgroup's
-// first list slot and out_count.  LAST: one workgroup holds every list and
-// finishes the tree.  More entries than kMergeCap (a block has ~8, but a skewed
-// key order can have hundreds) are passed on unmerged; LAST climbs them on
-// global memory.
+// 257 us (what is left there is the latency of cold scattered reads).  The frontier
+// that is left goes to the workgroup's first list slot and out_count.  LAST: one
+// workgroup holds every list and finishes the tree.
+// More entries than kMergeCap (a block leaves ~8, a skewed key order hundreds) are
+// merged in runs of kMergeCap until they fit.  A run's frontier is a row of nodes
+// whose boundaries' common prefixes strictly fall and then strictly rise, so it
+// holds at most twice as many nodes as there are prefix lengths (32 mesh bits, 64
+// key bits, 32 index bits: 2 x 129) and every pass shrinks the entries to less
+// than half; no workgroup leaves more than 258.  1.5M triangles of which ~50 nodes
+// straddle each block: the climb takes 0.68 ms (64 ms when such entries were passed
+// on for one last workgroup to climb, 0.28 ms for a climb on global memory by the
+// whole chip), 8.4M with ~45: 1.26 ms (3.4, 1.07).
 constexpr int kMergeThreads = 256;
 constexpr int kMergeCap = 640;
+static_assert(kMergeCap >= 2 * 258, "a full run shrinks to less than half");
 
 template <bool K64, bool LAST>
 __global__ __launch_bounds__(kMergeThreads) void k_lbvh_merge(ClimbArgs a, const int32_t* __restrict__ in_count,
@@ -1029,8 +948,10 @@ __global__ __launch_bounds__(kMergeThreads) void k_lbvh_merge(ClimbArgs a, const
         if (tid == 0) s_off[0] = 0;
     }
     __syncthreads();
-    const int E = s_off[l1 - l0];
+    int total = s_off[l1 - l0];
+    bool joined = false;         // the entries lie behind each other at `out`
     auto source = [&](int e) {   // entry e's place in a.frontier
+        if (joined) return out + e;
         int lo = 0, hi = l1 - l0 - 1;
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
@@ -1039,136 +960,144 @@ __global__ __launch_bounds__(kMergeThreads) void k_lbvh_merge(ClimbArgs a, const
         }
         return out + lo * stride + (e - s_off[lo]);
     };
-    if (E > C) {
-        // In place: an entry never moves right, and a chunk is read before it is written.
+    // Merges the entries [e0, e0 + E) and appends their frontier at out + w; the
+    // place of an entry is never left of its number, so no later one is hit.
+    // Returns the new end.
+    auto merge = [&](int e0, int E, int w) {
+        for (int e = tid; e < E; e += kMergeThreads) {
+            const int node = *source(e0 + e);
+            const int first = node >= n - 1 ? node - (n - 1) : a.first[node];
+            const int last = node >= n - 1 ? node - (n - 1) : a.last[node];
+            const float4 mn = a.nmin[node], mx = a.nmax[node];
+            s_id[e] = node;
+            s_end[e] = last;
+            const int sl = C + e;
+            s_box[0][sl] = mn.x; s_box[1][sl] = mn.y; s_box[2][sl] = mn.z;
+            s_box[3][sl] = mx.x; s_box[4][sl] = mx.y; s_box[5][sl] = mx.z;
+            s_cost[sl] = a.adaptive ? a.cost[node] : 0.0f;
+            s_delta[e] = (uint8_t)(first == 0 ? 0 : 1 + kdelta<K64>(first - 1, first, n, a.keys, a.mesh_of, a.mesh_off));
+            if (e == E - 1)
+                s_delta[E] =
+                    (uint8_t)(last == n - 1 ? 0 : 1 + kdelta<K64>(last, last + 1, n, a.keys, a.mesh_of, a.mesh_off));
+            s_cnt[e] = 0;
+            s_left[e] = s_right[e] = -1;
+            s_par[e] = s_par[C + e] = -1;
+            s_out[e] = -1;
+        }
+        __syncthreads();
+        const int leaf0 = E > 0 ? (s_id[0] >= n - 1 ? s_id[0] - (n - 1) : a.first[s_id[0]]) : 0;
+        auto first_leaf = [&](int i) { return i == 0 ? leaf0 : s_end[i - 1] + 1; };
+        auto box_mn = [&](int sl) { return make_float3(s_box[0][sl], s_box[1][sl], s_box[2][sl]); };
+        auto box_mx = [&](int sl) { return make_float3(s_box[3][sl], s_box[4][sl], s_box[5][sl]); };
+        // The node of slot sl: a boundary's node is numbered by its split position.
+        auto node_of = [&](int sl) { return sl < C ? s_end[sl] : s_id[sl - C]; };
+        for (int e = tid; e < E; e += kMergeThreads) {
+            int ns = C + e, i = e, j = e;
+            while (true) {
+                const bool as_left = s_delta[j + 1] > s_delta[i];
+                const int b = as_left ? j : i - 1;
+                if (b < 0 || b >= E - 1) {   // outside these lists, or the root
+                    s_out[i] = (int16_t)ns;
+                    break;
+                }
+                s_par[ns] = (int16_t)b;
+                if (as_left) {
+                    s_left[b] = (int16_t)ns;
+                    s_lo[b] = (int16_t)i;
+                } else {
+                    s_right[b] = (int16_t)ns;
+                    s_hi[b] = (int16_t)j;
+                }
+                if (__hip_atomic_fetch_add(&s_cnt[b], 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) == 0) break;
+                i = s_lo[b];
+                j = s_hi[b];
+                const int ls = s_left[b], rs = s_right[b];
+                const int l = first_leaf(i), r = s_end[j];
+                const Combined c =
+                    combine(a, l, r, box_mn(ls), box_mx(ls), s_cost[ls], box_mn(rs), box_mx(rs), s_cost[rs]);
+                s_box[0][b] = c.mn.x; s_box[1][b] = c.mn.y; s_box[2][b] = c.mn.z;
+                s_box[3][b] = c.mx.x; s_box[4][b] = c.mx.y; s_box[5][b] = c.mx.z;
+                s_cost[b] = c.cost;
+                s_state[b] = (int8_t)c.state;
+                if (c.state == 0 && !seg_top(a.mesh_of, a.mesh_off, n, l, r)) atomicMax(&a.end_at[l], r);
+                ns = b;
+            }
+        }
+        __syncthreads();
+        // Boundaries with one arrival: the arrived child stays on the frontier.
+        for (int b = tid; b < E; b += kMergeThreads)
+            if (s_cnt[b] == 1) {
+                const int ns = s_left[b] >= 0 ? s_left[b] : s_right[b];
+                s_out[ns < C ? s_lo[ns] : ns - C] = (int16_t)ns;
+                s_par[ns] = -1;
+            }
+        __syncthreads();
+        for (int k = tid; k < 2 * E; k += kMergeThreads) {
+            const int e = k < E ? k : k - E;
+            const int sl = k < E ? e : C + e;
+            if (sl < C && s_cnt[e] != 2) continue;   // no node at this boundary
+            const int node = node_of(sl);
+            const int po = s_par[sl];
+            a.parent[node] = po >= 0 ? s_end[po] : -1;
+            if (sl >= C) continue;
+            const int l = first_leaf(s_lo[e]), r = s_end[s_hi[e]];
+            const int ls = s_left[e], rs = s_right[e];
+            a.first[node] = l;
+            a.last[node] = r;
+            a.left[node] = node_of(ls);
+            a.right[node] = node_of(rs);
+            a.state[node] = s_state[e];
+            if (a.all_boxes || po < 0) {
+                a.nmin[node] = make_float4(s_box[0][sl], s_box[1][sl], s_box[2][sl], 0.0f);
+                a.nmax[node] = make_float4(s_box[3][sl], s_box[4][sl], s_box[5][sl], 0.0f);
+                if (a.adaptive) a.cost[node] = s_cost[sl];
+            }
+            if (s_state[e] == 1 || seg_top(a.mesh_of, a.mesh_off, n, l, r)) {
+                auto row = [&](int q, int x) { return make_float4(s_box[q][x], s_box[q + 1][x], s_box[q + 2][x], 0.0f); };
+                int4 r0, r1, r2;
+                bin_rows(row(0, ls), row(3, ls), row(0, rs), row(3, rs), r0, r1, r2);
+                int4* pr = reinterpret_cast<int4*>(a.proto + 3 * (int64_t)node);
+                pr[0] = r0;
+                pr[1] = r1;
+                pr[2] = r2;
+            }
+        }
+        if (LAST && E == total) {
+            // One node is left: the root.
+            if (tid == 0) *a.root_id = node_of(s_out[0]);
+            return w;
+        }
         for (int b = 0; b < E; b += kMergeThreads) {
             const int e = b + tid;
-            const int v = e < E ? *source(e) : 0;
+            const int ns = e < E ? s_out[e] : -1;
+            const uint64_t m = ballot64(ns >= 0);
             __syncthreads();
-            if (e < E) out[e] = v;
+            if (lane_id() == 0) s_wt[tid / kWave] = __popcll(m);
             __syncthreads();
-        }
-        if (LAST) lbvh_top<K64>(a, out, E);
-        else if (tid == 0) out_count[blockIdx.x] = E;
-        return;
-    }
-    for (int e = tid; e < E; e += kMergeThreads) {
-        const int node = *source(e);
-        const int first = node >= n - 1 ? node - (n - 1) : a.first[node];
-        const int last = node >= n - 1 ? node - (n - 1) : a.last[node];
-        const float4 mn = a.nmin[node], mx = a.nmax[node];
-        s_id[e] = node;
-        s_end[e] = last;
-        const int sl = C + e;
-        s_box[0][sl] = mn.x; s_box[1][sl] = mn.y; s_box[2][sl] = mn.z;
-        s_box[3][sl] = mx.x; s_box[4][sl] = mx.y; s_box[5][sl] = mx.z;
-        s_cost[sl] = a.adaptive ? a.cost[node] : 0.0f;
-        s_delta[e] = (uint8_t)(first == 0 ? 0 : 1 + kdelta<K64>(first - 1, first, n, a.keys, a.mesh_of, a.mesh_off));
-        if (e == E - 1)
-            s_delta[E] = (uint8_t)(last == n - 1 ? 0 : 1 + kdelta<K64>(last, last + 1, n, a.keys, a.mesh_of, a.mesh_off));
-        s_cnt[e] = 0;
-        s_left[e] = s_right[e] = -1;
-        s_par[e] = s_par[C + e] = -1;
-        s_out[e] = -1;
-    }
-    __syncthreads();
-    const int leaf0 = E > 0 ? (s_id[0] >= n - 1 ? s_id[0] - (n - 1) : a.first[s_id[0]]) : 0;
-    auto first_leaf = [&](int i) { return i == 0 ? leaf0 : s_end[i - 1] + 1; };
-    auto box_mn = [&](int sl) { return make_float3(s_box[0][sl], s_box[1][sl], s_box[2][sl]); };
-    auto box_mx = [&](int sl) { return make_float3(s_box[3][sl], s_box[4][sl], s_box[5][sl]); };
-    // The node of slot sl: a boundary's node is numbered by its split position.
-    auto node_of = [&](int sl) { return sl < C ? s_end[sl] : s_id[sl - C]; };
-    for (int e = tid; e < E; e += kMergeThreads) {
-        int ns = C + e, i = e, j = e;
-        while (true) {
-            const bool as_left = s_delta[j + 1] > s_delta[i];
-            const int b = as_left ? j : i - 1;
-            if (b < 0 || b >= E - 1) {   // outside these lists, or the root
-                s_out[i] = (int16_t)ns;
-                break;
+            int rank = w + count_below(m);
+            for (int v = 0; v < kMergeThreads / kWave; ++v) {
+                if (v < tid / kWave) rank += s_wt[v];
+                w += s_wt[v];
             }
-            s_par[ns] = (int16_t)b;
-            if (as_left) {
-                s_left[b] = (int16_t)ns;
-                s_lo[b] = (int16_t)i;
-            } else {
-                s_right[b] = (int16_t)ns;
-                s_hi[b] = (int16_t)j;
-            }
-            if (__hip_atomic_fetch_add(&s_cnt[b], 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) == 0) break;
-            i = s_lo[b];
-            j = s_hi[b];
-            const int ls = s_left[b], rs = s_right[b];
-            const int l = first_leaf(i), r = s_end[j];
-            const Combined c = combine(a, l, r, box_mn(ls), box_mx(ls), s_cost[ls], box_mn(rs), box_mx(rs), s_cost[rs]);
-            s_box[0][b] = c.mn.x; s_box[1][b] = c.mn.y; s_box[2][b] = c.mn.z;
-            s_box[3][b] = c.mx.x; s_box[4][b] = c.mx.y; s_box[5][b] = c.mx.z;
-            s_cost[b] = c.cost;
-            s_state[b] = (int8_t)c.state;
-            if (c.state == 0 && !seg_top(a.mesh_of, a.mesh_off, n, l, r)) atomicMax(&a.end_at[l], r);
-            ns = b;
+            if (ns >= 0) out[rank] = node_of(ns);
         }
+        return w;
+    };
+    while (true) {
+        const bool fits = total <= C;
+        int w = 0;
+        for (int e0 = 0; e0 < total; e0 += C) {
+            w = merge(e0, min(C, total - e0), w);
+            __syncthreads();  // the frontier is written and LDS is free
+        }
+        if (fits || w >= total) {   // (a full run always shrinks)
+            total = w;
+            break;
+        }
+        total = w;
+        joined = true;
     }
-    __syncthreads();
-    // Boundaries with one arrival: the arrived child stays on the frontier.
-    for (int b = tid; b < E; b += kMergeThreads)
-        if (s_cnt[b] == 1) {
-            const int ns = s_left[b] >= 0 ? s_left[b] : s_right[b];
-            s_out[ns < C ? s_lo[ns] : ns - C] = (int16_t)ns;
-            s_par[ns] = -1;
-        }
-    __syncthreads();
-    for (int k = tid; k < 2 * E; k += kMergeThreads) {
-        const int e = k < E ? k : k - E;
-        const int sl = k < E ? e : C + e;
-        if (sl < C && s_cnt[e] != 2) continue;   // no node at this boundary
-        const int node = node_of(sl);
-        const int po = s_par[sl];
-        a.parent[node] = po >= 0 ? s_end[po] : -1;
-        if (sl >= C) continue;
-        const int l = first_leaf(s_lo[e]), r = s_end[s_hi[e]];
-        const int ls = s_left[e], rs = s_right[e];
-        a.first[node] = l;
-        a.last[node] = r;
-        a.left[node] = node_of(ls);
-        a.right[node] = node_of(rs);
-        a.state[node] = s_state[e];
-        if (a.all_boxes || po < 0) {
-            a.nmin[node] = make_float4(s_box[0][sl], s_box[1][sl], s_box[2][sl], 0.0f);
-            a.nmax[node] = make_float4(s_box[3][sl], s_box[4][sl], s_box[5][sl], 0.0f);
-            if (a.adaptive) a.cost[node] = s_cost[sl];
-        }
-        if (s_state[e] == 1 || seg_top(a.mesh_of, a.mesh_off, n, l, r)) {
-            auto row = [&](int q, int x) { return make_float4(s_box[q][x], s_box[q + 1][x], s_box[q + 2][x], 0.0f); };
-            int4 r0, r1, r2;
-            bin_rows(row(0, ls), row(3, ls), row(0, rs), row(3, rs), r0, r1, r2);
-            int4* pr = reinterpret_cast<int4*>(a.proto + 3 * (int64_t)node);
-            pr[0] = r0;
-            pr[1] = r1;
-            pr[2] = r2;
-        }
-    }
-    if (LAST) {
-        // One node is left: the root.
-        if (tid == 0) *a.root_id = node_of(s_out[0]);
-        return;
-    }
-    int total = 0;
-    for (int b = 0; b < E; b += kMergeThreads) {
-        const int e = b + tid;
-        const int ns = e < E ? s_out[e] : -1;
-        const uint64_t m = ballot64(ns >= 0);
-        __syncthreads();
-        if (lane_id() == 0) s_wt[tid / kWave] = __popcll(m);
-        __syncthreads();
-        int rank = total + count_below(m);
-        for (int w = 0; w < kMergeThreads / kWave; ++w) {
-            if (w < tid / kWave) rank += s_wt[w];
-            total += s_wt[w];
-        }
-        if (ns >= 0) out[rank] = node_of(ns);
-    }
-    if (tid == 0) out_count[blockIdx.x] = total;
+    if (!LAST && tid == 0) out_count[blockIdx.x] = total;
 }
 
 // ---------------------------------------------------------------------------

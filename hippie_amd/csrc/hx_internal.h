@@ -143,7 +143,6 @@ struct ClimbArgs {
     const int32_t* split;     // n-1, or NULL for a Karras tree: last leaf of each node's left child
     const void* keys;         // launch_lbvh_climb: the sorted Morton keys,
     int keys64;
-    uint64_t* link;           // n-1 arrival words of the top level,
     int32_t* root_id;         // and the root's node id (out)
     int all_boxes;            // 1: store every node's box (else only those a later stage reads)
     float4* proto;            // n-1 x 3: Bin rows 0-2 (both child boxes) of every state-1 or root node

@@ -480,3 +480,42 @@ def test_smaller_sort_keeps_the_status_buffer(digits):
         torch.cuda.synchronize()
         assert np.array_equal(keys[1].cpu().numpy(), src[1][order].cpu().numpy())
         assert np.array_equal(vals[1].cpu().numpy(), order.int().cpu().numpy())
+
+
+# More than 640 entries of a merge go in runs that leave at most 258 nodes each: one
+# run and a few entries, several runs, and three levels of them.
+@pytest.mark.parametrize("clusters", [11, 12, 45, 300, 1200])
+@pytest.mark.parametrize("adaptive", [0, 1])
+def test_lbvh_merge_in_runs(oracle, ctx, clusters, adaptive):
+    v, t = _edge_heavy_blocks(clusters)
+    bvh = hx.LBVHBuilder(ctx, morton_bits=60, adaptive_leaf_size=adaptive, max_leaf_size=3).build(hx.Scene(v, t))
+    ref = oracle.build_lbvh(v, t, bits=60, adaptive=bool(adaptive), max_leaf_size=3)
+    a = oracle.bin_canonical(bvh.nodes_host(), bvh.n_interior, bvh.n_leaves, bvh.tri_indices_host())
+    b = oracle.bin_canonical(ref["nodes"], ref["n_interior"], ref["n_leaves"], ref["tri_idx"])
+    assert np.array_equal(a, b)
+
+
+def test_lbvh_merge_in_runs_batched(oracle, ctx):
+    meshes = [_edge_heavy_blocks(c) for c in (30, 1, 64)]
+    hb = hx.HipBatch(ctx, hx.MeshBatch.from_meshes(meshes), morton_bits=60)
+    for m, (v, t) in enumerate(meshes):
+        got, ref = hb.mesh_host(m), oracle.build_lbvh(v, t, bits=60)
+        a = oracle.bin_canonical(got["nodes"], got["n_interior"], got["n_leaves"], got["tri_idx"])
+        b = oracle.bin_canonical(ref["nodes"], ref["n_interior"], ref["n_leaves"], ref["tri_idx"])
+        assert np.array_equal(a, b), m
+
+
+def test_lbvh_merge_in_runs_time(ctx):
+    """1.5M triangles with ~50 nodes straddling each block: 0.68 ms for the climb; a single
+    workgroup's climb of what is left over took 64 ms."""
+    v, t = _edge_heavy_blocks(3000)
+    scene, builder = hx.Scene(v, t), hx.LBVHBuilder(ctx, morton_bits=60)
+    bvh = builder.build(scene)
+    ctx.set_profiling(True)
+    ctx.profile_reset()
+    try:
+        builder.rebuild(bvh, scene)
+        ms = ctx.profile()["climb"][1]
+    finally:
+        ctx.set_profiling(False)
+    assert ms < 10.0
