@@ -122,8 +122,19 @@ class Autotuner:
         def run():
             keys.copy_(src)
             core.sort_pairs(self.ctx, keys, vals, bits)
-        best = self._descend([("sort_digit_bits", SORT_DIGITS), ("sort_items", SORT_ITEMS),
-                              ("sort_lookback", SORT_LOOKBACK)], run)
+        knobs = [("sort_digit_bits", SORT_DIGITS), ("sort_items", SORT_ITEMS), ("sort_lookback", SORT_LOOKBACK)]
+        # A knob that does not reach sorts of this size keeps its value (candidates
+        # of one kernel differ by noise only, and larger sorts would inherit the
+        # pick): up to 8192 keys one workgroup sorts, and fewer than two 4096-key
+        # tiles a CU are sorted 8 a thread.
+        if n <= 8192:
+            reached = []
+        elif n < 4096 * torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count:
+            reached = [k for k in knobs if k[0] != "sort_items"]
+        else:
+            reached = knobs
+        best = {k: self.ctx.get_tuning(k) for k, _ in knobs}
+        best.update(self._descend(reached, run))
         self.cache[key] = best
         self._save()
         return best

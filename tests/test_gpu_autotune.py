@@ -69,3 +69,18 @@ def test_autotune_batch_trace_keeps_hits(ctx):
     assert hb.launch == best
     assert {k: ctx.get_tuning(k) for k in saved} == saved
     assert torch.equal(hb.trace(rays, owner), before)
+
+
+@pytest.mark.parametrize("keys, reached", [(5000, ()), (200000, ("sort_digit_bits", "sort_lookback")),
+                                           (1 << 21, ("sort_digit_bits", "sort_items", "sort_lookback"))])
+def test_tune_sort_leaves_what_it_does_not_reach(keys, reached):
+    """Sorts of few keys ignore some knobs: those are not timed and keep their values."""
+    c = hx.Context(0)
+    c.set_tuning("sort_items", 32)
+    knobs = ("sort_digit_bits", "sort_items", "sort_lookback")
+    before = {k: c.get_tuning(k) for k in knobs}
+    at = Autotuner(c, repeats=1)
+    best = at.tune_sort(keys, bits=60)
+    assert set(best) == set(knobs) and best == {k: c.get_tuning(k) for k in knobs}
+    assert {k for k, _, _ in at.history} == set(reached)
+    assert all(best[k] == before[k] for k in knobs if k not in reached)
