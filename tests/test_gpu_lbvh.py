@@ -519,3 +519,19 @@ def test_lbvh_merge_in_runs_time(ctx):
     finally:
         ctx.set_profiling(False)
     assert ms < 10.0
+
+
+@pytest.mark.parametrize("n", [64, 65, 66, 1000, 5000, 8192])
+@pytest.mark.parametrize("run", [63, 64, 65, 66, 8192])
+def test_sort_pairs_one_workgroup_runs(ctx, n, run):
+    """Runs of equal high bits up to, at and over the longest one ranked in place (64)."""
+    rng = np.random.default_rng(n + run)
+    high = np.repeat(rng.permutation(n // run + 1), run)[:n].astype(np.uint64) << np.uint64(40)
+    k = (high | rng.integers(0, 1 << 28, n, dtype=np.uint64))[rng.permutation(n)]
+    vals = rng.permutation(n).astype(np.int32)
+    kt = torch.from_numpy(k.view(np.int64).copy()).cuda()
+    vt = torch.from_numpy(vals.copy()).cuda()
+    hx.sort_pairs(ctx, kt, vt, 60)
+    order = np.argsort(k, kind="stable")
+    assert np.array_equal(kt.cpu().numpy().view(np.uint64), k[order])
+    assert np.array_equal(vt.cpu().numpy(), vals[order])
