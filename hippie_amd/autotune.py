@@ -122,19 +122,16 @@ class Autotuner:
         def run():
             keys.copy_(src)
             core.sort_pairs(self.ctx, keys, vals, bits)
-        knobs = [("sort_digit_bits", SORT_DIGITS), ("sort_items", SORT_ITEMS), ("sort_lookback", SORT_LOOKBACK)]
         # A knob that does not reach sorts of this size keeps its value (candidates
         # of one kernel differ by noise only, and larger sorts would inherit the
-        # pick): up to 8192 keys one workgroup sorts, and fewer than two 4096-key
-        # tiles a CU are sorted 8 a thread.
-        if n <= 8192:
-            reached = []
-        elif n < 4096 * torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count:
-            reached = [k for k in knobs if k[0] != "sort_items"]
-        else:
-            reached = knobs
-        best = {k: self.ctx.get_tuning(k) for k, _ in knobs}
-        best.update(self._descend(reached, run))
+        # pick): up to 8192 keys one workgroup sorts, and fewer than 2560 keys a CU
+        # (10-bit digits: 1024) are sorted 8 a thread.
+        best = {k: self.ctx.get_tuning(k) for k in ("sort_digit_bits", "sort_items", "sort_lookback")}
+        if n > 8192:
+            best.update(self._descend([("sort_digit_bits", SORT_DIGITS)], run))
+            cus = torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
+            items = [("sort_items", SORT_ITEMS)] if n >= cus * (2560 if best["sort_digit_bits"] == 8 else 1024) else []
+            best.update(self._descend(items + [("sort_lookback", SORT_LOOKBACK)], run))
         self.cache[key] = best
         self._save()
         return best

@@ -589,19 +589,18 @@ int64_t sort_status_words(int rb, int items, int64_t n, int bits) {
     return (int64_t)passes * sort_tiles(n, items) * (1 << rb) + (int64_t)passes * (1 << rb) + kMaxPasses;
 }
 
-// Keys per thread of a digit pass: the tunable, but at most 8 while 16 would not
-// give every CU two tiles.  A tile's latency grows with its keys per thread and
-// nothing else fills the chip there: 65,536 60-bit keys 119 -> 91 us, 262,143
-// 136 -> 117 us; above, the fewer and longer digit runs win (1,048,576: 151
-// against 158 us, 16.7M: 869 against 1044 us).  Twice the tiles need twice the
-// status words: a workspace of the caller that does not hold them (10-bit digits,
-// from 600,000 keys on in hx_trace_sorted_noalloc) gets the tunable's.
-inline int64_t sort_few_keys(const Context* c) { return (int64_t)c->cu_count * 2 * kSortBlock * 8; }
-int sort_items_for(const Context* c, int64_t n, int end_bit, const SortWorkspace* ws) {
-    const int items = n < sort_few_keys(c) ? std::min(c->tune.sort_items, 8) : c->tune.sort_items;
-    if (ws != nullptr && sort_status_words(c->tune.sort_digit_bits, items, n, end_bit) > ws->status_words)
-        return c->tune.sort_items;
-    return items;
+// Keys per thread of a digit pass: the tunable, but at most 8 for few keys.  A
+// tile's latency grows with its keys per thread and nothing else fills the chip
+// there; with more, the fewer and longer digit runs win, earlier with 10-bit digits
+// whose runs are a quarter as long.  8 against 16 keys, 60 key bits, 8-bit digits:
+// 100,000 keys 98 and 123 us, 500,000 115 and 119, 700,000 137 and 136, 1,000,000
+// 155 and 147, 16.7M 1044 and 869; 10-bit: 200,000 155 and 164, 300,000 153 and 151,
+// 900,000 244 and 204.
+inline int64_t sort_few_keys(const Context* c) {
+    return (int64_t)c->cu_count * (c->tune.sort_digit_bits == 8 ? 2560 : 1024);
+}
+int sort_items_for(const Context* c, int64_t n) {
+    return n < sort_few_keys(c) ? std::min(c->tune.sort_items, 8) : c->tune.sort_items;
 }
 
 // The context's status words for a sort of n keys with `items` each: also what
@@ -744,7 +743,7 @@ int launch_sort_pairs(Context* c, void* keys[2], int32_t* vals[2], int64_t n, in
         set_error("radix sort: n = %lld exceeds 2^30 - 1", (long long)n);
         return HX_ERR_INVALID_ARG;
     }
-    const int bits = c->tune.sort_digit_bits, items = sort_items_for(c, n, end_bit, ws), lb = c->tune.sort_lookback;
+    const int bits = c->tune.sort_digit_bits, items = sort_items_for(c, n), lb = c->tune.sort_lookback;
     // Long keys, many of them: four digit passes over the high bits leave runs
     // of equal high bits that are short for Morton codes (at most 19 keys for
     // the 16.7M-triangle benchmark scene at 32 high bits), which one pass

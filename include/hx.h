@@ -150,16 +150,18 @@ int hx_context_profile_entry(hx_context* ctx, int32_t index, char* name, int32_t
 int hx_context_profile_reset(hx_context* ctx);
 /* Launch-shape tunables chosen by the autotuner (no reference counterpart;
  * the reference hard-codes them, HipTracerBinKernels.cu:5-6,10-15):
- *   "trace_lds_stack"      traversal-stack entries held in LDS (0,16,24,32,64)
+ *   "trace_lds_stack"      traversal-stack entries held in LDS (0,16,24,32,64; Bin closest-hit
+ *                          traces of up to 16 rays a lane slot share rays between lanes with 16)
  *   "trace_fetch"          refill a wave when fewer of its 64 lanes are busy
  *   "trace_blocks_per_cu"  persistent trace workgroups per CU (0 = occupancy)
  *   "trace_postpone"       leaves a lane holds back while its wave traverses (1 to 4; Bin layout;
  *                          any-hit rays test theirs oldest first, so their hits stay the same)
  *   "trace_woop_ahead"     Woop rows of a leaf's next triangle read while the current one is
  *                          tested (1 or 2; Bin layout)
- *   "sort_digit_bits"      radix digit width of every sort (8 or 10)
- *   "sort_items"           keys per thread in a sort pass (8, 16 or 32; 8 while the tiles do not
- *                          fill the chip twice)
+ *   "sort_digit_bits"      radix digit width (8 or 10); this and the next two: of sorts of more
+ *                          than 8192 keys (one workgroup sorts up to that many)
+ *   "sort_items"           keys per thread in a sort pass (8, 16 or 32; at most 8 for fewer than
+ *                          2560 keys a CU, or 1024 with 10-bit digits)
  *   "sort_lookback"        tiles read per sort look-back round trip (4, 8, 16)
  *   "sort_local_run"       the builds' Morton sorts and hx_sort_pairs_u64 of
  *                          > 40-bit keys with at least 2^18 keys run four

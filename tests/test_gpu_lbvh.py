@@ -448,13 +448,13 @@ def test_lbvh_merge_level_edges(oracle, ctx, n, adaptive):
     assert np.array_equal(a, b)
 
 
-# Sorts of fewer keys than two 4096-key tiles a CU take smaller tiles and may need
-# more status words than a larger sort: those are reserved with the larger one's.
+# Sorts of fewer than 2560 keys a CU (10-bit digits: 1024) take smaller tiles and may
+# need more status words than a larger sort: those are reserved with the larger one's.
 @pytest.mark.parametrize("digits", [8, 10])
 def test_smaller_sort_keeps_the_status_buffer(digits):
     c = hx.Context(0)
     c.set_tuning("sort_digit_bits", digits)
-    line = torch.cuda.get_device_properties(0).multi_processor_count * 4096
+    line = torch.cuda.get_device_properties(0).multi_processor_count * (2560 if digits == 8 else 1024)
     rng = np.random.default_rng(digits)
     src = [torch.from_numpy(rng.integers(0, 1 << 62, n, dtype=np.int64)).cuda() for n in (line, line - 1)]
     keys = [k.clone() for k in src]
@@ -519,6 +519,40 @@ def test_lbvh_merge_in_runs_time(ctx):
     finally:
         ctx.set_profiling(False)
     assert ms < 10.0
+
+
+# Both sides of the line from which a sort takes the tunable's keys per thread, the
+# smallest tiled sort, and more keys than any clamp, with every instantiation.
+@pytest.mark.parametrize("digits", [8, 10])
+@pytest.mark.parametrize("items", [8, 16, 32])
+@pytest.mark.parametrize("lookback", [4, 8, 16])
+def test_sort_pairs_tiled_sizes(digits, items, lookback):
+    c = hx.Context(0)
+    for name, value in (("sort_digit_bits", digits), ("sort_items", items), ("sort_lookback", lookback)):
+        c.set_tuning(name, value)
+    line = torch.cuda.get_device_properties(0).multi_processor_count * (2560 if digits == 8 else 1024)
+    for n, bits in ((8193, 64), (line - 1, 41), (line, 60), (2 * line + 12345, 33)):
+        rng = np.random.default_rng(n + items)
+        k = rng.integers(0, 1 << 63, n, dtype=np.uint64) >> np.uint64(63 - min(bits, 63))
+        k[: n // 3] = k[0]
+        vals = rng.permutation(n).astype(np.int32)
+        kt = torch.from_numpy(k.view(np.int64).copy()).cuda()
+        vt = torch.from_numpy(vals.copy()).cuda()
+        hx.sort_pairs(c, kt, vt, bits)
+        order = np.argsort(k, kind="stable")
+        assert np.array_equal(kt.cpu().numpy().view(np.uint64), k[order])
+        assert np.array_equal(vt.cpu().numpy(), vals[order])
+
+
+@pytest.mark.parametrize("local_run", [1, 64])
+def test_lbvh_large_sort_32_keys_per_thread(oracle, local_run):
+    """32 keys per thread in a build whose sort is above the line; with runs of one key
+    allowed the split sort falls back to the remaining passes."""
+    c = hx.Context(0)
+    c.set_tuning("sort_items", 32)
+    c.set_tuning("sort_local_run", local_run)
+    v, t = scenes.gaussian_mixture_soup(800000, seed=5)
+    _check_build(oracle, c, v, t, 60)
 
 
 @pytest.mark.parametrize("n", [64, 65, 66, 1000, 5000, 8192])
