@@ -20,9 +20,10 @@
 //            added as 64-bit integers, so the total (and every convergence
 //            decision taken from it) is independent of the order of the
 //            additions.  The reference adds float block sums atomically.
-// The host reads the cost and the counts back after each step and applies the
-// reference's rules: keep the best tree, stop when the cost changes by at
-// most 0.01 (or nothing moved) at mod 1, lower mod when it stalls.
+// k_ins_step then applies the reference's rules on the device: keep the best
+// tree, stop when the cost changes by at most 0.01 (or nothing moved) at mod 1,
+// lower mod when it stalls.  The host launches kInsBatch steps at a time and reads
+// the state after them; steps past the end do nothing.
 #include <algorithm>
 #include <cmath>
 #include <vector>

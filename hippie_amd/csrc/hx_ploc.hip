@@ -172,10 +172,10 @@ HX_DEV bool ploc_pair_round(int m, const int32_t* cmesh, int n_meshes, int i, in
     return true;
 }
 
-// Place of the cluster nearest to the one at place `me` among the r places on
-// either side (the lowest on ties), -1 without one; sa, sb: boxes, sm: meshes.
+// Place of the cluster nearest to the one at place `me` among the places [q0, q1)
+// (the lowest on ties), -1 without one; sa, sb: boxes, sm: meshes.
 template <bool MESH>
-HX_DEV int scan_window(const float4* sa, const float2* sb, const int32_t* sm, int me, int r) {
+HX_DEV int scan_window(const float4* sa, const float2* sb, const int32_t* sm, int me, int q0, int q1) {
     const Box3 own = cluster_box(sa[me], sb[me]);
     const float3 lo = make_float3(vmin(own.mn.x, own.mx.x), vmin(own.mn.y, own.mx.y), vmin(own.mn.z, own.mx.z));
     const float3 hi = make_float3(vmax(own.mn.x, own.mx.x), vmax(own.mn.y, own.mx.y), vmax(own.mn.z, own.mx.z));
@@ -188,17 +188,17 @@ HX_DEV int scan_window(const float4* sa, const float2* sb, const int32_t* sm, in
         bestD = better ? d : bestD;
         best = better ? q : best;
     };
-    auto scan = [&](int q, int q1) {
-        for (; q + 4 <= q1; q += 4) {
+    auto scan = [&](int q, int end) {
+        for (; q + 4 <= end; q += 4) {
             step(q);
             step(q + 1);
             step(q + 2);
             step(q + 3);
         }
-        for (; q < q1; ++q) step(q);
+        for (; q < end; ++q) step(q);
     };
-    scan(me - r, me);
-    scan(me + 1, me + r + 1);
+    scan(q0, me);
+    scan(me + 1, q1);
     return best;
 }
 
@@ -232,7 +232,7 @@ __global__ __launch_bounds__(kBlock) void k_ploc_neighbours(const float4* __rest
     }
     __syncthreads();
     if (i >= m) return;
-    const int best = scan_window<MESH>(sa, sb, sm, threadIdx.x + r, r);
+    const int best = scan_window<MESH>(sa, sb, sm, threadIdx.x + r, threadIdx.x, threadIdx.x + 2 * r + 1);
     nb[i] = best < 0 ? -1 : best + b0 - r;
 }
 
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(kTile) void k_ploc_pairs(const float4* __restrict__
         }
         __syncthreads();
         if (i >= 0 && i < m) {
-            const int best = scan_window<MESH>(sa, sb, sm, t + r, r);
+            const int best = scan_window<MESH>(sa, sb, sm, t + r, t, t + 2 * r + 1);
             j = best < 0 ? -1 : best + b0 - 2 * r;
         }
     }
@@ -502,31 +502,7 @@ __global__ __launch_bounds__(kTailBlock) void k_ploc_tail(PlocArgs a, int src, i
                 s_nb[i] = (i ^ 1) < m ? (i ^ 1) : -1;
                 continue;
             }
-            const Box3 own = cluster_box(s_a[i], s_b[i]);
-            const float3 lo = make_float3(vmin(own.mn.x, own.mx.x), vmin(own.mn.y, own.mx.y),
-                                          vmin(own.mn.z, own.mx.z));
-            const float3 hi = make_float3(vmax(own.mn.x, own.mx.x), vmax(own.mn.y, own.mx.y),
-                                          vmax(own.mn.z, own.mx.z));
-            int best = -1;
-            float bestD = kHalfMax;
-            auto step = [&](int q) {
-                const float d = half_union_area(s_a[q], s_b[q], lo, hi);
-                const bool better = bestD > d && (!BATCHED || s_mesh[q] == s_mesh[i]);
-                bestD = better ? d : bestD;
-                best = better ? q : best;
-            };
-            auto scan = [&](int q, int q1) {
-                for (; q + 4 <= q1; q += 4) {
-                    step(q);
-                    step(q + 1);
-                    step(q + 2);
-                    step(q + 3);
-                }
-                for (; q < q1; ++q) step(q);
-            };
-            scan(max(0, i - r), i);
-            scan(i + 1, min(m - 1, i + r) + 1);
-            s_nb[i] = best;
+            s_nb[i] = scan_window<BATCHED>(s_a, s_b, s_mesh, i, max(0, i - r), min(m, i + r + 1));
         }
         __syncthreads();
         int2 f[kPer];
