@@ -113,8 +113,8 @@ def test_ploc_rebuild_reuses_handle(oracle, ctx):
     assert np.array_equal(cg, co)
 
 
-# Tiles of 1024 clusters, the one-workgroup tail from 2048 down, and the widest
-# window that fits in LDS (r = 1024).
+# The one-workgroup tail from 2048 clusters down (1024 threads, two clusters each
+# above 1024), a few sizes above it, and the widest window that fits in LDS (r = 1024).
 @pytest.mark.parametrize("n", [2, 3, 1023, 1024, 1025, 2047, 2048, 2049, 3073, 5000])
 @pytest.mark.parametrize("radius", [1, 3, 26, 1024, 1025])
 def test_ploc_tile_and_window_edges(oracle, ctx, n, radius):
@@ -129,6 +129,15 @@ def test_ploc_tile_and_window_edges(oracle, ctx, n, radius):
 def test_ploc_pair_tiles(oracle, ctx, n, radius):
     v, t = scenes.merge(scenes.uniform_soup(n - n // 2, seed=n), scenes.gaussian_mixture_soup(n // 2, seed=radius))
     _check(oracle, ctx, v, t, radius)
+
+
+# Larger radii count pairs over tiles of 512 clusters: whole tiles, one cluster more
+# and one less, above the tail.
+@pytest.mark.parametrize("n", [2559, 2560, 2561, 3071, 3073, 4096, 4097])
+@pytest.mark.parametrize("radius", [49, 300, 1025])
+def test_ploc_count_tiles(oracle, ctx, n, radius):
+    v, t = scenes.merge(scenes.uniform_soup(n - n // 2, seed=n), scenes.gaussian_mixture_soup(n // 2, seed=radius))
+    _check(oracle, ctx, v, t, radius, max_radius=2048)
 
 
 def test_ploc_pair_tiles_grow(oracle, ctx):

@@ -1,5 +1,5 @@
 """Ray hand-out of the trace kernels: every ray is traced exactly once whatever
-the rays per wave (16, 32, 64), the length of the runs a wave takes and the
+the rays per wave (8 to 64), the length of the runs a wave takes and the
 leaves it holds back, and any-hit rays report the first hit of the reference's
 traversal order.  Hits are compared bit for bit with the one-lane CPU oracle.
 """
