@@ -34,10 +34,11 @@ HBM_PEAK_GBS = 8000.0
 TRAFFIC_PROFILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "lbvh60_16M_hbm_traffic.md")
 
 
-# The kernels behind each timed build stage, as the PMC summary names them.
-PMC_KERNELS = {"scene_box": ("k_scene_box_partial", "k_scene_box_final"), "morton": ("k_morton",),
-               "sort_hist": ("k_sort_hist",), "climb": ("k_lbvh_local", "k_lbvh_top"),
-               "sort_local": ("k_sort_local",), "collapse_emit": ("k_emit",)}
+# The kernels behind each timed build stage, as the PMC summary names them, and
+# their dispatches in it (16,777,216 triangles take four levels of merges).
+PMC_KERNELS = {"scene_box": (("k_scene_box_partial", 1), ("k_scene_box_final", 1)), "morton": (("k_morton", 1),),
+               "sort_hist": (("k_sort_hist", 1),), "climb": (("k_lbvh_local", 1), ("k_lbvh_merge", 4)),
+               "sort_local": (("k_sort_local", 1),), "collapse_emit": (("k_emit", 1),)}
 
 
 def measured_traffic(kernel):
@@ -683,10 +684,11 @@ def main():
             # one histogram per sort: the build's keys and the two ray sets
             per_launch = (8 * n + 8 * (prim.shape[0] + sec.shape[0])) / (cnt / args.steps)
         gbs = per_launch / (tot / cnt * 1e-3) / 1e9
-        traffic = [measured_traffic(name) for name in PMC_KERNELS.get(k, ())]
+        traffic = [(measured_traffic(name), times) for name, times in PMC_KERNELS.get(k, ())]
         build_kernels[k] = {"avg_ms": round(tot / cnt, 5), "bytes_per_launch": int(per_launch),
                             "achieved_gbs": round(gbs, 1), "frac": round(gbs / HBM_PEAK_GBS, 4),
-                            "traffic": sum(traffic) if traffic and None not in traffic else None}
+                            "traffic": sum(b * c for b, c in traffic)
+                            if traffic and all(b is not None for b, _ in traffic) else None}
 
     ray_sort_ms, trace_only_ms = sort_and_trace_ms(tracer, [prim_rb, sec_rb])
     model = {"primary": traversal_model(ctx, bvh, prim_rb, hx), "diffuse": traversal_model(ctx, bvh, sec_rb, hx)}
