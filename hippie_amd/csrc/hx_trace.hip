@@ -824,18 +824,16 @@ __global__ void k_zero_control(int32_t* control) {
 // control[kControlAlike] is set if in more than half of them every ray is live (a
 // dead one, with an empty interval, ends at once whatever its origin: the secondary
 // rays of misses) and starts at the same point.
-constexpr int kAlikeBlock = 1024, kAlikeWindows = 64;
+constexpr int kAlikeBlock = 1024, kAlikeWindows = 16;
 __global__ __launch_bounds__(kAlikeBlock) void k_zero_control_alike(TraceArgs a) {
     __shared__ int s_alike[kAlikeBlock / kWave];
     const int w = threadIdx.x / kWave;
-    int count = 0;
-    for (int k = w; k < kAlikeWindows; k += kAlikeBlock / kWave) {
-        const int64_t slot = (a.n_rays - kWave) * k / (kAlikeWindows - 1) + lane_id();
-        const int64_t ray = a.order ? a.order[slot] : slot;
-        const float4 o = a.rays[2 * ray], d = a.rays[2 * ray + 1];
-        auto first = [](float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); };
-        count += __all(o.x == first(o.x) && o.y == first(o.y) && o.z == first(o.z) && d.w > o.w) ? 1 : 0;
-    }
+    static_assert(kAlikeWindows == kAlikeBlock / kWave, "one window a wave");
+    const int64_t slot = (a.n_rays - kWave) * w / (kAlikeWindows - 1) + lane_id();
+    const int64_t ray = a.order ? a.order[slot] : slot;
+    const float4 o = a.rays[2 * ray], d = a.rays[2 * ray + 1];
+    auto first = [](float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); };
+    int count = __all(o.x == first(o.x) && o.y == first(o.y) && o.z == first(o.z) && d.w > o.w) ? 1 : 0;
     if (lane_id() == 0) s_alike[w] = count;
     __syncthreads();
     if (threadIdx.x != 0) return;
@@ -845,21 +843,23 @@ __global__ __launch_bounds__(kAlikeBlock) void k_zero_control_alike(TraceArgs a)
 }
 
 // Large sets are looked over for rays from one point (k_zero_control_alike; RayPool
-// and k_trace say what they get): from 4 rays a
-// lane slot on (2.1M rays; the wide kernels and sorted sets), 12 in input order
-// (6.3M).  Below, and where half of the rays miss at the root, the one ray counter
-// would set the pace: unsorted 1,048,576 rays over 65,536 triangles 359 -> 370 us,
-// a step with 4.2M camera rays over 1.3M triangles 1.76 -> 1.81 ms.  Primaries of the Gaussian
-// mixture and ground grid, refill by refill with scalar reads against runs with
-// vector reads: 16.7M sorted rays over 16.7M / 1M / 65k triangles 6.39 -> 4.82,
-// 7.79 -> 6.46, 4.15 -> 3.49 ms (Quad, 16.7M and 65k: 6.79 -> 4.98, 4.51 -> 3.48;
-// Oct: 9.14 -> 7.01, 5.30 -> 4.30), 4.2M sorted 2.04 -> 1.53, 2.38 -> 2.02,
-// 1.27 -> 1.04 ms, 16.7M in input order 6.24 -> 5.15, 7.78 -> 7.02, 4.14 -> 3.52 ms.
-// Of the 1.6 ms at 16.7M triangles the hand-out gives 0.7 ms, the scalar reads 0.9.
-// The diffuse rays of these scenes take what they took (9.83, 10.4, 3.75 ms).  The
-// counts of a stats trace keep to one kernel.
+// and k_trace say what they get): sorted sets from 2 rays a lane slot on (1.05M;
+// any-hit rays, which seldom share an origin, from 4: the look costs 2.0M of them
+// 0.8 %), from 4 in the wide kernels (2.1M), from 12 in input order (6.3M).  Below, and where half of
+// the rays miss at the root, the one ray counter would set the pace: unsorted
+// 1,048,576 rays over 65,536 triangles 359 -> 369 us, a step with 4.2M camera rays
+// over 1.3M triangles 1.75 -> 1.79 ms.  Primaries of the Gaussian mixture and ground
+// grid, refill by refill with scalar reads against runs with vector reads: 16.7M
+// sorted rays over 16.7M / 1M / 65k triangles 6.39 -> 4.82, 7.79 -> 6.46, 4.15 ->
+// 3.49 ms (Quad, 16.7M and 65k: 6.79 -> 4.98, 4.51 -> 3.48; Oct: 9.14 -> 7.01, 5.30 ->
+// 4.30), 4.2M sorted 2.04 -> 1.53, 2.38 -> 2.02, 1.27 -> 1.04 ms, 1.05M sorted 0.83 ->
+// 0.68, 0.92 -> 0.80, 0.47 -> 0.42 ms, 16.7M in input order 6.24 -> 5.15, 7.78 -> 7.02,
+// 4.14 -> 3.52 ms.  Of the 1.6 ms at 16.7M triangles the hand-out gives 0.7 ms, the
+// scalar reads 0.9.  The diffuse rays of these scenes take what they took (16.7M: 9.83,
+// 10.4, 3.75 ms).  The counts of a stats trace keep to one kernel.
 bool alike_pays(const Context* c, const TraceArgs& a, bool wide) {
-    return !a.stats && a.n_rays >= (int64_t)c->cu_count * 8 * kTraceBlock * (a.order || wide ? 4 : 12);
+    return !a.stats && a.n_rays >= (int64_t)c->cu_count * 8 * kTraceBlock *
+                                      (wide ? 4 : !a.order ? 12 : a.any_hit ? 4 : 2);
 }
 
 int zero_control(Context* c, const TraceArgs& a, bool wide) {

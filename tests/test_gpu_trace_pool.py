@@ -127,16 +127,16 @@ def _point_rays(n, seed, kind):
     return r
 
 
-# Sets from 4 rays a lane slot on (sorted ones and the wide layouts; 12 in input
-# order) are looked over for rays from one point, which are handed out refill by
-# refill and read nodes by scalar loads: sizes around both, and sets that are only
-# partly alike.
+# Sorted sets from 2 rays a lane slot on (the wide layouts: 4, sorted or not; input
+# order: 12) are looked over for rays from one point, which are handed out refill by
+# refill and read nodes by scalar loads: sizes around the lines, and sets that are
+# only partly alike.
 @pytest.mark.parametrize("layout", ["bin", "quad", "oct"])
 @pytest.mark.parametrize("sort", [False, True])
 @pytest.mark.parametrize("kind, extra", [("point", -1), ("point", 0), ("point", 77), ("half", 1), ("dead", 1), ("nan", 1)])
 def test_rays_from_one_point(oracle, ctx, layout, sort, kind, extra):
     slots = torch.cuda.get_device_properties(0).multi_processor_count * 8 * 256
-    n = slots * (4 if sort or layout != "bin" else 12) + extra
+    n = slots * (4 if layout != "bin" else 2 if sort else 12) + extra
     v, t = scenes.uniform_soup(700, seed=41)
     bvh = hx.LBVHBuilder(ctx, morton_bits=60, layout=layout).build(hx.Scene(v, t))
     rays = _point_rays(n, 42, kind)
@@ -149,3 +149,20 @@ def test_rays_from_one_point(oracle, ctx, layout, sort, kind, extra):
     assert np.array_equal(res[:, :2], ref[:, :2])
     hit = ref[:, 0] >= 0
     assert hit.any() and np.array_equal(res[hit], ref[hit])
+
+
+@pytest.mark.parametrize("sort, per_slot", [(True, 4), (False, 12)])
+def test_any_hit_rays_from_one_point(oracle, ctx, sort, per_slot):
+    """Handed out refill by refill, any-hit rays still report the first hit of the
+    reference's traversal order."""
+    n = torch.cuda.get_device_properties(0).multi_processor_count * 8 * 256 * per_slot + 3
+    v, t = scenes.uniform_soup(700, seed=43)
+    bvh = hx.LBVHBuilder(ctx, morton_bits=60).build(hx.Scene(v, t))
+    rays = _point_rays(n, 44, "point")
+    rb = hx.RayBuffer(rays, closest_hit=False)
+    rb.results.fill_(0x7F7F7F7F)
+    tr = hx.HipTracer(ctx, bvh)
+    res = (tr.trace_sort(rb) if sort else tr.trace(rb)).cpu().numpy()
+    ref, _ = oracle.trace(bvh.nodes_host(), bvh.woop_host(), bvh.tri_indices_host(), rays, any_hit=True)
+    hit = ref[:, 0] >= 0
+    assert np.array_equal(res[:, :2], ref[:, :2]) and np.array_equal(res[hit], ref[hit])
